@@ -162,7 +162,7 @@ typedef struct {
     float    ms_device;     /* device time from the first to the last kernel of the frame, ms */
     float    ms_stage[6];   /* flatten, geometry (stroke + edges), tile setup, binning, coarse, fine */
     uint32_t graph;         /* 1 when the frame ran as a captured graph (stage times are then 0) */
-    uint32_t fine_words;    /* fine batch capacity in LDS words (commands per batch = words / tile^2) */
+    uint32_t fine_words;    /* fine batch capacity in LDS words (vkvg_hip_set_fine_words) */
 } vkh_stats;
 
 /* one autotuner measurement */
@@ -184,8 +184,9 @@ vkvg_public void        vkvg_hip_engine_destroy(vkh_engine *eng);
 vkvg_public int         vkvg_hip_set_tile_size(vkh_engine *eng, uint32_t tile);
 /* Optional external stream (a hipStream_t passed as void*); NULL = the engine's own. */
 vkvg_public void        vkvg_hip_set_stream(vkh_engine *eng, void *stream);
-/* Fine batch capacity in LDS words (2048, 4096 or 8192; 0 = 4096): commands staged per batch =
- * words / tile^2. Applies to the next execution. */
+/* Fine batch capacity in LDS words (2048, 4096 or 8192; 0 = 4096): commands rasterized per batch =
+ * words / tile^2, or half of that where more workgroups per CU pay more. Applies to the next
+ * execution. */
 vkvg_public int         vkvg_hip_set_fine_words(vkh_engine *eng, uint32_t words);
 /* Re-tiles the resident frame (8, 16 or 32 px) without uploading it again. */
 vkvg_public int         vkvg_hip_retile(vkh_engine *eng, uint32_t tile);

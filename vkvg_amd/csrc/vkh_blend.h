@@ -115,24 +115,43 @@ VKH_HD vkh_src16 vkh_src16_of(uint32_t op, uint32_t s) {
     return r;
 }
 
-// same result as blend_px_channels(op, d, s) for every input, S = vkh_src16_of(op, s)
-VKH_HD uint32_t blend_px16(uint32_t d, vkh_src16 S) {
-    const vkh_u16x2 h = {128, 128};
-    const vkh_u16x2 t_lo = vkh_u16x2_of(d & 0x00FF00FFu) * S.ia + h;
+// a pixel as two 16-bit lanes each of channels (0, 2) and (1, 3), the channel in the low byte
+typedef struct {
+    vkh_u16x2 lo, hi;
+} vkh_px16;
+
+VKH_HD vkh_px16 vkh_px16_of(uint32_t d) {
+    vkh_px16 r;
+    r.lo = vkh_u16x2_of(d & 0x00FF00FFu);
 #if defined(__HIP_DEVICE_COMPILE__)
-    // bytes 1 and 3 of d into the low bytes of the 16-bit lanes in one v_perm_b32
-    const vkh_u16x2 t_hi = vkh_u16x2_of(__builtin_amdgcn_perm(0u, d, 0x0c030c01u)) * S.ia + h;
+    r.hi = vkh_u16x2_of(__builtin_amdgcn_perm(0u, d, 0x0c030c01u)); // bytes 1 and 3 in one v_perm_b32
 #else
-    const vkh_u16x2 t_hi = vkh_u16x2_of((d >> 8) & 0x00FF00FFu) * S.ia + h;
+    r.hi = vkh_u16x2_of((d >> 8) & 0x00FF00FFu);
 #endif
-    const vkh_u16x2 v_lo = VKH_ADDSAT_U16X2(S.b_lo, t_lo + (t_lo >> 8));
-    const vkh_u16x2 v_hi = VKH_ADDSAT_U16X2(S.b_hi, t_hi + (t_hi >> 8));
+    return r;
+}
+VKH_HD uint32_t vkh_px_of(vkh_px16 p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    // high bytes: channel 0 = byte 1 of v_lo, 1 = byte 1 of v_hi, 2 = byte 3 of v_lo, 3 = byte 3 of v_hi
-    return __builtin_amdgcn_perm(vkh_u32_of(v_hi), vkh_u32_of(v_lo), 0x07030501u) ^ S.x;
+    return __builtin_amdgcn_perm(vkh_u32_of(p.hi), vkh_u32_of(p.lo), 0x06020400u);
 #else
-    return (((vkh_u32_of(v_lo) >> 8) & 0x00FF00FFu) | (vkh_u32_of(v_hi) & 0xFF00FF00u)) ^ S.x;
+    return vkh_u32_of(p.lo) | (vkh_u32_of(p.hi) << 8);
 #endif
 }
+
+// two channels of the blend: d (low bytes) under source operands ia and b, inverted by the mask x
+VKH_HD vkh_u16x2 vkh_blend_lanes(vkh_u16x2 d, vkh_u16x2 ia, vkh_u16x2 b, uint32_t x) {
+    const vkh_u16x2 h = {128, 128};
+    const vkh_u16x2 t = d * ia + h;
+    return vkh_u16x2_of(vkh_u32_of(VKH_ADDSAT_U16X2(b, t + (t >> 8))) ^ x) >> 8;
+}
+VKH_HD vkh_px16 vkh_blend16(vkh_px16 d, vkh_src16 S, uint32_t x) {
+    vkh_px16 r;
+    r.lo = vkh_blend_lanes(d.lo, S.ia, S.b_lo, x);
+    r.hi = vkh_blend_lanes(d.hi, S.ia, S.b_hi, x);
+    return r;
+}
+
+// same result as blend_px_channels(op, d, s) for every input, S = vkh_src16_of(op, s)
+VKH_HD uint32_t blend_px16(uint32_t d, vkh_src16 S) { return vkh_px_of(vkh_blend16(vkh_px16_of(d), S, S.x)); }
 
 #endif

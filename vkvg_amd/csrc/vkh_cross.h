@@ -16,6 +16,9 @@
 #define VKH_CR static inline
 #endif
 
+// the corrections after a quotient are needed by few lanes: one branch around both directions
+#define VKH_RARE(x) __builtin_expect(!!(x), 0)
+
 // n / d for the quotients below, each of which is followed by an exact correction of one step in
 // either direction, so it only has to be within one of the exact quotient: a single-precision
 // reciprocal (relative error below 2^-21, with d rounded to float) refined by one Newton step
@@ -41,12 +44,10 @@ VKH_CR int32_t cross_first_row(int32_t lx, int32_t ly, int32_t rx, int32_t ry, i
     const double C = (double)(ry - ly) * (double)(xs - lx);   // |C| < 2^48
     double f = floor(cross_quot(C, A)); // |C / A| < |ry - ly| <= 2^24; within one, corrected
     double rem = fma(-f, A, C);
-    if (rem < 0.0) {
-        f -= 1.0;
-        rem += A;
-    } else if (rem >= A) {
-        f += 1.0;
-        rem -= A;
+    if (VKH_RARE(rem < 0.0 || rem >= A)) {
+        const double c = rem < 0.0 ? -1.0 : 1.0;
+        f += c;
+        rem -= c * A;
     }
     // least u = y - ly that is not above: A u > C, or A u == C when ry <= ly
     const double t = (ry <= ly && rem == 0.0) ? f : f + 1.0;
@@ -60,9 +61,10 @@ VKH_CR int32_t cross_first_row(int32_t lx, int32_t ly, int32_t rx, int32_t ry, i
 // N = dy (xt - 128) + (xb - xt)(y - yt), D = 256 dy, dy = yb - yt. One row down adds
 // dN = 256 (xb - xt) to N, so with dq = floor(dN / D), dr = dN - dq D in [0, D) and rem = q D - N in
 // [0, D): q' = q + dq + (dr > rem), rem' = rem - dr, plus D when it carried.
+// rem and dr stay below D <= 2^32 (dy <= 2^24), so a step is 32-bit integer arithmetic modulo 2^32.
 typedef struct {
-    int32_t q, dq;      // column at the current row, whole-column step per row
-    double rem, dr, D;  // exact integers below 2^33
+    int32_t q, dq;       // column at the current row, whole-column step per row
+    uint32_t rem, dr, D; // D modulo 2^32
 } vkh_dda;
 
 // q = ceil(N / D) at row y, with rem = q D - N
@@ -72,12 +74,10 @@ VKH_CR double cross_column_rem(int32_t xt, int32_t yt, int32_t xb, int32_t yb, i
     const double N = fma(dy, (double)(xt - 128), (double)(xb - xt) * (double)(y - yt)); // exact, < 2^50
     double q = ceil(cross_quot(N, D)); // off by at most one
     double rem = fma(q, D, -N);
-    if (rem < 0.0) {
-        q += 1.0;
-        rem += D;
-    } else if (rem >= D) {
-        q -= 1.0;
-        rem -= D;
+    if (VKH_RARE(rem < 0.0 || rem >= D)) {
+        const double c = rem < 0.0 ? 1.0 : -1.0;
+        q += c;
+        rem += c * D;
     }
     *rem_out = rem;
     return q;
@@ -97,25 +97,23 @@ VKH_CR vkh_dda cross_dda_start(int32_t xt, int32_t yt, int32_t xb, int32_t yb, i
     const double dN = 256.0 * (double)(xb - xt);
     double dq = floor(cross_quot(dN, D));
     double dr = fma(-dq, D, dN);
-    if (dr < 0.0) {
-        dq -= 1.0;
-        dr += D;
-    } else if (dr >= D) {
-        dq += 1.0;
-        dr -= D;
+    if (VKH_RARE(dr < 0.0 || dr >= D)) {
+        const double c = dr < 0.0 ? -1.0 : 1.0;
+        dq += c;
+        dr -= c * D;
     }
     s.q = (int32_t)q;
     s.dq = (int32_t)dq;
-    s.rem = rem;
-    s.dr = dr;
-    s.D = D;
+    s.rem = (uint32_t)rem;
+    s.dr = (uint32_t)dr;
+    s.D = (uint32_t)(yb - yt) << 8;
     return s;
 }
 
 VKH_CR void cross_dda_step(vkh_dda *s) {
-    const int carry = s->dr > s->rem;
-    s->q += s->dq + (carry ? 1 : 0);
-    s->rem = carry ? s->rem + (s->D - s->dr) : s->rem - s->dr;
+    const uint32_t carry = s->rem < s->dr, t = s->rem - s->dr;
+    s->q += s->dq + (int32_t)carry;
+    s->rem = carry ? t + s->D : t;
 }
 
 #endif

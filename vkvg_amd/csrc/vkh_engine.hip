@@ -178,6 +178,7 @@ struct vkh_engine {
     uint32_t tile_total, bin_total, frame_tile, coarse_nch = 1, coarse_chunk = VKH_COARSE_CHUNK, n_cubic_items = 0;
     uint32_t most_draws = 1; // most draws on one target
     bool frame_ext = false; // the frame has surface sources or a target with a stencil plane
+    bool frame_sig = false; // a target of the frame keeps coverage signatures
 };
 
 static bool check(vkh_engine *e, hipError_t r, const char *what) {
@@ -466,7 +467,7 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     CK(hipStreamSynchronize(s)); // the staging blob may still feed an earlier copy
 
     // ---- host-side frame tables: work units and targets
-    bool any_stencil = false, any_source = false;
+    bool any_stencil = false, any_source = false, any_sig = false;
     std::vector<Unit> units;
     units.reserve(f->n_subpaths + 16);
     for (uint32_t d = 0; d < f->n_draws; d++) {
@@ -569,8 +570,8 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
             ti.stencil = f->targets[t].stencil;
             ti.stencil_load = f->targets[t].stencil_load ? 1u : 0u;
             ti.pad = 0;
-            if (ti.stencil)
-                any_stencil = true;
+            any_stencil |= ti.stencil != nullptr;
+            any_sig |= ti.sig != nullptr;
         }
     }
     const uint32_t n_units = (uint32_t)units.size();
@@ -637,6 +638,7 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     for (const TargetInfo &ti : tg)
         eng->most_draws = std::max(eng->most_draws, ti.draw_end - ti.draw_begin);
     eng->frame_ext = any_stencil || any_source;
+    eng->frame_sig = any_sig;
     eng->h_tileless.clear();
     for (uint32_t i = 0; i < n_draws; i++)
         if (!kind_has_tiles(f->draws[i].kind))
@@ -898,7 +900,7 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
         CK(hipEventRecord(eng->ev_stage[4], s)); // coarse done
     if (!cap)
         CK(hipEventRecord(eng->ev0, s));
-    vkh::launch_fine(s, eng->frame_ext, T, eng->fine_words, tile_total, d_tg, n_targets, P<DrawPrep>(eng->dprep), d_grec, d_grads, d_gprep,
+    vkh::launch_fine(s, eng->frame_ext, eng->frame_sig, T, eng->fine_words, tile_total, d_tg, n_targets, P<DrawPrep>(eng->dprep), d_grec, d_grads, d_gprep,
                      P<PathTile>(eng->ptiles),
                      P<Edge>(eng->segs), nch, P<uint32_t>(eng->tile_off),
                      P<Cmd>(eng->cmds), P<uint32_t>(eng->tile_order));

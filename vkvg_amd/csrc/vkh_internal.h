@@ -61,7 +61,6 @@ struct PathTile {
 enum : uint32_t {
     VKH_DP_GRAD = 1u << 9,     // meta: gradient source
     VKH_DP_SURF = 1u << 10,    // meta: surface source (the draw's GradRec slot holds a SurfRec)
-    VKH_DP_HASSEG = 1u << 8,   // meta (set per command in the fine kernel): the path tile has segments
     VKH_GF_UY0 = 1u,           // linear: direction has no y component
     VKH_GF_UXNEG = 2u,         // linear: ... and points to -x
     VKH_GF_UYNEG = 4u,         // linear: y component < 0
@@ -180,8 +179,9 @@ uint32_t coarse_chunk(uint32_t most_draws, uint32_t n_bins);
 void launch_coarse(hipStream_t s, bool write, uint32_t n_bins, uint32_t nch, uint32_t chunk, const TargetInfo *tg,
                    uint32_t n_targets, const vkh_draw *draws, const DrawTiles *dt, const PathTile *pts,
                    uint32_t *tile_count, const uint32_t *tile_off, Cmd *cmds);
-// ext: the frame has surface sources or a target with a stencil plane (the extended variant runs)
-void launch_fine(hipStream_t s, bool ext, uint32_t tile, uint32_t words, uint32_t n_tiles, const TargetInfo *tg,
+// ext: the frame has surface sources or a target with a stencil plane (the extended variant runs);
+// sig: a target keeps coverage signatures
+void launch_fine(hipStream_t s, bool ext, bool sig, uint32_t tile, uint32_t words, uint32_t n_tiles, const TargetInfo *tg,
                  uint32_t n_targets, const DrawPrep *dprep, const GradRec *grec, const vkh_gradient *grads,
                  const GradPrep *gprep, const PathTile *pts, const Edge *segs, uint32_t nch,
                  const uint32_t *tile_off, const Cmd *cmds, const uint32_t *order);

@@ -797,34 +797,64 @@ __device__ __forceinline__ uint32_t stencil_apply(uint32_t kind, uint32_t prm, u
 }
 
 
-// Blends one source into a covered pixel: once, and for strokes once more per further covering
-// triangle (w = the winding count, >= 1 here); the signature adds the draw's key per blend.
-__device__ __forceinline__ void blend_count(const vkh_src16 &S, bool stroke, int32_t w, uint32_t key, uint32_t &v,
+// Blends one source into a pixel covered w > 0 times: once, and for strokes once per covering triangle;
+// the signature adds the draw's key per blend. INV: the operator inverts the result (vkh_blend.h)
+template <bool INV, bool SIG>
+__device__ __forceinline__ void blend_count(const vkh_src16 &S, bool stroke, int32_t w, uint32_t key, vkh_px16 &v,
                                             uint32_t &sg) {
-    v = blend_px16(v, S);
-    sg += key;
+    v = vkh_blend16(v, S, INV ? S.x : 0u);
+    if (SIG)
+        sg += key;
     if (stroke)
         for (int32_t n = 1; n < w; n++) {
-            v = blend_px16(v, S);
-            sg += key;
+            v = vkh_blend16(v, S, INV ? S.x : 0u);
+            if (SIG)
+                sg += key;
         }
 }
 
-// One workgroup per T x T tile. Commands are processed in batches of B: the batch's command
-// records (draw record + path tile) are staged in LDS with one parallel load; every segment of the
-// batch (one thread each) adds its edge's crossings of the tile's sample rows into per-command
-// LDS row deltas, walking only the rows the edge spans; each row is prefix-summed once; then every
-// pixel applies the batch's commands in order, reading each command's record as wave-uniform
-// values. The dependent global loads (command -> draw / path tile -> segment -> edge) are thus
-// paid once per batch and once per segment.
-// WORDS: row-delta words of LDS per workgroup (B = WORDS / pixels commands per batch)
+// Inclusive prefix over a tile row: each T consecutive lanes (T = 8, 16 or 32) hold a row's T columns.
+// DPP row shifts (a DPP row is 16 lanes) instead of LDS; every lane of the wavefront must be active.
+template <int T> __device__ __forceinline__ int32_t tile_row_prefix(int32_t x, const int32_t (&m8)[2]) {
+    if (T == 8) { // a shift by 1 or 2 would also carry across the middle of a 16-lane row: masked
+        x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true) & m8[0];
+        x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true) & m8[1];
+        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xa, false); // lanes 4..7 of each 8
+        return x;
+    }
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true); // row_shr:1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    if (T == 32) // the total of the row's first half (lane 15) into its second half (row_bcast:15)
+        x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    return x;
+}
+
+// One workgroup of NT threads per T x T tile, PPT = T * T / NT pixels per thread. The tile's commands are
+// staged S at a time (their draw record and path tile: one chain of dependent loads per S commands) and
+// rasterized B at a time: every segment of the B commands (one thread each) adds its edge's crossings
+// of the tile's sample rows into per-command LDS row deltas, walking only the rows the edge spans;
+// then every pixel applies the commands in order: its winding is the prefix of its row's deltas,
+// taken across the lanes that hold the row, and the command's record is read as wave-uniform values.
+// Bound by vector issue (93 % of it on the 1920x1080 stroke scene, 9.8 M commands: 1.25 G wave VALU
+// instructions). Two pixels per thread share what a command costs once per wave (its record's LDS
+// reads, decode, branches); pixels stay unpacked in 16-bit lanes between blends; the row prefix is four
+// DPP additions instead of a pass of 16-way conflicting LDS reads and writes per row; signatures are
+// compiled out where no target keeps them. One pixel per thread with the row pass: 3.11 ms there and
+// 1.82 ms on the 4096x4096 dense scene (4.0 M commands); this form 2.29 and 1.55 ms (four pixels per
+// thread: 3.01 and 1.89 ms, at 10 KB of LDS per wavefront too few wavefronts are resident).
 // EXT: the frame has surface sources or targets with a stencil plane (the plain variant compiles
 // neither). With a stencil plane each pixel also carries its stencil word
 // (loaded from the plane or zero, stored back at the end): draws blend only where CLIP is 0, clear
 // zeroes the stencil byte, and the clip and stencil draws rewrite it (src/vkvg_context.c:698-795,
 // :1251-1512; pipeline states of src/vkvg_device_internal.c:226-246).
-template <int T, int WORDS, bool EXT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void k_fine(const TargetInfo *__restrict__ tg, uint32_t n_targets,
+// SIG: a target of the frame keeps coverage signatures.
+// The plain 128-thread variant is held to 64 VGPRs and 80 SGPRs: 8 wavefronts per SIMD (dense scene
+// 1.67 -> 1.59 ms).
+template <int T, int NT, int B, bool EXT, bool SIG>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(NT == 128 && !EXT ? 8 : 4)))
+void k_fine(const TargetInfo *__restrict__ tg, uint32_t n_targets,
                                               const DrawPrep *__restrict__ dprep,
                                               const GradRec *__restrict__ grec,
                                               const vkh_gradient *__restrict__ grads,
@@ -834,17 +864,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void k_fi
                                               const uint32_t *__restrict__ tile_off, const Cmd *__restrict__ cmds,
                                               const uint32_t *__restrict__ tile_order) {
     constexpr int NPIX = T * T;
-    constexpr int NT = NPIX >= 256 ? 256 : NPIX;  // threads
     constexpr int PPT = NPIX / NT;                // pixels per thread
-    constexpr int B = WORDS / NPIX;               // commands per batch
-    __shared__ int32_t sd[B][T][T];               // row deltas, then per-row inclusive prefix
+    constexpr int S = B >= 32 ? B : 32;           // commands staged at a time
+    static_assert(S % B == 0, "staged commands: whole batches");
+    __shared__ int32_t sd[B][T][T];               // row deltas; column 0 takes the row's V term
     __shared__ int32_t srow[B][T];                // V term: +-1 at the first row below a column crossing
-    __shared__ uint32_t c_item[B + 1];            // prefix of the commands' segment counts
-    __shared__ uint32_t c_nseg[B], c_segoff[B], c_draw[B];
-    __shared__ int32_t c_back[B];                 // path tile backdrop (the row prefix adds it)
-    __shared__ uint4 c_rec[B];  // meta, key, winding added in compositing (the backdrop without segments),
-                                // covering winding bits (the parameter of a stencil draw)
-    __shared__ uint4 c_src[B];  // blend operands of a solid source (vkh_src16)
+    __shared__ uint32_t c_item[S + 1];            // prefix of the commands' segment counts
+    __shared__ uint2 c_seg[S];                    // first segment less its position in that prefix, and the
+                                                  // winding of one crossing: 1, or 2^31 for even-odd (whose
+                                                  // sums modulo 2^32 are then zero where even)
+    __shared__ uint4 c_rec[S];  // meta, key, backdrop (or the winding of a paint or clear), the
+                                // parameter of a stencil draw
+    __shared__ uint4 c_src[S];  // blend operands of a solid source (vkh_src16); else x: the draw
 
     const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
     uint32_t c0 = tile_off[(size_t)gtile * nch], c1 = tile_off[(size_t)(gtile + 1) * nch];
@@ -869,19 +900,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void k_fi
     const float Wf = (float)TI.width, Hf = (float)TI.height;
     const int32_t xs0 = 256 * X0 + 128, s0y = 256 * Y0 + 128;
 
-    int lx[PPT], ly[PPT];
-    bool valid[PPT];
-    uint32_t px[PPT], sig[PPT];
-    float gx[PPT], gy[PPT]; // gradient coordinates gl_FragCoord.xy / size
+    const int lx = (int)tid % T, ly0 = (int)tid / T; // pixel q: column lx, row ly0 + q * (NT / T)
+    static_assert(NT % T == 0, "a thread's pixels share a column");
+    const int32_t m8[2] = {(lx & 7) >= 1 ? -1 : 0, (lx & 7) >= 2 ? -1 : 0};
+    vkh_px16 px[PPT];
+    uint32_t sig[PPT];
+    float gy[PPT]; // gradient coordinates gl_FragCoord.xy / size
+    const float gx = ((float)(X0 + lx) + 0.5f) / Wf;
+    const bool validx = X0 + lx < (int32_t)TI.width;
 #pragma unroll
     for (int q = 0; q < PPT; q++) {
-        int p = (int)tid + q * NT;
-        lx[q] = p % T;
-        ly[q] = p / T;
-        valid[q] = (X0 + lx[q]) < (int32_t)TI.width && (Y0 + ly[q]) < (int32_t)TI.height;
         sig[q] = 0;
-        gx[q] = ((float)(X0 + lx[q]) + 0.5f) / Wf;
-        gy[q] = ((float)(Y0 + ly[q]) + 0.5f) / Hf;
+        gy[q] = ((float)(Y0 + ly0 + q * (NT / T)) + 0.5f) / Hf;
     }
     // the destination need not be read when the first command overwrites every pixel (under a
     // stencil only a clear does: any other draw may be clipped)
@@ -900,225 +930,239 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void k_fi
                 need_read = false;
         }
     }
+    // pixels beyond the target's edge are composited like the others and never loaded or stored
+    auto inside = [&](int q) { return validx && Y0 + ly0 + q * (NT / T) < (int32_t)TI.height; };
+    auto at = [&](int q) { return (size_t)(Y0 + ly0 + q * (NT / T)) * TI.width + (size_t)(X0 + lx); };
     uint32_t st[PPT]; // stencil words
-#pragma unroll
-    for (int q = 0; q < PPT; q++) {
-        st[q] = 0u;
-        if (EXT && TI.stencil && TI.stencil_load && valid[q])
-            st[q] = TI.stencil[(size_t)(Y0 + ly[q]) * TI.width + (size_t)(X0 + lx[q])];
-    }
     uint32_t *img = (uint32_t *)TI.rgba;
 #pragma unroll
     for (int q = 0; q < PPT; q++) {
-        size_t o = (size_t)(Y0 + ly[q]) * TI.width + (size_t)(X0 + lx[q]);
-        px[q] = (need_read && valid[q]) ? img[o] : 0u;
+        st[q] = 0u;
+        if (EXT && TI.stencil && TI.stencil_load && inside(q))
+            st[q] = TI.stencil[at(q)];
+        px[q] = vkh_px16_of((need_read && inside(q)) ? img[at(q)] : 0u);
     }
 
-    // the row deltas start at zero; afterwards every batch leaves them at zero (the row prefix
+    // the row deltas start at zero; afterwards every batch leaves them at zero (the row scan
     // clears srow as it reads it, the compositing clears each pixel's word of sd after its last read)
     for (uint32_t k = tid; k < (uint32_t)(B * NPIX); k += NT)
         (&sd[0][0][0])[k] = 0;
     for (uint32_t k = tid; k < (uint32_t)(B * T); k += NT)
         (&srow[0][0])[k] = 0;
-    for (uint32_t base = c0; base < c1; base += B) {
-        const uint32_t nb = min((uint32_t)B, c1 - base);
-        // ---- stage the batch's records
-        for (uint32_t j = tid; j < nb; j += NT) {
-            const Cmd cm = cmds[base + j];
-            const DrawPrep &d = dprep[cm.draw];
-            uint32_t meta = d.meta;
-            const uint32_t kind = meta & 15;
-            if (cm.pt == VKH_NO_DRAW) {
-                if (kind <= VKH_DRAW_CLEAR)
-                    meta = (meta & ~15u) | (kind == VKH_DRAW_CLEAR ? VKH_DRAW_CLEAR : VKH_DRAW_PAINT);
-                c_back[j] = 0;
-                c_rec[j].z = kind <= VKH_DRAW_CLEAR ? 1u : 0u; // paint and clear: winding 1 everywhere
-                c_nseg[j] = 0;
-                c_segoff[j] = 0;
-            } else {
-                const PathTile p = pts[cm.pt];
-                c_back[j] = p.backdrop;
-                c_rec[j].z = p.nseg ? 0u : (uint32_t)p.backdrop;
-                c_nseg[j] = p.nseg;
-                c_segoff[j] = p.seg_off;
-                if (p.nseg)
-                    meta |= VKH_DP_HASSEG;
-            }
-            c_rec[j].x = meta;
-            c_rec[j].y = d.key;
-            // the winding bits that make a sample covered: odd for even-odd fills, any for non-zero
-            // fills, strokes (whose winding, a count of covering triangles, is never negative), paint
-            // and clear; the stencil draws read their parameter instead
-            c_rec[j].w = kind >= VKH_DRAW_CLIP_NZ ? d.solid : kind == VKH_DRAW_FILL_EO ? 1u : 0xFFFFFFFFu;
-            const vkh_src16 S = vkh_src16_of((meta >> 4) & 15, d.solid);
-            c_src[j] = make_uint4(vkh_u32_of(S.ia), vkh_u32_of(S.b_lo), vkh_u32_of(S.b_hi), S.x);
-            c_draw[j] = cm.draw;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t acc = 0;
-            for (uint32_t j = 0; j < nb; j++) {
-                c_item[j] = acc;
-                acc += c_nseg[j];
-            }
-            c_item[nb] = acc;
-        }
-        __syncthreads();
-        // ---- crossings: one thread per segment of the batch, walking only the sample rows its
-        // edge spans inside the tile
-        const uint32_t total = c_item[nb];
-        for (uint32_t it = tid; it < total; it += NT) {
-            uint32_t lo = 0, hi = nb; // last j with c_item[j] <= it
-            while (hi - lo > 1) {
-                uint32_t mid = (lo + hi) >> 1;
-                if (c_item[mid] <= it)
-                    lo = mid;
-                else
-                    hi = mid;
-            }
-            const uint32_t j = lo;
-            const Edge e = segs[c_segoff[j] + (it - c_item[j])];
-            // V term: the edge separates (xs0, s0y) from (xs0, sy(r)) for every row r >= r*
-            if (min(e.x0, e.x1) <= xs0 && xs0 < max(e.x0, e.x1)) {
-                const bool lr = e.x0 < e.x1;
-                const int32_t r = cross_first_row(lr ? e.x0 : e.x1, lr ? e.y0 : e.y1, lr ? e.x1 : e.x0,
-                                                  lr ? e.y1 : e.y0, xs0, s0y, 0, T);
-                if (r >= 1 && r < T) // r* = 0: (xs0, s0y) is not above the edge
-                    atomicAdd(&srow[j][r], lr ? -1 : 1);
-            }
-            // H term: rows with ytop <= sy(r) < ybot
-            const bool down = e.y0 < e.y1;
-            const int32_t xt = down ? e.x0 : e.x1, yt = down ? e.y0 : e.y1;
-            const int32_t xb = down ? e.x1 : e.x0, yb = down ? e.y1 : e.y0;
-            const int32_t r_lo = max(((yt - 128 + 255) >> 8) - Y0, 0);
-            const int32_t r_hi = min(((yb - 128 + 255) >> 8) - 1 - Y0, T - 1);
-            if (r_lo > r_hi)
-                continue;
-            const int32_t sgn = down ? 1 : -1;
-            vkh_dda dda = cross_dda_start(xt, yt, xb, yb, s0y + 256 * r_lo);
-            for (int32_t r = r_lo;; r++) {
-                const int32_t lc = dda.q - X0;
-                if (lc >= 1 && lc < T)
-                    atomicAdd(&sd[j][r][lc], sgn);
-                if (r == r_hi)
-                    break;
-                cross_dda_step(&dda);
-            }
-        }
-        __syncthreads();
-        // ---- per (command, row): inclusive prefix with the row's V term. The T rows of a command
-        // are T consecutive lanes (nb * T and the loop stride are multiples of T, so a group is
-        // wholly active or inactive): a segmented shuffle scan sums srow[j][1 .. r] (srow[j][0] is 0).
-        for (uint32_t q = tid; q < nb * (uint32_t)T; q += NT) {
-            const uint32_t j = q / T, r = q % T;
-            int32_t acc = srow[j][r];
-            srow[j][r] = 0;
-#pragma unroll
-            for (int o = 1; o < T; o <<= 1) {
-                const int32_t y = __shfl_up(acc, (unsigned)o, T);
-                if ((int)r >= o)
-                    acc += y;
-            }
-            if (!c_nseg[j])
-                continue;
-            acc += c_back[j];
-#pragma unroll
-            for (int c = 0; c < T; c++) {
-                acc += sd[j][r][c];
-                sd[j][r][c] = acc;
-            }
-        }
-        __syncthreads();
-        // ---- ordered compositing. A command's coverage count k is 0 or 1 for fills (no loop) and
-        // the winding number for strokes (a pixel covered by k triangles is blended k times); the
-        // blend operands of a solid source were computed once per command when the batch was staged.
-        for (uint32_t j = 0; j < nb; j++) {
-            const uint4 rec = c_rec[j];
-            const uint32_t meta = uniform_u32(rec.x);
-            const uint32_t kind = meta & 15, op = (meta >> 4) & 15;
-            const int32_t bk = (int32_t)rec.z; // 0 when the winding comes from the row deltas
-            const uint32_t key = rec.y;
-            if (EXT && kind >= VKH_DRAW_CLIP_NZ) { // stencil draws (uniform branch)
-                if (kind_is_clip(kind)) {
-#pragma unroll
-                    for (int q = 0; q < PPT; q++) {
-                        // the row deltas of a command without segments are zero
-                        const int32_t w = sd[j][ly[q]][lx[q]] + bk;
-                        sd[j][ly[q]][lx[q]] = 0;
-                        const bool cov = kind == VKH_DRAW_CLIP_NZ ? w != 0 : (w & 1) != 0;
-                        if (cov && !(st[q] & 2u)) {
-                            if (valid[q])
-                                sig[q] += key; // the clip's 1-sample mask
-                        } else {
-                            st[q] |= 2u;
-                        }
+    for (uint32_t base = c0; base < c1; base += S) {
+        const uint32_t ns = min((uint32_t)S, c1 - base);
+        // ---- stage the commands' records and the prefix of their segment counts (one wavefront)
+        if (tid < 64) {
+            uint32_t before = 0; // segments of the groups of 64 before this one
+            for (uint32_t g = 0; g < S; g += 64) {
+                const uint32_t j = g + tid;
+                uint32_t nseg = 0, segoff = 0, unit = 1;
+                if (j < ns) {
+                    const Cmd cm = cmds[base + j];
+                    const DrawPrep &d = dprep[cm.draw];
+                    uint32_t meta = d.meta;
+                    const uint32_t kind = meta & 15;
+                    unit = kind == VKH_DRAW_FILL_EO || kind == VKH_DRAW_CLIP_EO ? 0x80000000u : 1u;
+                    uint4 rec;
+                    if (cm.pt == VKH_NO_DRAW) {
+                        if (kind <= VKH_DRAW_CLEAR)
+                            meta = (meta & ~15u) | (kind == VKH_DRAW_CLEAR ? VKH_DRAW_CLEAR : VKH_DRAW_PAINT);
+                        rec.z = kind <= VKH_DRAW_CLEAR ? 1u : 0u; // paint and clear: winding 1 everywhere
+                    } else {
+                        const PathTile p = pts[cm.pt];
+                        rec.z = (uint32_t)p.backdrop * unit;
+                        nseg = p.nseg;
+                        segoff = p.seg_off;
                     }
+                    rec.x = meta;
+                    rec.y = d.key;
+                    rec.w = d.solid; // the parameter of a stencil draw
+                    c_rec[j] = rec;
+                    const vkh_src16 Sc = vkh_src16_of((meta >> 4) & 15, d.solid);
+                    uint4 sv = make_uint4(vkh_u32_of(Sc.ia), vkh_u32_of(Sc.b_lo), vkh_u32_of(Sc.b_hi), Sc.x);
+                    if (meta & (VKH_DP_GRAD | VKH_DP_SURF))
+                        sv.x = cm.draw;
+                    c_src[j] = sv;
+                }
+                uint32_t incl = nseg;
+#pragma unroll
+                for (int o = 1; o < (S < 64 ? S : 64); o <<= 1) {
+                    const uint32_t y = (uint32_t)__shfl_up((int)incl, o);
+                    if ((int)tid >= o)
+                        incl += y;
+                }
+                if (j < S) {
+                    c_item[j + 1] = before + incl;
+                    c_seg[j] = make_uint2(segoff - (before + incl - nseg), unit);
+                }
+                before += (uint32_t)__shfl((int)incl, 63);
+            }
+            if (tid == 0)
+                c_item[0] = 0;
+        }
+        __syncthreads();
+        for (uint32_t sub = 0; sub < ns; sub += B) {
+            const uint32_t nb = min((uint32_t)B, ns - sub);
+            // ---- crossings: one thread per segment of the batch, walking only the sample rows its
+            // edge spans inside the tile
+            const uint32_t it1 = c_item[sub + nb];
+            for (uint32_t it = c_item[sub] + tid; it < it1; it += NT) {
+                uint32_t j = 0; // last j with c_item[sub + j] <= it
+                if (B <= 8) {
+#pragma unroll
+                    for (uint32_t k = 1; k < (uint32_t)B; k++)
+                        j += c_item[sub + k] <= it ? 1u : 0u;
+                    j = min(j, nb - 1);
                 } else {
-                    const uint32_t prm = uniform_u32(rec.w);
-#pragma unroll
-                    for (int q = 0; q < PPT; q++)
-                        st[q] = stencil_apply(kind, prm, st[q]);
+                    uint32_t hi = nb;
+                    while (hi - j > 1) {
+                        const uint32_t mid = (j + hi) >> 1;
+                        if (c_item[sub + mid] <= it)
+                            j = mid;
+                        else
+                            hi = mid;
+                    }
                 }
-                continue;
-            }
-            const bool stroke = kind == VKH_DRAW_STROKE;
-            const uint32_t rule = rec.w; // covering winding bits
-            int32_t wq[PPT];
-            bool on[PPT];
-#pragma unroll
-            for (int q = 0; q < PPT; q++) {
-                // the row deltas of a command without segments are zero
-                const int32_t w = sd[j][ly[q]][lx[q]] + bk;
-                sd[j][ly[q]][lx[q]] = 0;
-                wq[q] = w;
-                on[q] = ((uint32_t)w & rule) != 0u && valid[q];
-                if (EXT && on[q]) {
-                    if (kind == VKH_DRAW_CLEAR)
-                        st[q] &= ~0xFFu; // vkCmdClearAttachments ignores the stencil test
-                    else if (st[q] & 2u)
-                        on[q] = false; // clipped
+                const uint2 cs = c_seg[sub + j];
+                const Edge e = segs[cs.x + it];
+                const uint32_t unit = cs.y;
+                // V term: the edge separates (xs0, s0y) from (xs0, sy(r)) for every row r >= r*
+                if (min(e.x0, e.x1) <= xs0 && xs0 < max(e.x0, e.x1)) {
+                    const bool lr = e.x0 < e.x1;
+                    const int32_t r = cross_first_row(lr ? e.x0 : e.x1, lr ? e.y0 : e.y1, lr ? e.x1 : e.x0,
+                                                      lr ? e.y1 : e.y0, xs0, s0y, 0, T);
+                    if (r >= 1 && r < T) // r* = 0: (xs0, s0y) is not above the edge
+                        atomicAdd(&srow[j][r], (int32_t)(lr ? 0u - unit : unit));
+                }
+                // H term: rows with ytop <= sy(r) < ybot
+                const bool down = e.y0 < e.y1;
+                const int32_t xt = down ? e.x0 : e.x1, yt = down ? e.y0 : e.y1;
+                const int32_t xb = down ? e.x1 : e.x0, yb = down ? e.y1 : e.y0;
+                const int32_t r_lo = max(((yt - 128 + 255) >> 8) - Y0, 0);
+                const int32_t r_hi = min(((yb - 128 + 255) >> 8) - 1 - Y0, T - 1);
+                if (r_lo > r_hi)
+                    continue;
+                const int32_t sgn = (int32_t)(down ? unit : 0u - unit);
+                vkh_dda dda = cross_dda_start(xt, yt, xb, yb, s0y + 256 * r_lo);
+                dda.q -= X0 + 1;
+                int32_t *row = &sd[j][r_lo][1];
+                for (int32_t n = r_hi - r_lo;; n--) {
+                    if ((uint32_t)dda.q < (uint32_t)(T - 1)) // columns 1 .. T - 1
+                        atomicAdd(row + dda.q, sgn);
+                    if (n == 0)
+                        break;
+                    row += T;
+                    cross_dda_step(&dda);
                 }
             }
-            // blend operands: once per command for a solid source, per pixel for a gradient or surface
-            vkh_src16 S[PPT];
-            if (!(meta & (EXT ? (VKH_DP_GRAD | VKH_DP_SURF) : VKH_DP_GRAD))) {
-                const uint4 sv = c_src[j];
-                const vkh_src16 S0 = {vkh_u16x2_of(sv.x), vkh_u16x2_of(sv.y), vkh_u16x2_of(sv.z), sv.w};
-#pragma unroll
-                for (int q = 0; q < PPT; q++)
-                    S[q] = S0;
-            } else {
+            __syncthreads();
+            // ---- per (command, row): the backdrop plus the V term's prefix over the rows, written to the
+            // row's first column (no crossing lands there). The T rows of a command are T consecutive
+            // lanes; srow[j][0] is 0.
+            for (uint32_t q0 = 0; q0 < nb * (uint32_t)T; q0 += NT) {
+                const uint32_t q = q0 + tid, j = q / T, r = q % T;
+                const bool live = j < nb; // every lane takes part in the prefix
+                int32_t acc = live ? srow[j][r] : 0;
+                acc = tile_row_prefix<T>(acc, m8);
+                if (live) {
+                    srow[j][r] = 0;
+                    sd[j][r][0] = acc + (int32_t)c_rec[sub + j].z;
+                }
+            }
+            __syncthreads();
+            // ---- ordered compositing. A command's coverage count k is 0 or 1 for fills (no loop) and
+            // the winding number for strokes (a pixel covered by k triangles is blended k times); the
+            // blend operands of a solid source were computed once per command when it was staged.
+            for (uint32_t j = 0; j < nb; j++) {
+                // the command's record, blend operands and row deltas in one round trip to LDS
+                const uint4 rec = c_rec[sub + j], sv = c_src[sub + j];
+                int32_t wq[PPT]; // the windings
 #pragma unroll
                 for (int q = 0; q < PPT; q++) {
-                    if (!on[q])
-                        continue;
-                    float col[4], op_;
-                    if (!EXT || (meta & VKH_DP_GRAD)) {
-                        const GradRec &P = grec[uniform_u32(c_draw[j])]; // scalar loads
-                        op_ = P.opacity;
-                        gradient_color(P, grads, gprep, gx[q], gy[q], col);
+                    int32_t *w = &sd[j][ly0 + q * (NT / T)][lx];
+                    wq[q] = *w;
+                    *w = 0;
+                }
+#pragma unroll
+                for (int q = 0; q < PPT; q++) {
+                    wq[q] = tile_row_prefix<T>(wq[q], m8);
+                    // keeps the sum whole: folded into its later uses it would no longer be DPP additions
+                    asm("" : "+v"(wq[q]));
+                }
+                const uint32_t meta = uniform_u32(rec.x);
+                const uint32_t kind = meta & 15, op = (meta >> 4) & 15;
+                const uint32_t key = rec.y;
+                if (EXT && kind >= VKH_DRAW_CLIP_NZ) { // stencil draws (uniform branch)
+                    if (kind_is_clip(kind)) {
+#pragma unroll
+                        for (int q = 0; q < PPT; q++) {
+                            if (wq[q] != 0 && !(st[q] & 2u))
+                                sig[q] += key; // the clip's 1-sample mask
+                            else
+                                st[q] |= 2u;
+                        }
                     } else {
-                        const SurfRec &R = *reinterpret_cast<const SurfRec *>(&grec[uniform_u32(c_draw[j])]);
-                        op_ = R.opacity;
-                        surface_color(R, (float)(X0 + lx[q]) + 0.5f, (float)(Y0 + ly[q]) + 0.5f, col);
+                        const uint32_t prm = uniform_u32(rec.w);
+#pragma unroll
+                        for (int q = 0; q < PPT; q++)
+                            st[q] = stencil_apply(kind, prm, st[q]);
                     }
-                    S[q] = vkh_src16_of(op, f2u8x4(col[0] * op_, col[1] * op_, col[2] * op_, col[3] * op_));
+                    continue;
+                }
+                const bool stroke = kind == VKH_DRAW_STROKE;
+                if (EXT) {
+#pragma unroll
+                    for (int q = 0; q < PPT; q++) {
+                        if (kind == VKH_DRAW_CLEAR)
+                            st[q] &= ~0xFFu; // vkCmdClearAttachments ignores the stencil test
+                        else if (st[q] & 2u)
+                            wq[q] = 0; // clipped
+                    }
+                }
+                if (!(meta & (EXT ? (VKH_DP_GRAD | VKH_DP_SURF) : VKH_DP_GRAD))) {
+                    const vkh_src16 S0 = {vkh_u16x2_of(sv.x), vkh_u16x2_of(sv.y), vkh_u16x2_of(sv.z), sv.w};
+                    if (op == 1 || op == 2) {
+#pragma unroll
+                        for (int q = 0; q < PPT; q++)
+                            if (wq[q] != 0)
+                                blend_count<false, SIG>(S0, stroke, wq[q], key, px[q], sig[q]);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < PPT; q++)
+                            if (wq[q] != 0)
+                                blend_count<true, SIG>(S0, stroke, wq[q], key, px[q], sig[q]);
+                    }
+                } else { // per pixel for a gradient or surface
+                    const GradRec *rp = &grec[uniform_u32(sv.x)];
+#pragma unroll
+                    for (int q = 0; q < PPT; q++) {
+                        if (wq[q] == 0)
+                            continue;
+                        float col[4], op_;
+                        if (!EXT || (meta & VKH_DP_GRAD)) {
+                            op_ = rp->opacity; // scalar loads
+                            gradient_color(*rp, grads, gprep, gx, gy[q], col);
+                        } else {
+                            const SurfRec &R = *reinterpret_cast<const SurfRec *>(rp);
+                            op_ = R.opacity;
+                            surface_color(R, (float)(X0 + lx) + 0.5f, (float)(Y0 + ly0 + q * (NT / T)) + 0.5f, col);
+                        }
+                        const vkh_src16 Sq =
+                            vkh_src16_of(op, f2u8x4(col[0] * op_, col[1] * op_, col[2] * op_, col[3] * op_));
+                        blend_count<true, SIG>(Sq, stroke, wq[q], key, px[q], sig[q]);
+                    }
                 }
             }
-#pragma unroll
-            for (int q = 0; q < PPT; q++)
-                if (on[q])
-                    blend_count(S[q], stroke, wq[q], key, px[q], sig[q]);
+            __syncthreads();
         }
-        __syncthreads();
     }
 #pragma unroll
     for (int q = 0; q < PPT; q++) {
-        if (!valid[q])
+        if (!inside(q))
             continue;
-        size_t o = (size_t)(Y0 + ly[q]) * TI.width + (size_t)(X0 + lx[q]);
-        img[o] = px[q];
-        if (TI.sig)
+        const size_t o = at(q);
+        img[o] = vkh_px_of(px[q]);
+        if (SIG && TI.sig)
             TI.sig[o] += sig[q];
         if (EXT && TI.stencil)
             TI.stencil[o] = st[q];
@@ -1237,53 +1281,45 @@ void launch_draw_prep(hipStream_t s, const vkh_draw *draws, uint32_t n, const Ta
     if (n_grads)
         hipLaunchKernelGGL(k_grad_prep, dim3((n_grads + 255) / 256), dim3(256), 0, s, grads, n_grads, gout);
 }
-template <int T, int W>
-static void fine_launch(hipStream_t s, bool ext, uint32_t n_tiles, const TargetInfo *tg, uint32_t n_targets,
-                        const DrawPrep *dprep, const GradRec *grec, const vkh_gradient *grads, const GradPrep *gprep,
-                        const PathTile *pts, const Edge *segs, uint32_t nch, const uint32_t *tile_off,
-                        const Cmd *cmds, const uint32_t *order) {
-    constexpr int NT = T * T >= 256 ? 256 : T * T;
+template <int T, int NT, int B, class... A>
+static void fine_launch(hipStream_t s, bool ext, bool sig, uint32_t n_tiles, A... args) {
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(n_tiles), dim3(NT), 0, s, args...); };
     if (ext)
-        hipLaunchKernelGGL((k_fine<T, W, true>), dim3(n_tiles), dim3(NT), 0, s, tg, n_targets, dprep, grec, grads, gprep,
-                           pts, segs, nch, tile_off, cmds, order);
+        launch(sig ? k_fine<T, NT, B, true, true> : k_fine<T, NT, B, true, false>);
     else
-        hipLaunchKernelGGL((k_fine<T, W, false>), dim3(n_tiles), dim3(NT), 0, s, tg, n_targets, dprep, grec, grads,
-                           gprep, pts, segs, nch, tile_off, cmds, order);
+        launch(sig ? k_fine<T, NT, B, false, true> : k_fine<T, NT, B, false, false>);
 }
-template <int T>
-static void fine_words(hipStream_t s, bool ext, uint32_t words, uint32_t n_tiles, const TargetInfo *tg, uint32_t n_targets,
-                       const DrawPrep *dprep, const GradRec *grec, const vkh_gradient *grads, const GradPrep *gprep,
-                       const PathTile *pts, const Edge *segs, uint32_t nch, const uint32_t *tile_off,
-                       const Cmd *cmds, const uint32_t *order) {
-    switch (words) {
-    case 2048:
-        fine_launch<T, 2048>(s, ext, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    case 8192:
-        fine_launch<T, 8192>(s, ext, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    default:
-        fine_launch<T, 4096>(s, ext, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    }
+// Threads and commands rasterized at a time, from the row-delta words W of the capacity setting. Tiles
+// of 16: two wavefronts with half of W, so that 16 workgroups fit a CU's LDS; but a frame of at most
+// VKH_FINE_WIDE tiles (all resident at once: 256 CUs x 16) leaves the chip partly idle and each tile's
+// chain of commands sets its time, so it takes four wavefronts and all of W per tile (512x512 with 200
+// paths: 114 us with two wavefronts, 78 us with four; 8160 heavy tiles of the stroke scene: 2.3 against
+// 3.1 ms). Tiles of 8 (one wavefront) and 32 (four) take half of W: more workgroups per CU (1500x1500
+// dense scene, tile 8: 0.24 -> 0.13 ms).
+#define VKH_FINE_WIDE 4096
+template <int W, class... A>
+static void fine_words(hipStream_t s, bool ext, bool sig, uint32_t tile, uint32_t n_tiles, A... args) {
+    if (tile == 8)
+        fine_launch<8, 64, W / 128>(s, ext, sig, n_tiles, args...);
+    else if (tile == 32)
+        fine_launch<32, 256, W / 2048>(s, ext, sig, n_tiles, args...);
+    else if (n_tiles <= VKH_FINE_WIDE)
+        fine_launch<16, 256, W / 256>(s, ext, sig, n_tiles, args...);
+    else
+        fine_launch<16, 128, W / 512>(s, ext, sig, n_tiles, args...);
 }
-void launch_fine(hipStream_t s, bool ext, uint32_t tile, uint32_t words, uint32_t n_tiles, const TargetInfo *tg,
+void launch_fine(hipStream_t s, bool ext, bool sig, uint32_t tile, uint32_t words, uint32_t n_tiles, const TargetInfo *tg,
                  uint32_t n_targets, const DrawPrep *dprep, const GradRec *grec, const vkh_gradient *grads,
                  const GradPrep *gprep, const PathTile *pts, const Edge *segs, uint32_t nch,
                  const uint32_t *tile_off, const Cmd *cmds, const uint32_t *order) {
     if (!n_tiles)
         return;
-    switch (tile) {
-    case 8:
-        fine_words<8>(s, ext, words, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    case 32:
-        fine_words<32>(s, ext, words, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    default:
-        fine_words<16>(s, ext, words, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
-        break;
-    }
+    if (words == 2048)
+        fine_words<2048>(s, ext, sig, tile, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
+    else if (words == 8192)
+        fine_words<8192>(s, ext, sig, tile, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
+    else
+        fine_words<4096>(s, ext, sig, tile, n_tiles, tg, n_targets, dprep, grec, grads, gprep, pts, segs, nch, tile_off, cmds, order);
 }
 size_t order_words(uint32_t n) { return (size_t)n + VKH_ORDER_BUCKETS; }
 template <class W>
