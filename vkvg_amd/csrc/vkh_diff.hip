@@ -270,7 +270,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uin
     return total;
 }
 
-// Per tile the list holds the edges touching the tile's columns first (PathTile.reserved of
+// Per tile the list holds the edges touching the tile's columns first (PathTile.ntouch of
 // them), then the edges entirely left of it, which only carry their rows' dy.
 template <typename R>
 __device__ __forceinline__ int32_t last_touch_col(const RV4<R> &v) {
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_
             pt.backdrop = 0;
             pt.nseg = next - off;
             pt.seg_off = base + off;
-            pt.reserved = s_touch[k]; // edges touching the tile, listed first
+            pt.ntouch = s_touch[k]; // edges touching the tile, listed first
             out[k] = pt;
         }
         __syncthreads();
@@ -422,7 +422,7 @@ __device__ __forceinline__ void stage_batch(uint32_t base, uint32_t nb, const Cm
         const PathTile p = ptl[cm.pt];
         c_draw[tid] = cm.draw;
         c_nseg[tid] = p.nseg;
-        c_ntouch[tid] = p.reserved;
+        c_ntouch[tid] = p.ntouch;
         c_segoff[tid] = p.seg_off;
     }
     __syncthreads();
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void k_dcov(uint32_t n_cmds, uint32_t max_unit
             u_cmd[tid] = c;
             u_s0[tid] = s0;
             u_n[tid] = min(p.nseg - min(p.nseg, s0), (uint32_t)VKD_U);
-            u_nt[tid] = p.reserved;
+            u_nt[tid] = p.ntouch;
             u_off[tid] = p.seg_off;
             u_tile[tid] = cmd_tile[c];
             u_single[tid] = unit_off[c + 1] - unit_off[c] == 1u;

@@ -860,7 +860,7 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
         vkh::launch_bin_draws(s, P<Edge>(eng->edges), P<uint2>(eng->erange),
                               P<DrawTiles>(eng->dtiles), n_draws, T, P<PathTile>(eng->ptiles), P<Edge>(eng->segs),
                               seg_cap, P<uint32_t>(eng->counters), P<uint32_t>(eng->draw_order), d_draws, d_tg, nch,
-                              eng->coarse_chunk, P<uint32_t>(eng->tile_cnt));
+                              eng->coarse_chunk, P<uint32_t>(eng->tile_cnt), P<DrawPrep>(eng->dprep));
         CK(hipGetLastError());
         if (totals(eng, cap, {P<uint32_t>(eng->counters)}, tot, 8))
             return -1;

@@ -53,7 +53,10 @@ struct PathTile {
     int32_t backdrop;  // winding at the tile's first sample (after the row prefix sum)
     uint32_t nseg;     // edges touching the tile
     uint32_t seg_off;  // into the segment index array
-    uint32_t reserved; // keeps the record at 16 bytes
+    union {
+        uint32_t sat;    // rendering: the gradient's colour over the tile is its first (1) or last (2) stop's
+        uint32_t ntouch; // differentiable renderer: of the edges, how many touch the tile (listed first)
+    };
 };
 
 // per draw, computed once per frame: what the compositing loop needs, with the per-draw parts of
@@ -69,13 +72,12 @@ struct DrawPrep {
     uint32_t meta;   // kind | op << 4 | VKH_DP_GRAD
     uint32_t solid;  // premultiplied RGBA8 of a solid source, opacity applied
     uint32_t key;    // coverage-signature key of the draw
-    int32_t grad;    // gradient index or -1
-    float opacity;
-    uint32_t gflags; // VKH_GF_*
-    float g[6];      // gradient invariants: linear p0x, l, m, bb, sqrt(1+m*m); radial c0x, c0y, r0, dx, dy, cc
-    float rg[2];     // linear: vkh_rcp_for_div of g[1] and g[4] (0: divide per pixel)
-    uint32_t pad[2];
+    uint32_t sat;    // gradient source: VKH_GS_* of its test for tiles of constant colour (vkh_gradsat.h)
+    float s[6];      // ... and its terms
+    uint32_t first, last; // premultiplied RGBA8 of its first and last stop, opacity applied
+    uint32_t pad[4];
 };
+static_assert(sizeof(DrawPrep) == 64, "DrawPrep: one cache line half");
 
 // Per gradient: rspan[i] = vkh_rcp_for_div(stops[i] - stops[i-1]) for the colour step i >= 1
 struct GradPrep {
@@ -89,7 +91,9 @@ struct GradPrep {
 struct GradRec {
     uint32_t type, count, gflags;
     float opacity;
-    float g[6], rg[2];                   // as in DrawPrep
+    float g[6];                          // invariants: linear p0x, l, m, bb, sqrt(1+m*m); radial c0x, c0y, r0,
+                                         // dx, dy, cc
+    float rg[2];                         // linear: vkh_rcp_for_div of g[1] and g[4] (0: divide per pixel)
     float stops[VKH_GR_INLINE];
     float rspan[VKH_GR_INLINE];          // as in GradPrep
     float colors[VKH_GR_INLINE][4];
@@ -168,7 +172,8 @@ void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n);
 void launch_bin_draws(hipStream_t s, const Edge *edges, const uint2 *erange,
                       const DrawTiles *dt, uint32_t n_draws, uint32_t tile, PathTile *pts, Edge *segs,
                       uint32_t seg_cap, uint32_t *seg_alloc, const uint32_t *order, const vkh_draw *draws,
-                      const TargetInfo *tg, uint32_t nch, uint32_t chunk_draws, uint32_t *tile_cnt);
+                      const TargetInfo *tg, uint32_t nch, uint32_t chunk_draws, uint32_t *tile_cnt,
+                      const DrawPrep *dprep);
 void launch_tile_cnt_init(hipStream_t s, const TargetInfo *tg, uint32_t n_targets, uint32_t nch,
                           const uint32_t *table, uint32_t *tile_cnt, uint32_t n_tc);
 void launch_draw_prep(hipStream_t s, const vkh_draw *draws, uint32_t n_draws, const TargetInfo *tg,

@@ -16,6 +16,7 @@
 #include "vkh_blend.h"
 #include "vkh_fdiv.h"
 #include "vkh_cross.h"
+#include "vkh_gradsat.h"
 
 #include <hip/hip_runtime.h>
 
@@ -210,7 +211,8 @@ __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges
                                                   uint32_t seg_cap, uint32_t *__restrict__ seg_alloc,
                                                   const uint32_t *__restrict__ draw_order,
                                                   const vkh_draw *__restrict__ draws, const TargetInfo *__restrict__ tg,
-                                                  uint32_t nch, uint32_t chunk_draws, uint32_t *__restrict__ tile_cnt) {
+                                                  uint32_t nch, uint32_t chunk_draws, uint32_t *__restrict__ tile_cnt,
+                                                  const DrawPrep *__restrict__ dprep) {
     __shared__ uint32_t s_cnt[VKH_BIN_LDS_TILES];
     __shared__ int32_t s_back[VKH_BIN_LDS_TILES];
     __shared__ uint32_t s_wave[4];
@@ -224,6 +226,12 @@ __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges
     const vkh_draw &dr = draws[d];
     const uint32_t kind = dr.kind;
     const bool clip = kind_is_clip(kind);
+    // A gradient's tiles of constant colour are marked here, where the draw's terms are uniform over the
+    // workgroup (per command in the fine kernel the test cost that kernel registers): the fine kernel
+    // then blends them as a solid source instead of some 100 (linear) to 200 (radial) vector
+    // instructions per wave and command. 4096x4096 dense scene, 30 % gradients: fine kernel
+    // 1.56 -> 1.39 ms, binning 0.464 -> 0.474 ms.
+    const uint32_t sat = dprep[d].sat;
     const TargetInfo &TI = tg[dr.target];
     const uint32_t chunk = (d - TI.draw_begin) / chunk_draws;
     const uint32_t bw = dt.bw, bh = (uint32_t)(dt.by1 - dt.by0 + 1);
@@ -291,10 +299,17 @@ __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges
             p.backdrop = s_back[k];
             p.nseg = next - off;
             p.seg_off = base + off;
-            p.reserved = 0;
+            const uint32_t r = k / bw, c = k - r * bw;
+            p.sat = 0;
+            if (sat) {
+                const int32_t x = (dt.bx0 + (int32_t)c) << lt, y = (ty_lo + (int32_t)r) << lt;
+                p.sat = (uint32_t)vkh_grad_sat_tile(
+                    sat, dprep[d].s, (float)x + 0.5f, (float)y + 0.5f,
+                    (float)min(x + (1 << lt), (int32_t)TI.width) - 0.5f,
+                    (float)min(y + (1 << lt), (int32_t)TI.height) - 0.5f, (float)TI.width, (float)TI.height);
+            }
             out[k] = p;
             if (p.nseg || clip || coverage_count(kind, p.backdrop) != 0) {
-                const uint32_t r = k / bw, c = k - r * bw;
                 const uint32_t gtile = TI.tile_base + (uint32_t)(ty_lo + (int32_t)r) * TI.tilesW + (uint32_t)dt.bx0 + c;
                 atomicAdd(&tile_cnt[(size_t)gtile * nch + chunk], 1u);
             }
@@ -412,7 +427,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_sgpr(80))) void k_co
             for (int u = 0; u < 4; u++) {
                 in[u] = false;
                 ptid[u] = VKH_NO_DRAW;
-                p[u] = PathTile{0, 0, 0, 0};
+                p[u] = PathTile{};
                 const uint32_t h = h0 + (uint32_t)u;
                 if (h < nh && valid) {
                     const DrawTiles hb = s_dt[h];
@@ -553,8 +568,6 @@ __global__ void k_draw_prep(const vkh_draw *__restrict__ draws, uint32_t n, cons
     const bool surf = d.source >= 0 && kind <= VKH_DRAW_PAINT; // fills, strokes, paint
     p.meta = kind | (op << 4) | (surf ? VKH_DP_SURF : (d.grad >= 0 ? VKH_DP_GRAD : 0u));
     p.key = draw_key(d.key_index);
-    p.grad = d.grad;
-    p.opacity = d.opacity;
     const uint32_t c = d.color;
     const float o = d.opacity;
     p.solid = (uint32_t)f2u8(((float)(c & 0xFF) / 255.0f) * o) |
@@ -563,58 +576,54 @@ __global__ void k_draw_prep(const vkh_draw *__restrict__ draws, uint32_t n, cons
               ((uint32_t)f2u8(((float)((c >> 24) & 0xFF) / 255.0f) * o) << 24);
     if (kind >= VKH_DRAW_CLIP_SAVE)
         p.solid = (uint32_t)d.style; // the saved bit or copy index of a stencil draw
-    p.gflags = 0;
+    p.sat = VKH_GS_NONE;
     for (int k = 0; k < 6; k++)
-        p.g[k] = 0.f;
-    p.rg[0] = p.rg[1] = 0.f;
-    p.pad[0] = p.pad[1] = 0;
+        p.s[k] = 0.f;
+    p.first = p.last = 0;
+    for (int k = 0; k < 4; k++)
+        p.pad[k] = 0;
     if (d.grad >= 0) {
         const vkh_gradient &g = grads[d.grad];
         const float W = (float)tg[d.target].width, H = (float)tg[d.target].height;
+        GradRec r;
+        r.type = g.type;
+        r.count = g.count;
+        r.gflags = 0;
+        r.opacity = o;
+        for (int k = 0; k < 6; k++)
+            r.g[k] = 0.f;
+        r.rg[0] = r.rg[1] = 0.f;
         if (g.type == 2) {
             float p0x = g.cp[0][0] / W, p0y = g.cp[0][1] / H;
             float p1x = g.cp[0][2] / W, p1y = g.cp[0][3] / H;
             float dx = p1x - p0x, dy = p1y - p0y;
             float l = sqrtf(dx * dx + dy * dy);
             float ux = dx / l, uy = dy / l;
-            p.g[0] = p0x;
-            p.g[1] = l;
+            r.g[0] = p0x;
+            r.g[1] = l;
             if (uy == 0) {
-                p.gflags = VKH_GF_UY0 | (ux < 0 ? VKH_GF_UXNEG : 0u);
+                r.gflags = VKH_GF_UY0 | (ux < 0 ? VKH_GF_UXNEG : 0u);
             } else {
                 float m = -ux / uy;
-                p.g[2] = m;
-                p.g[3] = p0y - m * p0x;
-                p.g[4] = sqrtf(1 + m * m);
-                p.gflags = uy < 0 ? VKH_GF_UYNEG : 0u;
-                p.rg[1] = vkh_rcp_for_div(p.g[4]);
+                r.g[2] = m;
+                r.g[3] = p0y - m * p0x;
+                r.g[4] = sqrtf(1 + m * m);
+                r.gflags = uy < 0 ? VKH_GF_UYNEG : 0u;
+                r.rg[1] = vkh_rcp_for_div(r.g[4]);
             }
-            p.rg[0] = vkh_rcp_for_div(l);
+            r.rg[0] = vkh_rcp_for_div(l);
         } else {
             float c0x = g.cp[0][0] / W, c0y = g.cp[0][1] / H;
             float c1x = g.cp[1][0] / W, c1y = g.cp[1][1] / H;
             float r0 = g.cp[0][2] / W, r1 = g.cp[1][2] / W;
             float diffx = c0x - c1x, diffy = c0y - c1y;
-            p.g[0] = c0x;
-            p.g[1] = c0y;
-            p.g[2] = r0;
-            p.g[3] = diffx;
-            p.g[4] = diffy;
-            p.g[5] = (diffx * diffx + diffy * diffy) - r1 * r1;
+            r.g[0] = c0x;
+            r.g[1] = c0y;
+            r.g[2] = r0;
+            r.g[3] = diffx;
+            r.g[4] = diffy;
+            r.g[5] = (diffx * diffx + diffy * diffy) - r1 * r1;
         }
-    }
-    out[i] = p;
-    if (d.grad >= 0) {
-        const vkh_gradient &g = grads[d.grad];
-        GradRec r;
-        r.type = g.type;
-        r.count = g.count;
-        r.gflags = p.gflags;
-        r.opacity = p.opacity;
-        for (int k = 0; k < 6; k++)
-            r.g[k] = p.g[k];
-        r.rg[0] = p.rg[0];
-        r.rg[1] = p.rg[1];
         for (int k = 0; k < VKH_GR_INLINE; k++) {
             r.stops[k] = g.stops[k];
             r.rspan[k] = k ? vkh_rcp_for_div(g.stops[k] - g.stops[k - 1]) : 0.f;
@@ -624,7 +633,17 @@ __global__ void k_draw_prep(const vkh_draw *__restrict__ draws, uint32_t n, cons
         r.grad = d.grad;
         r.pad[0] = r.pad[1] = r.pad[2] = 0;
         rec[i] = r;
+        const vkh_grad_sat gs = vkh_grad_sat_of(&g, W, H);
+        if (gs.type != VKH_GS_NONE) {
+            const float *a = g.colors[0], *z = g.colors[g.count - 1];
+            p.sat = gs.type;
+            for (int k = 0; k < 6; k++)
+                p.s[k] = gs.s[k];
+            p.first = f2u8x4(a[0] * o, a[1] * o, a[2] * o, a[3] * o);
+            p.last = f2u8x4(z[0] * o, z[1] * o, z[2] * o, z[3] * o);
+        }
     }
+    out[i] = p;
     if (surf) {
         const vkh_surface_source &src = srcs[d.source];
         SurfRec r;
@@ -963,6 +982,7 @@ void k_fine(const TargetInfo *__restrict__ tg, uint32_t n_targets,
                     uint32_t meta = d.meta;
                     const uint32_t kind = meta & 15;
                     unit = kind == VKH_DRAW_FILL_EO || kind == VKH_DRAW_CLIP_EO ? 0x80000000u : 1u;
+                    uint32_t solid = d.solid;
                     uint4 rec;
                     if (cm.pt == VKH_NO_DRAW) {
                         if (kind <= VKH_DRAW_CLEAR)
@@ -973,15 +993,19 @@ void k_fine(const TargetInfo *__restrict__ tg, uint32_t n_targets,
                         rec.z = (uint32_t)p.backdrop * unit;
                         nseg = p.nseg;
                         segoff = p.seg_off;
+                        if (p.sat) { // a gradient that is constant over the tile is a solid source
+                            solid = p.sat == 1u ? d.first : d.last;
+                            meta &= ~VKH_DP_GRAD;
+                        }
                     }
-                    rec.x = meta;
                     rec.y = d.key;
                     rec.w = d.solid; // the parameter of a stencil draw
-                    c_rec[j] = rec;
-                    const vkh_src16 Sc = vkh_src16_of((meta >> 4) & 15, d.solid);
+                    rec.x = meta;
+                    const vkh_src16 Sc = vkh_src16_of((meta >> 4) & 15, solid);
                     uint4 sv = make_uint4(vkh_u32_of(Sc.ia), vkh_u32_of(Sc.b_lo), vkh_u32_of(Sc.b_hi), Sc.x);
                     if (meta & (VKH_DP_GRAD | VKH_DP_SURF))
                         sv.x = cm.draw;
+                    c_rec[j] = rec;
                     c_src[j] = sv;
                 }
                 uint32_t incl = nseg;
@@ -1250,10 +1274,11 @@ void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n) {
 void launch_bin_draws(hipStream_t s, const Edge *edges, const uint2 *erange,
                       const DrawTiles *dt, uint32_t n_draws, uint32_t tile, PathTile *pts, Edge *segs,
                       uint32_t seg_cap, uint32_t *seg_alloc, const uint32_t *order, const vkh_draw *draws,
-                      const TargetInfo *tg, uint32_t nch, uint32_t chunk_draws, uint32_t *tile_cnt) {
+                      const TargetInfo *tg, uint32_t nch, uint32_t chunk_draws, uint32_t *tile_cnt,
+                      const DrawPrep *dprep) {
     if (n_draws)
         hipLaunchKernelGGL(k_bin_draw, dim3(n_draws), dim3(256), 0, s, edges, erange, dt, tile, pts, segs,
-                           seg_cap, seg_alloc, order, draws, tg, nch, chunk_draws, tile_cnt);
+                           seg_cap, seg_alloc, order, draws, tg, nch, chunk_draws, tile_cnt, dprep);
 }
 void launch_tile_cnt_init(hipStream_t s, const TargetInfo *tg, uint32_t n_targets, uint32_t nch,
                           const uint32_t *table, uint32_t *tile_cnt, uint32_t n_tc) {
