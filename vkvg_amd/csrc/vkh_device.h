@@ -45,6 +45,12 @@ VKH_HD bool equf(float a, float b) { return fabsf(a - b) <= VKH_FLT_EPSILON; }
 VKH_HD float d_atan2f(float y, float x) { return (float)atan2((double)y, (double)x); }
 VKH_HD float d_cosf(float a) { return (float)cos((double)a); }
 VKH_HD float d_sinf(float a) { return (float)sin((double)a); }
+VKH_HD void d_sincosf(float a, float *s, float *c) {
+    double ds, dc;
+    sincos((double)a, &ds, &dc);
+    *s = (float)ds;
+    *c = (float)dc;
+}
 VKH_HD float d_acosf(float a) { return (float)acos((double)a); }
 
 // ---------------------------------------------------------------------------------------
@@ -471,12 +477,14 @@ VKH_HD int f32_lowbit(float v) {
 
 struct DashPeriod {
     double sum; // exact sum of the dashes
+    double rcp; // 1 / sum, rounded down by more than its error
     int lowbit; // lowest set bit over the non-zero dashes
     bool ok;    // dashes finite, >= 0, with a non-zero exact sum
+    float reach; // offsets from here on have no exact addition (2^(lowbit + 24); 0 when not ok)
 };
 
 VKH_HD DashPeriod dash_period(const float *dashes, uint32_t n) {
-    DashPeriod p{0.0, 1 << 20, n > 0};
+    DashPeriod p{0.0, 0.0, 1 << 20, n > 0, 0.f};
     for (uint32_t i = 0; i < n; i++) {
         const float v = dashes[i];
         if (!(v >= 0.f) || !(v <= 3.0e38f)) {
@@ -490,15 +498,18 @@ VKH_HD DashPeriod dash_period(const float *dashes, uint32_t n) {
     // every partial sum is a multiple of 2^lowbit; below 2^(lowbit + 52) the double additions were exact
     if (!(p.sum > 0.0) || !(p.sum < ldexp(1.0, p.lowbit + 52)))
         p.ok = false;
+    p.rcp = p.ok ? (1.0 / p.sum) * (1.0 - 0x1p-50) : 0.0;
+    p.reach = p.ok ? ldexpf(1.f, p.lowbit + 24 < 127 ? p.lowbit + 24 : 127) : 0.f;
     return p;
 }
 
 // Whole periods the loop takes from offset off < segLen with every float addition exact and every
-// offset before an addition below segLen: the largest k with off + k * sum < min(2^(g+24), segLen).
+// offset before an addition below segLen: the largest k (or one less) with off + k * sum < min(2^(g+24), segLen).
 // (A k of at least 1 needs sum < 2^(g+24), so off + k * sum is a multiple of 2^g below 2^(g+25) and
-// exact in double; the quotient's rounding is corrected by the exact test.)
+// exact in double; the exact test corrects the quotient. One period less than that is as exact.)
 VKH_HD uint32_t dash_whole_periods(const DashPeriod &p, float off, float segLen) {
-    if (!p.ok || !(off >= 0.f))
+    // beyond reach no addition is exact; less than a period left
+    if (!(off >= 0.f) || off >= p.reach || !((double)segLen - (double)off > p.sum))
         return 0;
     int g = p.lowbit;
     if (off > 0.f) {
@@ -509,12 +520,15 @@ VKH_HD uint32_t dash_whole_periods(const DashPeriod &p, float off, float segLen)
     const double room = lim - (double)off;
     if (!(room > p.sum))
         return 0;
-    const double kd = floor(room / p.sum);
+    const double kd = floor(room * p.rcp); // at most the quotient's floor, at least one less
     uint32_t k = kd < 16777216.0 ? (uint32_t)kd : 16777216u;
     if ((double)off + (double)k * p.sum >= lim)
         k--;
     return k;
 }
+
+// fmodf(x, y) without its reduction loop where x is already reduced
+VKH_HD float dash_mod(float x, float y) { return fabsf(x) < y ? x : fmodf(x, y); }
 
 // The loop over one segment: advances (on, cur, off) and returns the number of caps it makes. On a
 // segment some 2^24 dash lengths long or longer the offset's float additions stop advancing it
@@ -524,6 +538,7 @@ VKH_HD uint32_t dash_whole_periods(const DashPeriod &p, float off, float segLen)
 VKH_HD uint32_t dash_walk_segment(const float *dashes, uint32_t n, const DashPeriod &p, float segLen, bool &on,
                                   uint32_t &cur, float &off, bool &over) {
     uint32_t caps = 0;
+    float v = dashes[cur]; // the next dash is read ahead of the addition that the loop waits for
     while (off < segLen) {
         if (caps >= VKH_DASH_MAX_CAPS) {
             over = true;
@@ -538,9 +553,10 @@ VKH_HD uint32_t dash_walk_segment(const float *dashes, uint32_t n, const DashPer
             on = on != (((w * n) & 1u) != 0);
         }
         on = !on;
-        off += dashes[cur];
+        off += v;
         if (++cur == n)
             cur = 0;
+        v = dashes[cur];
         caps++;
     }
     return caps;

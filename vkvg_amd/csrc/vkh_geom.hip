@@ -545,36 +545,14 @@ struct DashState {
     v2 normal;
 };
 
-// _draw_dashed_segment, src/vkvg_context_internal.c:1240-1264
-template <typename S>
-__device__ void dashed_segment(const StrokeCtx &c, S &s, DashState &dc, uint32_t iL, uint32_t cp, uint32_t iR,
-                               bool isCurve) {
-    v2 p = c.P[cp];
-    v2 pR = c.P[iR];
-    if (!dc.dashOn)
-        vb_step(c, s, iL, cp, iR, isCurve);
-    v2 d = vsub(pR, p);
-    dc.normal = vnorm(d);
-    float segLen = vlen(d);
-    while (dc.curDashOffset < segLen) {
-        v2 p0 = vadd(p, vmul(dc.normal, dc.curDashOffset));
-        stroke_cap(c, s, p0, dc.normal, dc.dashOn);
-        dc.dashOn = !dc.dashOn;
-        dc.curDashOffset += c.dashes[dc.curDash];
-        if (++dc.curDash == c.dashCount)
-            dc.curDash = 0;
-    }
-    dc.curDashOffset -= segLen;
-    dc.curDashOffset = fmodf(dc.curDashOffset, dc.totDashLength);
-}
-
 // A dashed sub-path of _stroke_preserve (src/vkvg_context.c:836-945) in pieces: piece k < last is
-// the dashed segment from point k (iL is the last point for k = 0, as there), a closed path adds
-// the closing segment as piece `last`, and the last piece also emits the final cap. Run one after
-// another over all pieces, dash_start / dash_piece perform the reference's operations in its order;
-// k_dash_walk records the dash state at each piece's start so that the pieces can be counted (one
-// thread each, dash_piece_count) and emitted independently: by one thread each (k_stroke_steps),
-// or, for a piece of many caps, by a wavefront (k_dash_pieces).
+// the dashed segment (_draw_dashed_segment, src/vkvg_context_internal.c:1240-1264) from point k (iL is
+// the last point for k = 0, as there), a closed path adds the closing segment as piece `last`, and the
+// last piece also emits the final cap. A piece emits a join at its start point if it starts inside a
+// gap, then a cap at every dash boundary within its length (stroke_cap); k_dash_walk records the dash
+// state at each piece's start so that the pieces can be counted (one thread each, dash_piece_count)
+// and emitted independently: by one thread each (dash_piece_emit in k_stroke_steps), or, for a piece
+// of many caps, by a wavefront (k_dash_pieces). Every value takes the reference's float operations.
 __device__ __forceinline__ uint32_t dash_pieces(uint32_t n, bool closed) { return n < 2 ? 0u : (closed ? n : n - 1); }
 
 __device__ __forceinline__ DashState dash_start(const StrokeCtx &c, float dashOffset) {
@@ -584,7 +562,7 @@ __device__ __forceinline__ DashState dash_start(const StrokeCtx &c, float dashOf
     dc.totDashLength = 0;
     for (uint32_t i = 0; i < c.dashCount; i++)
         dc.totDashLength += c.dashes[i];
-    dc.curDashOffset = fmodf(dashOffset, dc.totDashLength);
+    dc.curDashOffset = dash_mod(dashOffset, dc.totDashLength);
     dc.normal = V(0, 0);
     return dc;
 }
@@ -619,68 +597,186 @@ __device__ void dash_final_cap(const StrokeCtx &c, S &s, DashState &dc, uint32_t
     stroke_cap(c, s, p, dc.normal, false);
 }
 
-// piece k in one thread, in the reference's order of operations
-template <typename S>
-__device__ void dash_piece(const StrokeCtx &c, bool closed, uint32_t k, DashState &dc, S &s) {
-    uint32_t iL, cp, iR;
-    bool curved;
-    dash_piece_points(c, k, iL, cp, iR, curved);
-    dashed_segment(c, s, dc, iL, cp, iR, curved);
-    if (k + 1 == dash_pieces(c.n, closed) && !dc.dashOn)
-        dash_final_cap(c, s, dc, iR);
-}
-
-// The dash state after piece k without emitting anything: dashed_segment's state updates only
-// (the join and caps it emits do not change the state), with the same float operations.
+// The dash state after a piece of length segLen without emitting anything: dashed_segment's state
+// updates only (the join and caps it emits do not change the state), with the same float operations.
 // Returns the number of caps the piece emits (the loop's iterations).
-__device__ __forceinline__ uint32_t dash_walk_piece(const StrokeCtx &c, const DashPeriod &per, uint32_t k,
+__device__ __forceinline__ uint32_t dash_walk_piece(const StrokeCtx &c, const DashPeriod &per, float segLen,
                                                    DashState &dc, bool &over) {
-    const uint32_t last = c.n - 1;
-    const uint32_t cp = k < last ? k : last, iR = k < last ? k + 1 : 0;
-    v2 d = vsub(c.P[iR], c.P[cp]);
-    float segLen = vlen(d);
     const uint32_t caps =
         dash_walk_segment(c.dashes, c.dashCount, per, segLen, dc.dashOn, dc.curDash, dc.curDashOffset, over);
     dc.curDashOffset -= segLen;
-    dc.curDashOffset = fmodf(dc.curDashOffset, dc.totDashLength);
+    dc.curDashOffset = dash_mod(dc.curDashOffset, dc.totDashLength);
     return caps;
 }
 
-// The vertex and index counts of piece k (dash_piece's) from its start state, without running its
-// caps one by one: a cap's counts depend only on whether it starts or ends a dash and on the
-// piece's direction (a round cap's arc steps run from the direction's angle; the cap's position
-// does not enter), the caps alternate between the two from the start state, and the dash walk
-// gives their number and the state the piece ends in.
-__device__ void dash_piece_count(const StrokeCtx &c, const DashPeriod &per, bool closed, uint32_t k, DashState dc,
+// The vertex and index counts of piece k from its start state dc and its number of caps (both from the
+// dash walk), without running the caps: a cap's counts depend only on whether it starts or ends a dash
+// and on the piece's direction (a round cap's arc steps run from the direction's angle; the cap's
+// position does not enter), and the caps alternate between the two from the start state.
+__device__ void dash_piece_count(const StrokeCtx &c, bool closed, uint32_t k, const DashState &dc, uint32_t caps,
                                  CountSink &s) {
     uint32_t iL, cp, iR;
     bool curved;
     dash_piece_points(c, k, iL, cp, iR, curved);
     if (!dc.dashOn)
         vb_step(c, s, iL, cp, iR, curved);
-    const v2 d = vsub(c.P[iR], c.P[cp]);
-    const v2 n = vnorm(d);
-    const float segLen = vlen(d);
-    const bool on0 = dc.dashOn;
-    bool over = false; // the dash walk of the same piece has flagged the frame
-    const uint32_t caps =
-        dash_walk_segment(c.dashes, c.dashCount, per, segLen, dc.dashOn, dc.curDash, dc.curDashOffset, over);
+    const v2 n = vnorm(vsub(c.P[iR], c.P[cp]));
     CountSink cs, ce;
     stroke_cap(c, cs, V(0.f, 0.f), n, true);
     stroke_cap(c, ce, V(0.f, 0.f), n, false);
-    const uint32_t starts = on0 ? (caps + 1) / 2 : caps / 2, ends = caps - starts;
+    const uint32_t starts = dc.dashOn ? (caps + 1) / 2 : caps / 2, ends = caps - starts;
     s.nv += starts * cs.nv + ends * ce.nv;
     s.ni += starts * cs.ni + ends * ce.ni;
-    if (k + 1 == dash_pieces(c.n, closed) && !dc.dashOn) { // the final cap ends a dash
+    const bool end_on = dc.dashOn == ((caps & 1) == 0);
+    if (k + 1 == dash_pieces(c.n, closed) && !end_on) { // the final cap ends a dash
         s.nv += ce.nv;
         s.ni += ce.ni;
     }
 }
 
+// The caps of one piece. They all have the piece's direction, so a round cap's arc angles (the loops of
+// stroke_cap) are the same for every start cap and for every end cap of the piece: their sines and
+// cosines (in double, some 100 instructions per vertex) are evaluated once per piece, and a cap is
+// then its position plus these offsets. Caps alternate between start and end, so the place of
+// cap j's vertices and triangles follows from j.
+struct DashCaps {
+    v2 p, n;              // the piece's start point and direction
+    float hw, step;       // half width, arc step
+    int cap;
+    uint32_t ks, ke;      // arc vertices of a start and of an end cap
+    bool on0;             // cap 0 starts a dash
+    // vertices and triangles of a start cap (arc, then 2 vertices; arc fan, then 2 triangles to the
+    // next cap's first two vertices) and of an end cap (2 vertices, then the arc; its fan)
+    __device__ uint32_t nv(bool start) const { return 2 + (start ? ks : ke); }
+    __device__ uint32_t nt(bool start) const { return start ? ks + 2 : ke; }
+    __device__ bool start(uint32_t j) const { return on0 == ((j & 1) == 0); }
+    __device__ uint32_t starts(uint32_t j) const { return on0 ? (j + 1) / 2 : j / 2; } // start caps before cap j
+    __device__ uint32_t nv_before(uint32_t j) const { return starts(j) * nv(true) + (j - starts(j)) * nv(false); }
+    __device__ uint32_t nt_before(uint32_t j) const { return starts(j) * nt(true) + (j - starts(j)) * nt(false); }
+    __device__ v2 at(float off) const { return vadd(p, vmul(n, off)); } // a cap's position
+    // the first or second vertex of the pair of a cap at p0
+    __device__ v2 side(bool start, v2 p0, bool second) const {
+        v2 vhw = vmul(n, hw);
+        if (cap == 2)
+            p0 = start ? vsub(p0, vhw) : vadd(p0, vhw);
+        vhw = vperp(vhw);
+        return second ? vsub(p0, vhw) : vadd(p0, vhw);
+    }
+    // the arc vertex of a cap at p0 with cos and sin times the half width cx, sy
+    __device__ static v2 arc(v2 p0, float cx, float sy) { return V(cx + p0.x, sy + p0.y); }
+    // triangle t of a cap whose first vertex is f
+    __device__ void tri(bool start, uint32_t f, uint32_t t, uint32_t *o) const {
+        if (start) {
+            const uint32_t q = f + ks; // the pair
+            o[0] = t < ks ? q + 1 : t == ks ? q : q + 1;
+            o[1] = t < ks ? f + t : q + 2;
+            o[2] = t < ks ? f + t + 1 : t == ks ? q + 1 : q + 3;
+        } else {
+            o[0] = f + 2 + t;
+            o[1] = f + 1 + t;
+            o[2] = f;
+        }
+    }
+};
+
+// the first angle of a round cap's arc (one step before its first vertex) and its end
+__device__ __forceinline__ float dash_arc_angle(v2 n, bool start, float &a1) {
+    float a = d_acosf(n.x) + VKH_PIF_2;
+    if (n.y < 0)
+        a = VKH_PIF - a;
+    a1 = start ? a + VKH_PIF : a - VKH_PIF;
+    return a;
+}
+// arc vertices of a round cap: the angles a + step, a + 2 step, ... (float additions) before a1
+__device__ __forceinline__ uint32_t dash_arc_count(float a, float a1, bool start, float step) {
+    uint32_t k = 0;
+    for (a = start ? a + step : a - step; start ? a < a1 : a > a1; a = start ? a + step : a - step)
+        k++;
+    return k;
+}
+
 // A piece's start state: dashOn in bit 0, the dash index above it, and in bit 31 whether the piece
 // has enough caps to be emitted by a whole wavefront (k_dash_pieces) rather than by one thread.
 #define VKH_DASH_WAVE_BIT 0x80000000u
-#define VKH_DASH_WAVE_MIN 64 // caps from which a piece is given a wavefront
+// Caps from which a piece is given a wavefront: a wavefront's set-up costs about as much as a thread's
+// work on some 16 caps when the pieces fill the chip; with few pieces only the longest chain counts.
+#ifndef VKH_DASH_WAVE_MIN
+#define VKH_DASH_WAVE_MIN 16
+#endif
+#define VKH_DASH_WAVE_MIN_FEW 4
+#define VKH_DASH_FEW 16384 // stroke steps up to which a frame counts as having few pieces
+static_assert(VKH_DASH_WAVE_MIN_FEW <= VKH_DASH_WAVE_MIN, "the caps of a thread's piece fit its row of offsets");
+
+// A piece of fewer than VKH_DASH_WAVE_MIN caps emitted by one thread: the dash offsets of its caps go to the thread's row offs (stride lanes apart), then every arc angle is
+// evaluated once and written for all caps.
+__device__ void dash_piece_emit(const StrokeCtx &c, bool closed, uint32_t k, DashState dc, EmitSink s, float *offs,
+                                uint32_t stride) {
+    uint32_t iL, cp, iR;
+    bool curved;
+    dash_piece_points(c, k, iL, cp, iR, curved);
+    if (!dc.dashOn)
+        vb_step(c, s, iL, cp, iR, curved);
+    DashCaps C;
+    C.p = c.P[cp];
+    const v2 d = vsub(c.P[iR], C.p);
+    C.n = vnorm(d);
+    C.hw = c.hw;
+    C.step = c.arcStep;
+    C.cap = c.cap;
+    C.ks = C.ke = 0;
+    C.on0 = dc.dashOn;
+    dc.normal = C.n;
+    const float segLen = vlen(d);
+    uint32_t m = 0;
+    while (dc.curDashOffset < segLen && m < VKH_DASH_WAVE_MIN) {
+        offs[m * stride] = dc.curDashOffset;
+        m++;
+        dc.dashOn = !dc.dashOn;
+        dc.curDashOffset += c.dashes[dc.curDash];
+        if (++dc.curDash == c.dashCount)
+            dc.curDash = 0;
+    }
+    dc.curDashOffset -= segLen;
+    dc.curDashOffset = dash_mod(dc.curDashOffset, dc.totDashLength);
+    float a0 = 0.f, a1s = 0.f, a1e = 0.f;
+    if (c.cap == 1) {
+        a0 = dash_arc_angle(C.n, true, a1s);
+        dash_arc_angle(C.n, false, a1e);
+        C.ks = dash_arc_count(a0, a1s, true, C.step);
+        C.ke = dash_arc_count(a0, a1e, false, C.step);
+    }
+    const uint32_t nv = s.nv;
+    uint32_t *idx = s.idx + s.ni;
+    for (int w = 0; w < 2; w++) { // the arcs of the start caps, then of the end caps
+        const bool st = w == 0;
+        const uint32_t n = st ? C.ks : C.ke, at = st ? 0u : 2u;
+        float a = a0;
+        for (uint32_t i = 0; i < n; i++) {
+            a = st ? a + C.step : a - C.step;
+            float sy, cx;
+            d_sincosf(a, &sy, &cx);
+            cx *= C.hw;
+            sy *= C.hw;
+            for (uint32_t j = st == C.on0 ? 0 : 1; j < m; j += 2)
+                s.verts[nv + C.nv_before(j) + at + i] = C.arc(C.at(offs[j * stride]), cx, sy);
+        }
+    }
+    for (uint32_t j = 0; j < m; j++) {
+        const bool st = C.start(j);
+        const uint32_t f = nv + C.nv_before(j), q = f + (st ? C.ks : 0u);
+        const v2 p0 = C.at(offs[j * stride]);
+        s.verts[q] = C.side(st, p0, false);
+        s.verts[q + 1] = C.side(st, p0, true);
+        uint32_t *o = idx + 3 * C.nt_before(j);
+        for (uint32_t t = 0; t < C.nt(st); t++)
+            C.tri(st, f, t, o + 3 * t);
+    }
+    s.nv += C.nv_before(m);
+    s.ni += 3 * C.nt_before(m);
+    if (k + 1 == dash_pieces(c.n, closed) && !dc.dashOn)
+        dash_final_cap(c, s, dc, iR);
+}
+
 __device__ __forceinline__ uint2 dash_pack(const DashState &dc, bool wave) {
     return make_uint2((dc.dashOn ? 1u : 0u) | (dc.curDash << 1) | (wave ? VKH_DASH_WAVE_BIT : 0u),
                       __float_as_uint(dc.curDashOffset));
@@ -790,7 +886,8 @@ __global__ void k_dash_walk(const Unit *__restrict__ units, uint32_t n_units, co
                             const uint32_t *__restrict__ sp_first, const uint32_t *__restrict__ sp_count,
                             const v2 *__restrict__ pts, const uint8_t *__restrict__ pf,
                             const vkh_stroke_style *__restrict__ styles, const float *__restrict__ dashes,
-                            uint2 *__restrict__ dash_st, uint4 *__restrict__ dlist, uint32_t *__restrict__ dcount) {
+                            uint2 *__restrict__ dash_st, uint32_t *__restrict__ step_caps, uint32_t *__restrict__ dcount,
+                            uint32_t wave_min) {
     __shared__ float s_dash[256 * VKH_DASH_ROW];
     const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
     if (u >= n_units)
@@ -808,55 +905,56 @@ __global__ void k_dash_walk(const Unit *__restrict__ units, uint32_t n_units, co
     StrokeCtx c = make_stroke_ctx(st, dashes, pts, pf, sp_first[un.subpath], sp_count[un.subpath]);
     stage_dashes(c, s_dash);
     const DashPeriod per = dash_period(c.dashes, c.dashCount);
-    // pieces of many caps join the list that k_dash_pieces takes a wavefront per entry from
     DashState dc = dash_start(c, st.dash_offset);
     // a segment too long for its dash pattern stops the walk and refuses the frame (dcount[1]); the
     // later pieces keep the last state (a valid dash index), so their counting ends at once
     bool over = false;
-    for (uint32_t k = 0; k < s1 - s0; k++) {
-        const DashState d0 = dc;
-        const uint32_t caps = over ? 0u : dash_walk_piece(c, per, k, dc, over);
-        const bool wave = !over && caps >= VKH_DASH_WAVE_MIN;
-        dash_st[s0 + k] = dash_pack(d0, wave);
-        if (wave)
-            dlist[atomicAdd(dcount, 1u)] = make_uint4(s0 + k, caps, u, 0u);
+    // The walk is one chain of float additions per sub-path. The points are loaded eight pieces ahead (one
+    // load per piece in the chain made it 1 us a piece), and the dashes one step ahead.
+    const uint32_t last = c.n - 1, n = s1 - s0;
+    constexpr uint32_t AHEAD = 8;
+    v2 from = c.P[0], next[AHEAD];
+    auto fetch = [&](uint32_t k0) {
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; i++)
+            next[i] = c.P[k0 + i + 1 <= last ? k0 + i + 1 : 0]; // the closing piece ends at point 0
+    };
+    fetch(0);
+    for (uint32_t k0 = 0; k0 < n; k0 += AHEAD) {
+        v2 to[AHEAD];
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; i++)
+            to[i] = next[i];
+        fetch(k0 + AHEAD);
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; i++) {
+            if (k0 + i >= n)
+                break;
+            const DashState d0 = dc;
+            const uint32_t caps = over ? 0u : dash_walk_piece(c, per, vlen(vsub(to[i], from)), dc, over);
+            dash_st[s0 + k0 + i] = dash_pack(d0, !over && caps >= wave_min);
+            step_caps[s0 + k0 + i] = caps;
+            from = to[i];
+        }
     }
     if (over)
         atomicOr(dcount + 1, 1u);
 }
 
-// The dash updates of dashed_segment's loop without the cap: the state at the next boundary
-__device__ __forceinline__ void dash_advance(const StrokeCtx &c, float dreg, DashState &dc) {
-    dc.dashOn = !dc.dashOn;
-    dc.curDashOffset += c.dashCount <= 64 ? __shfl(dreg, (int)dc.curDash) : c.dashes[dc.curDash];
-    if (++dc.curDash == c.dashCount)
-        dc.curDash = 0;
-}
-
-// wave-wide exclusive prefix sum of v (all 64 lanes active); total in *tot
-__device__ __forceinline__ uint32_t wave_exclusive(uint32_t v, uint32_t lane, uint32_t *tot) {
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, (unsigned)o);
-        if ((int)lane >= o)
-            x += y;
-    }
-    *tot = __shfl(x, 63);
-    return x - v;
-}
-
-// One wavefront per dashed piece (entries of the list written by k_dash_walk): the piece's
-// operations of dashed_segment (and the final cap after the sub-path's last piece), with its caps
-// spread over the lanes. Lane l takes the caps l, l + 64,
-// ...; it reaches cap j's dash state by applying the loop's updates one by one from the piece's
-// start state (the same float additions in the same order as the sequential loop), and the cap
-// exists while the offset stays below the segment length. A cap's vertex and index counts come
-// from running it against a counting sink; their wave-wide prefix places it, so the caps land where
-// the sequential emission puts them and their relative vertex references (a start cap refers to
-// the next cap's first two vertices) resolve to the same vertices. The join before the first cap
-// and the final cap are emitted by lane 0. (The piece's totals come from dash_piece_count.)
-__global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ units, uint32_t n_units,
+// One wavefront per dashed piece of many caps (entries of the list that the counting pass of
+// k_stroke_steps writes): the piece's caps, and the final cap after the sub-path's last piece; the join
+// before the first cap is emitted by the piece's thread in k_stroke_steps. The dash offsets of 64 caps at
+// a time are brought to LDS: lane l adds the first l dashes to the offset of the round's first cap (the
+// loop's own float additions in its order; the dash of step t is the same for every lane). The arcs'
+// sines and cosines are evaluated once per piece (one lane per vertex, the angle by the same additions
+// as the loop) and kept in LDS; then the lanes write the caps' vertices and triangles in order, each its
+// own, so that the stores are contiguous (a start cap refers to the next cap's first two vertices, which
+// lie where the sequential emission puts them). The piece's totals come from dash_piece_count; what its
+// caps leave of them is the join's.
+// 1920x1080 strokes, a quarter of them dashed: a lane per cap that evaluated its own arc, and threads
+// doing so for pieces below 64 caps, took 830 us (threads) + 457 us (wavefronts); now 55 + 235 us.
+#define VKH_DASH_ARC 128 // arc vertices kept per cap kind; finer arcs are evaluated per vertex
+__global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ units,
                                                      const uint32_t *__restrict__ step_off,
                                                      const vkh_draw *__restrict__ draws,
                                                      const vkh_subpath *__restrict__ sps,
@@ -864,18 +962,23 @@ __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ un
                                                      const uint32_t *__restrict__ sp_count, const v2 *__restrict__ pts,
                                                      const uint8_t *__restrict__ pf,
                                                      const vkh_stroke_style *__restrict__ styles,
-                                                     const float *__restrict__ dashes, uint32_t *__restrict__ step_nv,
-                                                     uint32_t *__restrict__ step_nt, const uint32_t *__restrict__ sv_off,
+                                                     const float *__restrict__ dashes, const uint32_t *__restrict__ sv_off,
                                                      const uint32_t *__restrict__ st_off, v2 *__restrict__ verts,
                                                      uint32_t *__restrict__ tris, const uint2 *__restrict__ dash_st,
                                                      const uint4 *__restrict__ dlist,
                                                      const uint32_t *__restrict__ dcount) {
+    __shared__ float2 s_arc[4][2][VKH_DASH_ARC];
+    __shared__ float s_off[4][64];
     const uint32_t lane = threadIdx.x & 63;
+    float2(*arc)[VKH_DASH_ARC] = s_arc[threadIdx.x >> 6];
+    float *offs = s_off[threadIdx.x >> 6];
     const uint32_t n_list = *dcount;
     const uint32_t stride = gridDim.x * (blockDim.x >> 6);
     for (uint32_t li = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); li < n_list; li += stride) {
         const uint4 ent = dlist[li]; // step, caps, unit
-        const uint32_t sidx = ent.x, u = ent.z;
+        const uint32_t sidx = (uint32_t)__builtin_amdgcn_readfirstlane((int)ent.x);
+        const uint32_t caps = (uint32_t)__builtin_amdgcn_readfirstlane((int)ent.y);
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)ent.z);
         const Unit un = units[u];
         const vkh_draw &d = draws[un.draw];
         const vkh_stroke_style &st = styles[d.style];
@@ -883,88 +986,114 @@ __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ un
         const bool closed = (sps[un.subpath].flags & VKH_SP_CLOSED) != 0;
         const uint32_t k = sidx - step_off[u];
         const float dreg = lane < c.dashCount ? c.dashes[lane] : 0.f; // lane i holds dash i
+        auto dash = [&](uint32_t i) { // dash i, the same i in every lane
+            return c.dashCount <= 64
+                       ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(dreg), (int)i))
+                       : c.dashes[i];
+        };
         uint32_t iL, cp, iR;
         bool curved;
         dash_piece_points(c, k, iL, cp, iR, curved);
-        DashState dc0 = dash_unpack(c, st.dash_offset, dash_st[sidx]);
-        uint32_t nv = sv_off[sidx], ni = 3u * st_off[sidx];
-        const v2 p = c.P[cp], pR = c.P[iR];
-        if (!dc0.dashOn) { // the join at the piece's start point
-            CountSink cs;
-            vb_step(c, cs, iL, cp, iR, curved);
-            if (lane == 0) {
-                EmitSink es;
-                es.verts = verts;
-                es.nv = nv;
-                es.idx = tris + ni;
-                es.ni = 0;
-                vb_step(c, es, iL, cp, iR, curved);
-            }
-            nv += cs.nv;
-            ni += cs.ni;
-        }
-        const v2 dv = vsub(pR, p);
-        dc0.normal = vnorm(dv);
+        const DashState dc0 = dash_unpack(c, st.dash_offset, dash_st[sidx]);
+        const v2 dv = vsub(c.P[iR], c.P[cp]);
         const float segLen = vlen(dv);
-        // lane l: the state at cap l
-        DashState my = dc0;
-        const uint32_t setup = min(ent.y, 63u); // lane min(caps, 63) is the last one that matters
-        for (uint32_t t = 0; t < setup; t++) { // every lane takes part in the shuffles of the update
-            DashState nx = my;
-            dash_advance(c, dreg, nx);
-            if (t < lane)
-                my = nx;
+        DashCaps C;
+        C.p = c.P[cp];
+        C.n = vnorm(dv);
+        C.hw = c.hw;
+        C.step = c.arcStep;
+        C.cap = c.cap;
+        C.ks = C.ke = 0;
+        C.on0 = dc0.dashOn;
+        float a0 = 0.f;
+        // arc and offs are this wavefront's own; its LDS accesses complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (c.cap == 1) {
+            float a1s, a1e;
+            a0 = dash_arc_angle(C.n, true, a1s);
+            dash_arc_angle(C.n, false, a1e);
+            C.ks = dash_arc_count(a0, a1s, true, C.step);
+            C.ke = dash_arc_count(a0, a1e, false, C.step);
+            for (int w = 0; w < 2; w++) {
+                const uint32_t n = min(w ? C.ke : C.ks, (uint32_t)VKH_DASH_ARC);
+                float a = a0; // advanced to vertex i's angle
+                uint32_t at = 0;
+                for (uint32_t i = lane; i < n; i += 64) {
+                    for (; at <= i; at++)
+                        a = w ? a - C.step : a + C.step;
+                    float sy, cx;
+                    d_sincosf(a, &sy, &cx);
+                    arc[w][i] = make_float2(cx * C.hw, sy * C.hw);
+                }
+            }
         }
-        DashState fin;
-        while (true) {
-            const bool act = my.curDashOffset < segLen;
-            const uint64_t am = __ballot(act);
-            CountSink cs;
-            const v2 p0 = vadd(p, vmul(my.normal, my.curDashOffset));
-            if (act)
-                stroke_cap(c, cs, p0, my.normal, my.dashOn);
-            uint32_t tv, ti;
-            const uint32_t ov = wave_exclusive(cs.nv, lane, &tv), oi = wave_exclusive(cs.ni, lane, &ti);
-            if (act) {
-                EmitSink es;
-                es.verts = verts;
-                es.nv = nv + ov;
-                es.idx = tris + ni + oi;
-                es.ni = 0;
-                stroke_cap(c, es, p0, my.normal, my.dashOn);
+        auto arc_at = [&](bool start, uint32_t i) {
+            if (i < VKH_DASH_ARC)
+                return arc[start ? 0 : 1][i];
+            float a = a0, sy, cx;
+            for (uint32_t t = 0; t <= i; t++)
+                a = start ? a + C.step : a - C.step;
+            d_sincosf(a, &sy, &cx);
+            return make_float2(cx * C.hw, sy * C.hw);
+        };
+        auto vertex = [&](bool start, v2 p0, uint32_t q) { // vertex q of a cap at p0
+            const uint32_t pair = start ? C.ks : 0u;
+            if (q == pair || q == pair + 1)
+                return C.side(start, p0, q != pair);
+            const float2 e = arc_at(start, start ? q : q - 2);
+            return C.arc(p0, e.x, e.y);
+        };
+        const bool end_on = C.on0 == ((caps & 1) == 0); // dashOn after the last cap
+        const bool final_cap = k + 1 == dash_pieces(c.n, closed) && !end_on;
+        uint32_t nv = sv_off[sidx + 1] - C.nv_before(caps) - (final_cap ? C.nv(false) : 0u);
+        uint32_t nt = st_off[sidx + 1] - C.nt_before(caps) - (final_cap ? C.nt(false) : 0u);
+        const uint32_t per = C.nv(true) + C.nv(false), first = C.nv(C.on0);
+        const uint32_t pert = C.nt(true) + C.nt(false), firstt = C.nt(C.on0);
+        float base = dc0.curDashOffset; // the offset of cap j0, whose dash is cur
+        uint32_t cur = (uint32_t)__builtin_amdgcn_readfirstlane((int)dc0.curDash);
+        for (uint32_t j0 = 0; j0 < caps; j0 += 64) { // j0 is even, so cap j0 is of the kind of cap 0
+            const uint32_t m = min(64u, caps - j0);
+            float off = base;
+            for (uint32_t t = 0; t < m; t++) { // lane l stops at cap j0 + l; base becomes cap j0 + m's
+                const float v = dash(cur);
+                const float nx = base + v; // base: cap j0 + t's
+                if (t < lane)
+                    off = nx;
+                base = nx;
+                if (++cur == c.dashCount)
+                    cur = 0;
             }
-            nv += tv;
-            ni += ti;
-            if (am != ~0ull) {
-                // the first lane without a cap holds the state after the last cap's update
-                const int l0 = __ffsll((unsigned long long)~am) - 1;
-                fin.dashOn = __shfl((int)my.dashOn, l0) != 0;
-                fin.curDash = (uint32_t)__shfl((int)my.curDash, l0);
-                fin.curDashOffset = __shfl(my.curDashOffset, l0);
-                fin.totDashLength = my.totDashLength;
-                fin.normal = my.normal;
-                break;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            offs[lane] = off;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const uint32_t n_v = C.nv_before(m), n_t = C.nt_before(m);
+            for (uint32_t i = lane; i < n_v; i += 64) {
+                const uint32_t pair = i / per, r = i - pair * per;
+                const bool second = r >= first, start = second ? !C.on0 : C.on0;
+                verts[nv + i] = vertex(start, C.at(offs[2 * pair + (second ? 1u : 0u)]), second ? r - first : r);
             }
-            for (uint32_t t = 0; t < 64; t++)
-                dash_advance(c, dreg, my);
+            for (uint32_t i = lane; i < n_t; i += 64) {
+                const uint32_t pair = i / pert, r = i - pair * pert;
+                const bool second = r >= firstt, start = second ? !C.on0 : C.on0;
+                uint32_t o[3];
+                C.tri(start, nv + pair * per + (second ? first : 0u), second ? r - firstt : r, o);
+                uint32_t *w = tris + 3 * ((size_t)nt + i);
+                w[0] = o[0];
+                w[1] = o[1];
+                w[2] = o[2];
+            }
+            nv += n_v;
+            nt += n_t;
         }
-        fin.curDashOffset -= segLen;
-        fin.curDashOffset = fmodf(fin.curDashOffset, fin.totDashLength);
-        if (k + 1 == dash_pieces(c.n, closed) && !fin.dashOn) {
-            CountSink cs;
-            DashState f1 = fin;
-            dash_final_cap(c, cs, f1, iR);
-            if (lane == 0) {
-                EmitSink es;
-                es.verts = verts;
-                es.nv = nv;
-                es.idx = tris + ni;
-                es.ni = 0;
-                DashState f2 = fin;
-                dash_final_cap(c, es, f2, iR);
-            }
-            nv += cs.nv;
-            ni += cs.ni;
+        if (final_cap) { // src/vkvg_context.c:936-944 (dash_final_cap), spread over the lanes
+            const float end = dash_mod(base - segLen, dc0.totDashLength);
+            const uint32_t prev = cur ? cur - 1 : c.dashCount - 1, now = cur ? cur : c.dashCount - 1;
+            const float back = fminf(dash(prev) - end, dash(now));
+            const v2 p0 = vsub(c.P[iR], vmul(C.n, back));
+            for (uint32_t i = lane; i < C.nv(false); i += 64)
+                verts[nv + i] = vertex(false, p0, i);
+            for (uint32_t i = lane; i < C.nt(false); i += 64)
+                C.tri(false, nv, i, tris + 3 * ((size_t)nt + i));
         }
     }
 }
@@ -978,8 +1107,10 @@ __global__ void k_stroke_steps(const Unit *__restrict__ units, uint32_t n_units,
                                const float *__restrict__ dashes, uint32_t *__restrict__ step_nv,
                                uint32_t *__restrict__ step_nt, const uint32_t *__restrict__ sv_off,
                                const uint32_t *__restrict__ st_off, v2 *__restrict__ verts,
-                               uint32_t *__restrict__ tris, uint2 *__restrict__ dash_st) {
+                               uint32_t *__restrict__ tris, uint2 *__restrict__ dash_st, uint4 *__restrict__ dlist,
+                               uint32_t *__restrict__ dcount) {
     __shared__ float s_dash[256 * VKH_DASH_ROW];
+    __shared__ float s_off[EMIT ? 256 * VKH_DASH_WAVE_MIN : 1];
     uint32_t sidx = blockIdx.x * blockDim.x + threadIdx.x;
     if (sidx >= n_steps)
         return;
@@ -987,34 +1118,49 @@ __global__ void k_stroke_steps(const Unit *__restrict__ units, uint32_t n_units,
     Unit un = units[u];
     const vkh_draw &d = draws[un.draw];
     const vkh_stroke_style &st = styles[d.style];
-    uint2 ds = make_uint2(0u, 0u);
-    if (st.dash_count) {
-        ds = dash_st[sidx];
-        if (EMIT && (ds.x & VKH_DASH_WAVE_BIT))
-            return; // a piece of many caps: emitted by k_dash_pieces
-    }
+    const uint2 ds = st.dash_count ? dash_st[sidx] : make_uint2(0u, 0u);
+    const bool wave = (ds.x & VKH_DASH_WAVE_BIT) != 0; // a piece of many caps: they are k_dash_pieces'
     StrokeCtx c = make_stroke_ctx(st, dashes, pts, pf, sp_first[un.subpath], sp_count[un.subpath]);
     stage_dashes(c, s_dash);
     bool closed = (sps[un.subpath].flags & VKH_SP_CLOSED) != 0;
     uint32_t i = sidx - step_off[u];
     if (!EMIT) {
         CountSink k;
-        if (st.dash_count)
-            dash_piece_count(c, dash_period(c.dashes, c.dashCount), closed, i,
-                             dash_unpack(c, st.dash_offset, ds), k);
-        else
+        uint32_t caps = 0;
+        if (st.dash_count) {
+            caps = step_nv[sidx]; // from the dash walk
+            dash_piece_count(c, closed, i, dash_unpack(c, st.dash_offset, ds), caps, k);
+        } else {
             stroke_step(c, closed, i, k);
+        }
         step_nv[sidx] = k.nv;
         step_nt[sidx] = k.ni / 3;
+        const uint64_t wm = __ballot(wave); // the list of k_dash_pieces: one atomic per wavefront
+        if (wave) {
+            const uint32_t lane = threadIdx.x & 63, leader = (uint32_t)__ffsll((unsigned long long)wm) - 1;
+            uint32_t at = 0;
+            if (lane == leader)
+                at = atomicAdd(dcount, (uint32_t)__popcll((unsigned long long)wm));
+            at = (uint32_t)__shfl((int)at, (int)leader) +
+                 (uint32_t)__popcll((unsigned long long)(wm & ((1ull << lane) - 1ull)));
+            dlist[at] = make_uint4(sidx, caps, u, 0u);
+        }
     } else {
         EmitSink k;
         k.verts = verts;
         k.nv = sv_off[sidx];
         k.idx = tris + 3 * (size_t)st_off[sidx];
         k.ni = 0;
-        if (st.dash_count) {
-            DashState dc = dash_unpack(c, st.dash_offset, ds);
-            dash_piece(c, closed, i, dc, k);
+        if (wave) {
+            const DashState dc = dash_unpack(c, st.dash_offset, ds);
+            if (!dc.dashOn) { // the join at the piece's start point
+                uint32_t iL, cp, iR;
+                bool curved;
+                dash_piece_points(c, i, iL, cp, iR, curved);
+                vb_step(c, k, iL, cp, iR, curved);
+            }
+        } else if (st.dash_count) {
+            dash_piece_emit(c, closed, i, dash_unpack(c, st.dash_offset, ds), k, s_off + threadIdx.x, 256);
         } else {
             stroke_step(c, closed, i, k);
         }
@@ -1406,20 +1552,20 @@ void launch_stroke_steps(hipStream_t s, bool emit, const Unit *units, uint32_t n
         return;
     if (!emit)
         hipLaunchKernelGGL(k_dash_walk, dim3((n_units + 255) / 256), dim3(256), 0, s, units, n_units, step_off, n_steps,
-                           draws, sps, spf, spc, pts, pf, styles, dashes, dash_st, dlist, dcount);
+                           draws, sps, spf, spc, pts, pf, styles, dashes, dash_st, step_nv, dcount,
+                           n_steps <= VKH_DASH_FEW ? VKH_DASH_WAVE_MIN_FEW : VKH_DASH_WAVE_MIN);
     // a wavefront per dashed piece, at most 4096 wavefronts walking the list
     const uint32_t dblocks = (uint32_t)std::min<uint64_t>(((uint64_t)n_steps + 3) / 4, 1024);
     if (emit) {
         hipLaunchKernelGGL(k_stroke_steps<true>, dim3((n_steps + 255) / 256), dim3(256), 0, s, units, n_units, step_off,
                            n_steps, draws, sps, spf, spc, pts, pf, styles, dashes, step_nv, step_nt, sv_off, st_off,
-                           verts, tris, dash_st);
-        hipLaunchKernelGGL(k_dash_pieces, dim3(dblocks), dim3(256), 0, s, units, n_units, step_off, draws, sps, spf,
-                           spc, pts, pf, styles, dashes, step_nv, step_nt, sv_off, st_off, verts, tris, dash_st, dlist,
-                           dcount);
+                           verts, tris, dash_st, dlist, dcount);
+        hipLaunchKernelGGL(k_dash_pieces, dim3(dblocks), dim3(256), 0, s, units, step_off, draws, sps, spf, spc, pts, pf,
+                           styles, dashes, sv_off, st_off, verts, tris, dash_st, dlist, dcount);
     } else {
         hipLaunchKernelGGL(k_stroke_steps<false>, dim3((n_steps + 255) / 256), dim3(256), 0, s, units, n_units,
                            step_off, n_steps, draws, sps, spf, spc, pts, pf, styles, dashes, step_nv, step_nt, sv_off,
-                           st_off, verts, tris, dash_st);
+                           st_off, verts, tris, dash_st, dlist, dcount);
     }
 }
 void launch_stroke_patch(hipStream_t s, const Unit *units, uint32_t n_units, const uint32_t *step_off,
