@@ -25,7 +25,8 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fno-gpu-rdc", "-Wno-unused-result", f"-I{INC}", f"-I{CSRC}",
 ]
-C_FLAGS = ["-O2", "-fPIC", "-std=c11", "-ffp-contract=off", "-fno-fast-math", "-Wall",
+# the recorder's entry points call each other and are never interposed
+C_FLAGS = ["-O2", "-fPIC", "-fno-semantic-interposition", "-std=c11", "-ffp-contract=off", "-fno-fast-math", "-Wall",
            "-Wno-unused-function", f"-I{INC}"]
 
 HIP_SOURCES = ["vkh_geom.hip", "vkh_raster.hip", "vkh_engine.hip", "vkh_diff.hip"]

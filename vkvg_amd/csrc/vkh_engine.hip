@@ -253,6 +253,7 @@ static int read_totals(vkh_engine *eng, const std::vector<const uint32_t *> &src
     return 0;
 }
 
+#define VKH_UPLOAD_ITEMS 65536u // items per piece of an upload (2.6 MB)
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 extern "C" {
@@ -591,8 +592,20 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     if (!ensure_host(eng, eng->hblob, total) || !ensure(eng, eng->blob, total))
         return -1;
     uint8_t *hb = (uint8_t *)eng->hblob.p;
-    if (n_items)
-        memcpy(hb + o_items, f->items, sizeof(vkh_item) * n_items);
+    // the items, most of a large frame, in pieces: the copy to the device of one runs while the next is
+    // staged, and its cubics are counted while it is in the cache
+    uint32_t n_cubics = 0;
+    size_t sent = 0;
+    for (uint32_t i0 = 0; i0 < n_items; i0 += VKH_UPLOAD_ITEMS) {
+        const uint32_t k = std::min<uint32_t>(n_items - i0, VKH_UPLOAD_ITEMS);
+        memcpy(hb + o_items + sizeof(vkh_item) * i0, f->items + i0, sizeof(vkh_item) * k);
+        for (uint32_t i = i0; i < i0 + k; i++)
+            n_cubics += (f->items[i].flags & VKH_ITEM_CUBIC) ? 1u : 0u;
+        if (k == VKH_UPLOAD_ITEMS) {
+            CK(hipMemcpyAsync((uint8_t *)eng->blob.p + sent, hb + sent, sizeof(vkh_item) * k, hipMemcpyHostToDevice, s));
+            sent += sizeof(vkh_item) * k;
+        }
+    }
     if (n_sp)
         memcpy(hb + o_sp, f->subpaths, sizeof(vkh_subpath) * n_sp);
     if (n_draws)
@@ -609,7 +622,7 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
         memcpy(hb + o_units, units.data(), sizeof(Unit) * n_units);
     if (f->n_sources)
         memcpy(hb + o_srcs, f->sources, sizeof(vkh_surface_source) * f->n_sources);
-    CK(hipMemcpyAsync(eng->blob.p, hb, total, hipMemcpyHostToDevice, s));
+    CK(hipMemcpyAsync((uint8_t *)eng->blob.p + sent, hb + sent, total - sent, hipMemcpyHostToDevice, s));
     eng->o_items = o_items;
     eng->o_sp = o_sp;
     eng->o_draws = o_draws;
@@ -631,9 +644,7 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     eng->bin_total = bin_total;
     eng->frame_tile = T;
     eng->h_tg = tg;
-    eng->n_cubic_items = 0;
-    for (uint32_t i = 0; i < n_items; i++)
-        eng->n_cubic_items += (f->items[i].flags & VKH_ITEM_CUBIC) ? 1u : 0u;
+    eng->n_cubic_items = n_cubics;
     eng->most_draws = 1;
     for (const TargetInfo &ti : tg)
         eng->most_draws = std::max(eng->most_draws, ti.draw_end - ti.draw_begin);

@@ -61,12 +61,27 @@
 typedef struct { float x, y; } v2;
 
 /* ---------------------------------------------------------------------------- objects */
+typedef struct {
+    VEC(vkh_item) items;
+    VEC(vkh_subpath) sps;
+    VEC(vkh_draw) draws;
+    VEC(vkh_stroke_style) styles;
+    VEC(float) dashes;
+    VEC(vkh_gradient) grads;
+    VEC(vkh_surface_source) srcs;
+    VEC(VkvgSurface) src_refs; /* source surfaces referenced until the frame has rendered */
+} frame_t;
+
 struct _vkvg_device_t {
     vkvg_status_t status;
     uint32_t      references;
     vkh_engine   *eng;
     int           hdpy, vdpy;
     uint32_t      ctx_cache_size; /* vkvg_device_set_context_cache_size: kept, contexts are not cached */
+    /* Recording buffers of an ended context, empty, for the next one (swapped in and out atomically:
+     * contexts of one device may live in several threads). Growing fresh arrays costs a frame of 324 k
+     * items some 3000 page faults per pass; kept are at most FRAME_KEEP_BYTES, until the device ends. */
+    frame_t      *spare;
 };
 
 struct _vkvg_surface_t {
@@ -98,17 +113,6 @@ struct _vkvg_pattern_t {
     grad_data           g;
     VkvgSurface         surf; /* SURFACE patterns: the referenced source surface */
 };
-
-typedef struct {
-    VEC(vkh_item) items;
-    VEC(vkh_subpath) sps;
-    VEC(vkh_draw) draws;
-    VEC(vkh_stroke_style) styles;
-    VEC(float) dashes;
-    VEC(vkh_gradient) grads;
-    VEC(vkh_surface_source) srcs;
-    VEC(VkvgSurface) src_refs; /* source surfaces referenced until the frame has rendered */
-} frame_t;
 
 struct _vkvg_context_t {
     vkvg_status_t status;
@@ -275,6 +279,58 @@ void vkvg_matrix_get_scale(const vkvg_matrix_t *m, float *sx, float *sy) {
     *sy = (float)sqrt(m->yx * m->yx + m->yy * m->yy);
 }
 
+/* ---------------------------------------------------------------------------- frames */
+static void frame_release_sources(frame_t *f) {
+    for (uint32_t i = 0; i < f->src_refs.n; i++)
+        vkvg_surface_destroy(f->src_refs.p[i]);
+    f->src_refs.n = 0;
+}
+static void frame_free(frame_t *f) {
+    frame_release_sources(f);
+    free(f->src_refs.p);
+    free(f->items.p);
+    free(f->sps.p);
+    free(f->draws.p);
+    free(f->styles.p);
+    free(f->dashes.p);
+    free(f->grads.p);
+    free(f->srcs.p);
+    memset(f, 0, sizeof(*f));
+}
+#define FRAME_KEEP_BYTES ((size_t)64 << 20)
+static size_t frame_bytes(const frame_t *f) {
+    return sizeof(vkh_item) * f->items.cap + sizeof(vkh_subpath) * f->sps.cap + sizeof(vkh_draw) * f->draws.cap +
+           sizeof(vkh_stroke_style) * f->styles.cap + sizeof(float) * f->dashes.cap +
+           sizeof(vkh_gradient) * f->grads.cap + sizeof(vkh_surface_source) * f->srcs.cap +
+           sizeof(VkvgSurface) * f->src_refs.cap;
+}
+/* f (zeroed) takes the device's spare buffers, if there are any */
+static void frame_take(VkvgDevice dev, frame_t *f) {
+    frame_t *s = __atomic_exchange_n(&dev->spare, NULL, __ATOMIC_ACQ_REL);
+    if (s) {
+        *f = *s;
+        free(s);
+    }
+}
+/* empties f and leaves its buffers to the device, or frees them when they are too large or the device
+ * has some already */
+static void frame_give(VkvgDevice dev, frame_t *f) {
+    frame_release_sources(f);
+    frame_t *s = f->items.cap && frame_bytes(f) <= FRAME_KEEP_BYTES ? (frame_t *)malloc(sizeof(frame_t)) : NULL;
+    if (!s) {
+        frame_free(f);
+        return;
+    }
+    f->items.n = f->sps.n = f->draws.n = f->styles.n = f->dashes.n = f->grads.n = f->srcs.n = 0;
+    *s = *f;
+    memset(f, 0, sizeof(*f));
+    frame_t *none = NULL;
+    if (!__atomic_compare_exchange_n(&dev->spare, &none, s, false, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED)) {
+        frame_free(s);
+        free(s);
+    }
+}
+
 /* ---------------------------------------------------------------------------- device */
 /* src/vkvg_device.c:286-291: a NULL create-info is an error; its samples and Vulkan handles have no
  * meaning here (1 sample, HIP device 0) */
@@ -326,6 +382,10 @@ void vkvg_device_destroy(VkvgDevice dev) {
     if (--dev->references > 0)
         return;
     vkvg_hip_engine_destroy(dev->eng);
+    if (dev->spare) {
+        frame_free(dev->spare);
+        free(dev->spare);
+    }
     free(dev);
 }
 void vkvg_device_set_dpy(VkvgDevice dev, int hdpy, int vdpy) {
@@ -726,24 +786,6 @@ VkvgPattern vkvg_pattern_create_for_surface(VkvgSurface surf) {
 }
 
 /* ---------------------------------------------------------------------------- context */
-static void frame_release_sources(frame_t *f) {
-    for (uint32_t i = 0; i < f->src_refs.n; i++)
-        vkvg_surface_destroy(f->src_refs.p[i]);
-    f->src_refs.n = 0;
-}
-static void frame_free(frame_t *f) {
-    frame_release_sources(f);
-    free(f->src_refs.p);
-    free(f->items.p);
-    free(f->sps.p);
-    free(f->draws.p);
-    free(f->styles.p);
-    free(f->dashes.p);
-    free(f->grads.p);
-    free(f->srcs.p);
-    memset(f, 0, sizeof(*f));
-}
-
 static void reset_open_subpath(VkvgContext c) {
     c->cur_first_item = c->f.items.n;
     c->cur_count = 0;
@@ -766,6 +808,7 @@ VkvgContext vkvg_create(VkvgSurface surf) {
     c->references = 1;
     c->surf = surf;
     vkvg_surface_reference(surf);
+    frame_take(surf->dev, &c->f);
     /* defaults of src/vkvg_context.c:24-69 */
     c->lineWidth = 1.f;
     c->miterLimit = 10.f;
@@ -911,7 +954,7 @@ void vkvg_destroy(VkvgContext ctx) {
         vkvg_pattern_destroy(ctx->pattern);
     vkvg_rec_free(ctx->recording); /* a recording never stopped (src/vkvg_context.c:261-264) */
     free(ctx->dashes);
-    frame_free(&ctx->f);
+    frame_give(ctx->surf->dev, &ctx->f);
     vkvg_surface_destroy(ctx->surf);
     free(ctx);
 }
@@ -924,11 +967,11 @@ static inline bool no_committed_subpath(VkvgContext c) { return c->f.sps.n == c-
 static void add_point(VkvgContext c, float x, float y) {
     if (isnan(x) || isnan(y))
         return;
-    vkh_item it;
-    memset(&it, 0, sizeof(it));
-    it.p[0] = x;
-    it.p[1] = y;
-    VEC_PUSH(c->f.items, it);
+    VEC_RESERVE(c->f.items, c->f.items.n + 1);
+    vkh_item *it = &c->f.items.p[c->f.items.n++];
+    memset(it, 0, sizeof(*it));
+    it->p[0] = x;
+    it->p[1] = y;
     v2 p = {x, y};
     if (c->cur_count == 0)
         c->cur_first = p;
@@ -2399,6 +2442,12 @@ vkvg_status_t vkvg_amd_replay_sources(VkvgContext ctx, const uint32_t *words, si
         return vkvg_status(ctx);
     size_t i = 0;
     while (i < n && !ctx->status) {
+        /* the points of a polyline, most of a stream, without a call each */
+        if (words[i] == 2 && n - i >= 3 && !ctx->recording) {
+            line_to_i(ctx, F(words + i + 1), F(words + i + 2));
+            i += 3;
+            continue;
+        }
         size_t used = 0;
         int r = stream_step(ctx, words + i, n - i, &used, sources, sources ? n_sources : 0);
         if (r < 0) {
@@ -2423,72 +2472,46 @@ vkvg_status_t vkvg_amd_upload_batch(VkvgDevice dev, uint32_t n, const VkvgSurfac
         return VKVG_STATUS_DEVICE_ERROR;
     if (!n)
         return VKVG_STATUS_SUCCESS;
-    VkvgContext *ctxs = (VkvgContext *)calloc(n, sizeof(VkvgContext));
     vkh_target *tg = (vkh_target *)calloc(n, sizeof(vkh_target));
+    /* every context records into the same frame: its items, styles, ... go on where the last one's end */
     frame_t all;
     memset(&all, 0, sizeof(all));
     uint32_t n_draws_total = 0;
     vkvg_status_t st = VKVG_STATUS_SUCCESS;
-    if (!ctxs || !tg) {
+    if (!tg) {
         st = VKVG_STATUS_NO_MEMORY;
         goto done;
     }
+    frame_take(dev, &all);
     for (uint32_t i = 0; i < n && !st; i++) {
         if (vkvg_surface_status(surfs[i]) || surfs[i]->dev != dev) {
             st = VKVG_STATUS_INVALID_SURFACE;
             break;
         }
-        ctxs[i] = vkvg_create(surfs[i]);
-        if (vkvg_status(ctxs[i])) {
-            st = vkvg_status(ctxs[i]);
-            ctxs[i] = NULL;
+        VkvgContext c = vkvg_create(surfs[i]);
+        if (vkvg_status(c)) {
+            st = vkvg_status(c);
             break;
         }
-        ctxs[i]->deferred = true;
-        st = vkvg_amd_replay(ctxs[i], streams[i], n_words[i]);
-        if (st)
-            break;
-        /* append this context's frame, rebasing indices */
-        frame_t *f = &ctxs[i]->f;
-        uint32_t ib = all.items.n, sb = all.sps.n, stb = all.styles.n, db = all.dashes.n, gb = all.grads.n,
-                 srb = all.srcs.n;
-        VEC_RESERVE(all.items, all.items.n + f->items.n);
-        memcpy(all.items.p + all.items.n, f->items.p, sizeof(vkh_item) * f->items.n);
-        all.items.n += f->items.n;
-        for (uint32_t k = 0; k < f->sps.n; k++) {
-            vkh_subpath sp = f->sps.p[k];
-            sp.first_item += ib;
-            VEC_PUSH(all.sps, sp);
-        }
-        for (uint32_t k = 0; k < f->styles.n; k++) {
-            vkh_stroke_style s = f->styles.p[k];
-            s.dash_first += db;
-            VEC_PUSH(all.styles, s);
-        }
-        for (uint32_t k = 0; k < f->dashes.n; k++)
-            VEC_PUSH(all.dashes, f->dashes.p[k]);
-        for (uint32_t k = 0; k < f->grads.n; k++)
-            VEC_PUSH(all.grads, f->grads.p[k]);
-        for (uint32_t k = 0; k < f->srcs.n; k++)
-            VEC_PUSH(all.srcs, f->srcs.p[k]);
-        for (uint32_t k = 0; k < f->draws.n; k++) {
-            vkh_draw d = f->draws.p[k];
-            d.first_subpath += sb;
-            if (d.kind == VKH_DRAW_STROKE && d.style >= 0)
-                d.style += (int32_t)stb;
-            if (d.grad >= 0)
-                d.grad += (int32_t)gb;
-            if (d.source >= 0)
-                d.source += (int32_t)srb;
-            d.target = i;
-            VEC_PUSH(all.draws, d);
-        }
+        const uint32_t first_draw = all.draws.n;
+        frame_free(&c->f);
+        c->f = all;
+        c->deferred = true;
+        c->path_item_begin = all.items.n;
+        c->path_sp_begin = all.sps.n;
+        reset_open_subpath(c);
+        st = vkvg_amd_replay(c, streams[i], n_words[i]);
+        all = c->f;
+        memset(&c->f, 0, sizeof(c->f));
+        for (uint32_t k = first_draw; k < all.draws.n; k++)
+            all.draws.p[k].target = i;
         tg[i].rgba = surfs[i]->img;
         tg[i].width = surfs[i]->width;
         tg[i].height = surfs[i]->height;
         tg[i].sig = surfs[i]->sig;
-        tg[i].stencil = ctxs[i]->stencil_use ? surfs[i]->stencil : NULL;
+        tg[i].stencil = c->stencil_use ? surfs[i]->stencil : NULL;
         tg[i].stencil_load = 0; /* a fresh context: its stencil starts from zero */
+        vkvg_destroy(c);
     }
     n_draws_total = all.draws.n;
     if (!st && all.draws.n) {
@@ -2515,14 +2538,7 @@ vkvg_status_t vkvg_amd_upload_batch(VkvgDevice dev, uint32_t n, const VkvgSurfac
         }
     }
 done:
-    for (uint32_t i = 0; ctxs && i < n; i++) {
-        if (ctxs[i]) {
-            ctxs[i]->f.draws.n = 0; /* already rendered as part of the batch */
-            vkvg_destroy(ctxs[i]);
-        }
-    }
-    frame_free(&all);
-    free(ctxs);
+    frame_give(dev, &all);
     free(tg);
     if (!st && n_draws_total == 0)
         st = VKVG_STATUS_INVALID_STATUS; /* nothing to execute */
