@@ -10,6 +10,7 @@
 
 #define VKH_BIN_TILES 16        // a coarse bin is 16 x 16 tiles
 #define VKH_COARSE_CHUNK 1024   // most draws per coarse workgroup
+#define VKH_COARSE_MIN 16       // fewest
 #define VKH_FLAT_SLOT 128       // flattened points kept per cubic by the subdivision pass
 
 // one (draw, subpath) pair of the frame; fills and strokes are expanded per unit
@@ -179,7 +180,8 @@ void launch_tile_cnt_init(hipStream_t s, const TargetInfo *tg, uint32_t n_target
 void launch_draw_prep(hipStream_t s, const vkh_draw *draws, uint32_t n_draws, const TargetInfo *tg,
                       const vkh_gradient *grads, uint32_t n_grads, const vkh_surface_source *srcs, DrawPrep *out,
                       GradRec *rec, GradPrep *gout);
-// draws per coarse workgroup: about 1024 workgroups over n_bins bins, 64 .. VKH_COARSE_CHUNK draws
+// draws per coarse workgroup: about 1024 workgroups over n_bins bins, VKH_COARSE_MIN ..
+// VKH_COARSE_CHUNK draws
 uint32_t coarse_chunk(uint32_t most_draws, uint32_t n_bins);
 void launch_coarse(hipStream_t s, bool write, uint32_t n_bins, uint32_t nch, uint32_t chunk, const TargetInfo *tg,
                    uint32_t n_targets, const vkh_draw *draws, const DrawTiles *dt, const PathTile *pts,

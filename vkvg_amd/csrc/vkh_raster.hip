@@ -1288,8 +1288,11 @@ void launch_tile_cnt_init(hipStream_t s, const TargetInfo *tg, uint32_t n_target
 uint32_t coarse_chunk(uint32_t most_draws, uint32_t n_bins) {
     const uint32_t want = (1024 + std::max(n_bins, 1u) - 1) / std::max(n_bins, 1u); // chunks per bin
     uint32_t c = (most_draws + want - 1) / want;
-    c = (c + 63) / 64 * 64;
-    return std::min<uint32_t>(std::max<uint32_t>(c, 64), VKH_COARSE_CHUNK);
+    // A workgroup walks its draws four at a time, each step a round trip to memory, so a frame of few bins
+    // takes small chunks. Coarse stage with chunks of at least 64 / 16 draws: 512x512 with 200 draws
+    // 82 / 52 us, 1920x1080 with 7000 514 / 464 us; at 8 the chunks' prefix sums take back what is won.
+    c = (c + VKH_COARSE_MIN - 1) / VKH_COARSE_MIN * VKH_COARSE_MIN;
+    return std::min<uint32_t>(std::max<uint32_t>(c, VKH_COARSE_MIN), VKH_COARSE_CHUNK);
 }
 void launch_coarse(hipStream_t s, bool write, uint32_t n_bins, uint32_t nch, uint32_t chunk, const TargetInfo *tg,
                    uint32_t n_targets, const vkh_draw *draws, const DrawTiles *dt, const PathTile *pts,
