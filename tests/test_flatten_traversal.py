@@ -69,3 +69,11 @@ def test_stack_and_stackless_traversals_emit_the_oracle_points(L):
     # some cubic had more points than a tree of 8 levels (more than the kernel stacks) has leaves:
     # its nodes below the stacked levels were recomputed from the deepest stacked ancestor
     assert deepest > 256
+
+
+def test_parts_of_the_split_kernel_emit_the_oracle_points_in_order(L):
+    from oracle import ovg
+    for k, (p, tol) in enumerate(_cases()):
+        want = ovg.flatten_cubic(p, tol)[:-1]
+        got = _points(L, p, tol, 2)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (k, p, tol)

@@ -366,22 +366,19 @@ __host__ __device__ void agg_flatten(const Cubic &root, float tol, Emit emit) {
 }
 
 // The same traversal with the ancestors of the current node on a stack (levels 0 .. D-1 kept by the
-// caller, e.g. in LDS): every move costs one split. The parent of a right sibling at `level` is
+// caller, e.g. in LDS), from `node` at `level` below a root at the absolute level `base`; it visits the
+// rest of that root's subtree (level 0: node is that root). Every move costs one split. The parent of a right sibling at `level` is
 // read from the stack, or, beyond level D-1, recomputed from the level D-1 ancestor along the path
 // bits; all nodes come from the same chain of splits as in the recursion. Every iteration tests one
 // node and makes exactly one split (the left child of an inner node, or the right sibling of the
 // first left child above a leaf), so lanes of a wavefront that take different moves still share it;
 // the right children above a leaf are popped in one count of the path's leading ones.
 template <int D, typename Emit, typename Store, typename Load>
-__host__ __device__ void agg_flatten_stack(const Cubic &root, float tol, Emit emit, Store store, Load load) {
+__host__ __device__ void agg_flatten_walk(Cubic node, int base, int level, float tol, Emit emit, Store store, Load load) {
     uint64_t path_lo = 0, path_hi = 0; // bit (l-1): the node at level l is a right child
-    int level = 1;
-    store(0, root);
-    Cubic node;
-    agg_split(root, false, node);
     while (true) {
         bool leaf;
-        if (level > 100) {
+        if (base + level > 100) {
             leaf = true; // recursion limit: returns without emitting
         } else {
             v2 pts[2];
@@ -394,6 +391,8 @@ __host__ __device__ void agg_flatten_stack(const Cubic &root, float tol, Emit em
             if (n > 1)
                 emit(pts[1]);
         }
+        if (leaf && level == 0)
+            return; // a subtree's own root
         Cubic src;
         bool right;
         if (!leaf) { // descend to the left child
@@ -448,6 +447,41 @@ __host__ __device__ void agg_flatten_stack(const Cubic &root, float tol, Emit em
         }
         agg_split(src, right, node);
     }
+}
+// the whole subdivision of a cubic, whose root always splits
+template <int D, typename Emit, typename Store, typename Load>
+__host__ __device__ void agg_flatten_stack(const Cubic &root, float tol, Emit emit, Store store, Load load) {
+    store(0, root);
+    Cubic node;
+    agg_split(root, false, node);
+    agg_flatten_walk<D>(node, 0, 1, tol, emit, store, load);
+}
+// Part s of 2^B of the subdivision, in order: the points below node s of level B, or, where that node has
+// a leaf above it, the leaf's points with the first part under it. The parts' points one after another
+// are agg_flatten_stack's.
+template <int D, int B, typename Emit, typename Store, typename Load>
+__host__ __device__ void agg_flatten_part(const Cubic &root, uint32_t s, float tol, Emit emit, Store store, Load load) {
+    Cubic node = root;
+    for (int l = 1; l <= B; l++) {
+        Cubic nx;
+        agg_split(node, (s >> (B - l)) & 1u, nx);
+        node = nx;
+        if (l == B)
+            break;
+        v2 pts[2];
+        int n = agg_leaf_fast(node, tol, pts);
+        if (n < 0)
+            n = agg_leaf(node, tol, pts);
+        if (n > 0) {
+            if (!(s & ((1u << (B - l)) - 1u))) {
+                emit(pts[0]);
+                if (n > 1)
+                    emit(pts[1]);
+            }
+            return;
+        }
+    }
+    agg_flatten_walk<D>(node, B, 0, tol, emit, store, load);
 }
 
 // ---------------------------------------------------------------------------------------

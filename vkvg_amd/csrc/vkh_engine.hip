@@ -149,7 +149,7 @@ struct vkh_engine {
     DevBuf blob, units, tgts, item_cnt, item_off, pts, pflags, sp_first, sp_count;
     DevBuf fe, nv, nt, fe_off, nv_off, nt_off, verts, tris, edges;
     DevBuf bbox, erange, dtiles, pt_count, pt_off, ptiles, counters, segs, dprep; // counters: [0] segment allocator, [1] flatten slots, [2] overflow cubics, [3] dashed pieces
-    DevBuf tile_cnt, tile_off, tile_order, draw_order, cmds, scan_tmp, readback, item_slot, slot_item, flat_scratch, flat_perm, flat_ovf,
+    DevBuf tile_cnt, tile_off, tile_order, draw_order, cmds, scan_tmp, readback, slot_item, flat_scratch, flat_perm, flat_ovf,
         flat_wh, dash_list, tl_table;
     DevBuf step_nv, step_nt, sv_off, st_off, u_toff, u_vbeg, u_vend, dash_st; // dash_st: per dashed piece, its starting dash state
     HostBuf hblob, htot;
@@ -301,8 +301,8 @@ void vkvg_hip_engine_destroy(vkh_engine *e) {
                       &e->verts, &e->tris, &e->edges, &e->bbox, &e->dtiles, &e->pt_count, &e->pt_off,
                       &e->erange, &e->ptiles, &e->counters, &e->segs, &e->dprep, &e->tile_cnt,
                       &e->tile_off, &e->tile_order, &e->draw_order, &e->cmds, &e->scan_tmp, &e->readback, &e->step_nv, &e->step_nt,
-                      &e->sv_off, &e->st_off, &e->dash_st, &e->u_toff, &e->u_vbeg, &e->u_vend, &e->item_slot,
-                      &e->slot_item, &e->flat_scratch, &e->flat_perm, &e->flat_ovf, &e->flat_wh, &e->dash_list, &e->tl_table};
+                      &e->sv_off, &e->st_off, &e->dash_st, &e->u_toff, &e->u_vbeg, &e->u_vend, &e->slot_item,
+                      &e->flat_scratch, &e->flat_perm, &e->flat_ovf, &e->flat_wh, &e->dash_list, &e->tl_table};
     for (DevBuf *b : bufs)
         if (b->p)
             (void)hipFree(b->p);
@@ -702,10 +702,12 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     const Unit *d_units = (const Unit *)(db + eng->o_units);
 
     // ---- flatten
-    const uint32_t n_cubics = eng->n_cubic_items;
+    // a frame of few cubics splits each over several threads (split points kept per part)
+    const uint32_t n_cubics = eng->n_cubic_items, split = vkh::flat_split_points(n_cubics);
+    const size_t n_parts = split ? vkh::flat_split_parts(n_cubics) : n_cubics;
     if (!need(eng, cap, eng->item_cnt, 4 * (n_items + 1)) || !need(eng, cap, eng->item_off, 4 * (n_items + 1)) ||
-        !need(eng, cap, eng->item_slot, 4 * (n_items + 1)) || !need(eng, cap, eng->slot_item, 4ull * (n_cubics + 1)) ||
-        !need(eng, cap, eng->flat_scratch, 8ull * VKH_FLAT_SLOT * (n_cubics + 1)) ||
+        !need(eng, cap, eng->slot_item, 4ull * (n_parts + 1)) ||
+        !need(eng, cap, eng->flat_scratch, 8ull * (split ? split : VKH_FLAT_SLOT) * (n_parts + 1)) ||
         !need(eng, cap, eng->flat_perm, 4 * (n_items + 1)) || !need(eng, cap, eng->flat_ovf, 4ull * (n_cubics + 1)) ||
         !need(eng, cap, eng->counters, 1024))
         return -1;
@@ -724,9 +726,14 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
             return -1;
         vkh::launch_flat_scatter(s, d_items, n_items, wcur, P<uint32_t>(eng->flat_perm));
     }
-    vkh::launch_flatten_stage(s, d_items, n_items, P<uint32_t>(eng->flat_perm), P<uint32_t>(eng->item_cnt), ctr + 1,
-                              P<uint32_t>(eng->slot_item), P<uint32_t>(eng->item_slot), P<v2>(eng->flat_scratch),
-                              ctr + 2, P<uint32_t>(eng->flat_ovf));
+    if (split)
+        vkh::launch_flatten_split(s, d_items, n_items, n_cubics, P<uint32_t>(eng->flat_perm), P<uint32_t>(eng->item_cnt),
+                                  P<uint32_t>(eng->slot_item), P<v2>(eng->flat_scratch), ctr + 2,
+                                  P<uint32_t>(eng->flat_ovf));
+    else
+        vkh::launch_flatten_stage(s, d_items, n_items, P<uint32_t>(eng->flat_perm), P<uint32_t>(eng->item_cnt), ctr + 1,
+                                  P<uint32_t>(eng->slot_item), P<v2>(eng->flat_scratch), ctr + 2,
+                                  P<uint32_t>(eng->flat_ovf));
     if (scan_u32(eng, P<uint32_t>(eng->item_cnt), n_items, P<uint32_t>(eng->item_off), cap))
         return -1;
     uint32_t tot[8];
@@ -737,9 +744,14 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     if (!need(eng, cap, eng->pts, 8ull * n_pts + 8) || !need(eng, cap, eng->pflags, n_pts + 8) ||
         !need(eng, cap, eng->sp_first, 4 * (n_sp + 1)) || !need(eng, cap, eng->sp_count, 4 * (n_sp + 1)))
         return -1;
-    vkh::launch_flatten_copy(s, d_items, n_cubics, P<uint32_t>(eng->slot_item), P<uint32_t>(eng->item_cnt),
-                             P<uint32_t>(eng->item_off), P<v2>(eng->flat_scratch), P<v2>(eng->pts),
-                             P<uint8_t>(eng->pflags));
+    if (split)
+        vkh::launch_flatten_split_copy(s, d_items, n_cubics, P<uint32_t>(eng->flat_perm), P<uint32_t>(eng->slot_item),
+                                       P<uint32_t>(eng->item_off), P<v2>(eng->flat_scratch), P<v2>(eng->pts),
+                                       P<uint8_t>(eng->pflags));
+    else
+        vkh::launch_flatten_copy(s, d_items, n_cubics, P<uint32_t>(eng->slot_item), P<uint32_t>(eng->item_cnt),
+                                 P<uint32_t>(eng->item_off), P<v2>(eng->flat_scratch), P<v2>(eng->pts),
+                                 P<uint8_t>(eng->pflags));
     vkh::launch_flatten_lines(s, d_items, n_items, P<uint32_t>(eng->item_off), P<v2>(eng->pts),
                               P<uint8_t>(eng->pflags));
     vkh::launch_flatten_overflow(s, d_items, P<uint32_t>(eng->flat_ovf), n_ovf, P<uint32_t>(eng->item_off),

@@ -85,8 +85,7 @@ __global__ __launch_bounds__(256) void k_flat_scatter(const vkh_item *__restrict
 
 __global__ __launch_bounds__(VKH_FLAT_BLOCK) void k_flatten_stage(const vkh_item *__restrict__ items, uint32_t n, const uint32_t *__restrict__ perm,
                                 uint32_t *__restrict__ counts, uint32_t *__restrict__ slot_alloc,
-                                uint32_t *__restrict__ slot_item, uint32_t *__restrict__ item_slot,
-                                v2 *__restrict__ scratch, uint32_t *__restrict__ ovf_count,
+                                uint32_t *__restrict__ slot_item, v2 *__restrict__ scratch, uint32_t *__restrict__ ovf_count,
                                 uint32_t *__restrict__ ovf_list) {
     __shared__ float4 s_stk[VKH_FLAT_STACK][2][VKH_FLAT_BLOCK]; // ancestors, two float4 per cubic
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -115,7 +114,6 @@ __global__ __launch_bounds__(VKH_FLAT_BLOCK) void k_flatten_stage(const vkh_item
     }
     const uint32_t slot = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
     slot_item[slot] = i;
-    item_slot[i] = slot;
     v2 *out = scratch + (size_t)slot * VKH_FLAT_SLOT;
     Cubic cb{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6], it.p[7]};
     uint32_t k = 0;
@@ -213,10 +211,95 @@ __global__ void k_flatten_overflow(const vkh_item *__restrict__ items, const uin
     }
 }
 
+// Frames of few cubics (at most VKH_FLAT_SPLIT_MAX): one thread per cubic leaves the chip idle while the
+// largest cubic's subdivision runs as one chain (its ~100 points, 140 us on 512x512 with 200 paths of large
+// cubics), so VKH_FLAT_PARTS threads take the subtrees below level VKH_FLAT_PART_LEVELS (agg_flatten_part):
+// now 31 us with the copy. Each repeats the splits above its subtree, about three times the work on a cubic of ten
+// points: 113 -> 37 us on 51 k such cubics, which still do not fill the chip; beyond the limit one
+// thread per cubic stays. A part keeps up to part_points points, a cubic with a longer part joins the
+// overflow list. The order puts cubics first, so a cubic's slot is its position.
+#define VKH_FLAT_PART_LEVELS 3
+#define VKH_FLAT_PARTS (1u << VKH_FLAT_PART_LEVELS)
+#define VKH_FLAT_OVER 0x80000000u // in a slot's first part count: the cubic overflows
+__global__ __launch_bounds__(VKH_FLAT_BLOCK) void k_flatten_split(
+    const vkh_item *__restrict__ items, uint32_t n, uint32_t n_cubics, const uint32_t *__restrict__ perm,
+    uint32_t *__restrict__ counts, uint32_t *__restrict__ part_cnt, v2 *__restrict__ scratch, uint32_t part_points,
+    uint32_t *__restrict__ ovf_count, uint32_t *__restrict__ ovf_list) {
+    __shared__ float4 s_stk[VKH_FLAT_STACK][2][VKH_FLAT_BLOCK];
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, nt = n_cubics * VKH_FLAT_PARTS;
+    if (t >= nt) { // the items that are not cubics
+        const uint32_t p = n_cubics + (t - nt);
+        if (p < n)
+            counts[perm[p]] = item_points(items[perm[p]]);
+        return;
+    }
+    const uint32_t slot = t / VKH_FLAT_PARTS, part = t % VKH_FLAT_PARTS, i = perm[slot];
+    const vkh_item it = items[i];
+    const Cubic cb{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6], it.p[7]};
+    v2 *out = scratch + (size_t)t * part_points;
+    uint32_t k = 0;
+    auto emit = [&](v2 p) {
+        if (k < part_points)
+            out[k] = p;
+        k++;
+    };
+    agg_flatten_part<VKH_FLAT_STACK, VKH_FLAT_PART_LEVELS>(
+        cb, part, it.tol, emit,
+        [&](int l, const Cubic &c) {
+            s_stk[l][0][threadIdx.x] = make_float4(c.x1, c.y1, c.x2, c.y2);
+            s_stk[l][1][threadIdx.x] = make_float4(c.x3, c.y3, c.x4, c.y4);
+        },
+        [&](int l) {
+            const float4 a = s_stk[l][0][threadIdx.x], b = s_stk[l][1][threadIdx.x];
+            return Cubic{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        });
+    if (part == VKH_FLAT_PARTS - 1 && !(it.flags & VKH_ITEM_NO_END))
+        emit(V(it.p[6], it.p[7]));
+    uint32_t total = k, over = k > part_points ? 1u : 0u; // a slot's parts are VKH_FLAT_PARTS lanes
+#pragma unroll
+    for (uint32_t o = 1; o < VKH_FLAT_PARTS; o <<= 1) {
+        total += (uint32_t)__shfl_xor((int)total, (int)o);
+        over |= (uint32_t)__shfl_xor((int)over, (int)o);
+    }
+    part_cnt[t] = k | (part == 0 && over ? VKH_FLAT_OVER : 0u);
+    if (part == 0) {
+        counts[i] = total;
+        if (over)
+            ovf_list[atomicAdd(ovf_count, 1u)] = i;
+    }
+}
+
+// VKH_FLAT_PARTS lanes per slot: the points of its parts one after another to their final positions
+__global__ void k_flatten_split_copy(const vkh_item *__restrict__ items, uint32_t n_cubics,
+                                     const uint32_t *__restrict__ perm, const uint32_t *__restrict__ part_cnt,
+                                     const uint32_t *__restrict__ offs, const v2 *__restrict__ scratch,
+                                     uint32_t part_points, v2 *__restrict__ pts, uint8_t *__restrict__ pflags) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t slot = t / VKH_FLAT_PARTS, lane = t % VKH_FLAT_PARTS;
+    if (slot >= n_cubics)
+        return;
+    const uint32_t *cnt = part_cnt + (size_t)slot * VKH_FLAT_PARTS;
+    if (cnt[0] & VKH_FLAT_OVER)
+        return; // written by k_flatten_overflow
+    const uint32_t i = perm[slot];
+    const uint8_t f = (items[i].flags & VKH_ITEM_CURVED) ? 1 : 0;
+    uint32_t o = offs[i];
+    for (uint32_t q = 0; q < VKH_FLAT_PARTS; q++) {
+        const v2 *src = scratch + ((size_t)slot * VKH_FLAT_PARTS + q) * part_points;
+        const uint32_t n = cnt[q];
+        for (uint32_t k = lane; k < n; k += VKH_FLAT_PARTS) {
+            pts[o + k] = src[k];
+            pflags[o + k] = f;
+        }
+        o += n;
+    }
+}
+
 // Diagnostic, not part of the public headers: the subdivision points of one cubic item (without its
 // end point), computed on the host by the flattening kernel's stack traversal (stack != 0, the
-// ancestors in a local array as the kernel keeps them in LDS) or by the stackless traversal of the
-// overflow kernel; returns the number of points, of which the first cap are written to xy.
+// ancestors in a local array as the kernel keeps them in LDS; stack == 2: part by part, as the split
+// kernel's lanes do) or by the stackless traversal of the overflow kernel; returns the number of points,
+// of which the first cap are written to xy.
 extern "C" uint32_t vkvg_hip_flatten_points(const vkh_item *it, int stack, float *xy, uint32_t cap) {
     const Cubic cb{it->p[0], it->p[1], it->p[2], it->p[3], it->p[4], it->p[5], it->p[6], it->p[7]};
     uint32_t k = 0;
@@ -227,7 +310,12 @@ extern "C" uint32_t vkvg_hip_flatten_points(const vkh_item *it, int stack, float
         }
         k++;
     };
-    if (stack) {
+    if (stack == 2) {
+        Cubic stk[VKH_FLAT_STACK];
+        for (uint32_t p = 0; p < VKH_FLAT_PARTS; p++)
+            agg_flatten_part<VKH_FLAT_STACK, VKH_FLAT_PART_LEVELS>(
+                cb, p, it->tol, emit, [&](int l, const Cubic &c) { stk[l] = c; }, [&](int l) { return stk[l]; });
+    } else if (stack) {
         Cubic stk[VKH_FLAT_STACK];
         agg_flatten_stack<VKH_FLAT_STACK>(
             cb, it->tol, emit, [&](int l, const Cubic &c) { stk[l] = c; }, [&](int l) { return stk[l]; });
@@ -1505,12 +1593,33 @@ void launch_flat_scatter(hipStream_t s, const vkh_item *items, uint32_t n, const
                            flat_order_groups(n), perm);
 }
 void launch_flatten_stage(hipStream_t s, const vkh_item *items, uint32_t n, const uint32_t *perm, uint32_t *counts,
-                          uint32_t *slot_alloc, uint32_t *slot_item, uint32_t *item_slot, v2 *scratch,
+                          uint32_t *slot_alloc, uint32_t *slot_item, v2 *scratch,
                           uint32_t *ovf_count, uint32_t *ovf_list) {
     if (n)
         hipLaunchKernelGGL(k_flatten_stage, dim3((n + VKH_FLAT_BLOCK - 1) / VKH_FLAT_BLOCK), dim3(VKH_FLAT_BLOCK), 0, s,
                            items, n, perm, counts, slot_alloc,
-                           slot_item, item_slot, scratch, ovf_count, ovf_list);
+                           slot_item, scratch, ovf_count, ovf_list);
+}
+uint32_t flat_split_points(uint32_t n_cubics) {
+    return n_cubics > VKH_FLAT_SPLIT_MAX ? 0u : n_cubics > VKH_FLAT_SPLIT_MAX / 4 ? 32u : 64u;
+}
+size_t flat_split_parts(uint32_t n_cubics) { return (size_t)n_cubics * VKH_FLAT_PARTS; }
+void launch_flatten_split(hipStream_t s, const vkh_item *items, uint32_t n, uint32_t n_cubics, const uint32_t *perm,
+                          uint32_t *counts, uint32_t *part_cnt, v2 *scratch, uint32_t *ovf_count,
+                          uint32_t *ovf_list) {
+    const uint32_t threads = n_cubics * VKH_FLAT_PARTS + (n - n_cubics);
+    if (threads)
+        hipLaunchKernelGGL(k_flatten_split, dim3((threads + VKH_FLAT_BLOCK - 1) / VKH_FLAT_BLOCK), dim3(VKH_FLAT_BLOCK),
+                           0, s, items, n, n_cubics, perm, counts, part_cnt, scratch, flat_split_points(n_cubics),
+                           ovf_count, ovf_list);
+}
+void launch_flatten_split_copy(hipStream_t s, const vkh_item *items, uint32_t n_cubics, const uint32_t *perm,
+                               const uint32_t *part_cnt, const uint32_t *offs, const v2 *scratch, v2 *pts,
+                               uint8_t *pf) {
+    const uint32_t threads = n_cubics * VKH_FLAT_PARTS;
+    if (threads)
+        hipLaunchKernelGGL(k_flatten_split_copy, dim3((threads + 255) / 256), dim3(256), 0, s, items, n_cubics, perm,
+                           part_cnt, offs, scratch, flat_split_points(n_cubics), pts, pf);
 }
 void launch_flatten_copy(hipStream_t s, const vkh_item *items, uint32_t n_slots, const uint32_t *slot_item,
                          const uint32_t *counts, const uint32_t *offs, const v2 *scratch, v2 *pts, uint8_t *pf) {

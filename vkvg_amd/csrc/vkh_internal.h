@@ -12,6 +12,7 @@
 #define VKH_COARSE_CHUNK 1024   // most draws per coarse workgroup
 #define VKH_COARSE_MIN 16       // fewest
 #define VKH_FLAT_SLOT 128       // flattened points kept per cubic by the subdivision pass
+#define VKH_FLAT_SPLIT_MAX 65536u // cubics up to which a frame's cubics are split over several threads
 
 // one (draw, subpath) pair of the frame; fills and strokes are expanded per unit
 struct Unit {
@@ -129,8 +130,18 @@ uint32_t flat_order_groups(uint32_t n); // workgroups of the flattening order's 
 void launch_flat_hist(hipStream_t s, const vkh_item *items, uint32_t n, uint32_t *whist);
 void launch_flat_scatter(hipStream_t s, const vkh_item *items, uint32_t n, const uint32_t *wcur, uint32_t *perm);
 void launch_flatten_stage(hipStream_t s, const vkh_item *items, uint32_t n, const uint32_t *perm, uint32_t *counts,
-                          uint32_t *slot_alloc, uint32_t *slot_item, uint32_t *item_slot, v2 *scratch,
+                          uint32_t *slot_alloc, uint32_t *slot_item, v2 *scratch,
                           uint32_t *ovf_count, uint32_t *ovf_list);
+// frames of few cubics: several threads per cubic. The points kept per part (0: the frame has too many
+// cubics for this path), the parts of all cubics
+uint32_t flat_split_points(uint32_t n_cubics);
+size_t flat_split_parts(uint32_t n_cubics);
+void launch_flatten_split(hipStream_t s, const vkh_item *items, uint32_t n, uint32_t n_cubics, const uint32_t *perm,
+                          uint32_t *counts, uint32_t *part_cnt, v2 *scratch, uint32_t *ovf_count,
+                          uint32_t *ovf_list);
+void launch_flatten_split_copy(hipStream_t s, const vkh_item *items, uint32_t n_cubics, const uint32_t *perm,
+                               const uint32_t *part_cnt, const uint32_t *offs, const v2 *scratch, v2 *pts,
+                               uint8_t *pf);
 void launch_flatten_copy(hipStream_t s, const vkh_item *items, uint32_t n_slots, const uint32_t *slot_item,
                          const uint32_t *counts, const uint32_t *offs, const v2 *scratch, v2 *pts, uint8_t *pf);
 void launch_flatten_lines(hipStream_t s, const vkh_item *items, uint32_t n, const uint32_t *offs, v2 *pts,
