@@ -58,27 +58,34 @@ VKH_HD float d_acosf(float a) { return (float)acos((double)a); }
 // :485-498) and of elliptic arcs (src/vkvg_context_internal.c:1555-1574), one point per step of
 // the reference's sequential angle recurrence. The float (circle) or double (ellipse) angle is
 // advanced by one addition per point, as the reference's loop does, so every point repeats the
-// reference's operations exactly; the host counted the points with the same additions.
+// reference's operations exactly; the host counted the points with the same additions. Several
+// threads can share an arc: each takes every step-th point from first on, and repeats the additions.
 VKH_HD uint32_t item_points(const vkh_item &it) {
     return (it.flags & (VKH_ITEM_ARC | VKH_ITEM_EARC)) ? it.flags >> VKH_ITEM_COUNT_SHIFT : 1u;
 }
-template <class F> VKH_HD void arc_points(const vkh_item &it, F emit) {
+template <class F> VKH_HD void arc_points(const vkh_item &it, F emit, uint32_t first = 0, uint32_t step = 1) {
     const uint32_t n = it.flags >> VKH_ITEM_COUNT_SHIFT;
     if (it.flags & VKH_ITEM_ARC) {
         const float xc = it.p[0], yc = it.p[1], r = it.p[2], s = it.p[4];
         float a = it.p[3];
-        for (uint32_t k = 0; k < n; k++) {
-            emit(V(d_cosf(a) * r + xc, d_sinf(a) * r + yc));
+        for (uint32_t j = 0; j < first; j++)
             a += s;
+        for (uint32_t k = first; k < n; k += step) {
+            emit(V(d_cosf(a) * r + xc, d_sinf(a) * r + yc));
+            for (uint32_t j = 0; j < step; j++)
+                a += s;
         }
     } else {
         double th;
         memcpy(&th, it.p, sizeof(th));
         const float s = it.p[2], rx = it.p[3], ry = it.p[4], cph = it.p[5], sph = it.p[6], cx = it.p[7], cy = it.tol;
-        for (uint32_t k = 0; k < n; k++) {
+        for (uint32_t j = 0; j < first; j++)
+            th += s;
+        for (uint32_t k = first; k < n; k += step) {
             const float ex = rx * d_cosf((float)th), ey = ry * d_sinf((float)th);
             emit(V(((cph * ex) + (-sph * ey)) + cx, ((sph * ex) + (cph * ey)) + cy));
-            th += s;
+            for (uint32_t j = 0; j < step; j++)
+                th += s;
         }
     }
 }

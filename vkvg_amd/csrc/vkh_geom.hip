@@ -165,27 +165,52 @@ __global__ void k_flatten_copy(const vkh_item *__restrict__ items, uint32_t n_sl
     }
 }
 
-__global__ void k_flatten_lines(const vkh_item *__restrict__ items, uint32_t n, const uint32_t *__restrict__ offs,
-                                v2 *__restrict__ pts, uint8_t *__restrict__ pflags) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    const vkh_item it = items[i];
-    if (it.flags & VKH_ITEM_CUBIC)
-        return;
-    const uint32_t o = offs[i];
-    const uint8_t f = (it.flags & VKH_ITEM_CURVED) ? 1 : 0;
-    if (it.flags & (VKH_ITEM_ARC | VKH_ITEM_EARC)) {
-        uint32_t k = o;
-        arc_points(it, [&](v2 p) {
-            pts[k] = p;
-            pflags[k] = f;
-            k++;
-        });
-        return;
+// Lines, one per thread, and arcs: a wavefront's arcs are shared out over its lanes, 64 lanes to a lone
+// one down to eight each, since a point's sine and cosine are a chain of hundreds of instructions and one
+// thread per arc runs them in series for the longest arc of the frame, while the angle's additions, which
+// every lane repeats, are one instruction a point. 777x777 with 150 shapes: 87 -> 23 us; a wavefront
+// full of arcs does an eighth of the points per lane for each eighth of its arcs, as much as before.
+#define VKH_ARC_LANES 8u
+__global__ __launch_bounds__(256) void k_flatten_lines(const vkh_item *__restrict__ items, uint32_t n,
+                                                       const uint32_t *__restrict__ offs, v2 *__restrict__ pts,
+                                                       uint8_t *__restrict__ pflags) {
+    __shared__ uint32_t s_arc[256];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+    bool arc = false;
+    if (i < n) {
+        const uint32_t fl = items[i].flags;
+        arc = (fl & (VKH_ITEM_ARC | VKH_ITEM_EARC)) != 0;
+        if (!arc && !(fl & VKH_ITEM_CUBIC)) {
+            const uint32_t o = offs[i];
+            pts[o] = V(items[i].p[0], items[i].p[1]);
+            pflags[o] = (fl & VKH_ITEM_CURVED) ? 1 : 0;
+        }
     }
-    pts[o] = V(it.p[0], it.p[1]);
-    pflags[o] = f;
+    const uint64_t m = __ballot(arc);
+    if (!m)
+        return;
+    const uint32_t n_arcs = (uint32_t)__popcll(m);
+    uint32_t *list = s_arc + (threadIdx.x & ~63u); // this wavefront's own; its LDS accesses complete in order
+    if (arc)
+        list[__popcll(m & ((1ull << lane) - 1ull))] = i;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint32_t lanes = 64;
+    while (lanes > VKH_ARC_LANES && lanes * n_arcs > 64u)
+        lanes >>= 1;
+    for (uint32_t a = lane / lanes; a < n_arcs; a += 64u / lanes) {
+        const vkh_item it = items[list[a]];
+        const uint32_t first = lane & (lanes - 1u);
+        uint32_t k = offs[list[a]] + first;
+        const uint8_t f = (it.flags & VKH_ITEM_CURVED) ? 1 : 0;
+        arc_points(
+            it,
+            [&](v2 p) {
+                pts[k] = p;
+                pflags[k] = f;
+                k += lanes;
+            },
+            first, lanes);
+    }
 }
 
 // the listed cubics with more points than a slot holds, traversed again into their positions
