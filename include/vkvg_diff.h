@@ -41,8 +41,8 @@ vkvg_public VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint
                                const uint32_t *is_stroke);
 vkvg_public void vkvg_diff_destroy(VkvgDiffScene s);
 
-/* Renders the image. With keep != 0 the compositing checkpoints the backward pass needs are kept
- * (coverage itself is recomputed by the backward pass). */
+/* Renders the image. With keep != 0 the compositing checkpoints and the coverage that the
+ * backward pass needs are kept. */
 vkvg_public int vkvg_diff_forward(VkvgDiffScene s, const float *ctrl, const float *rgba, const float *width, float *image,
                       int keep);
 
@@ -58,7 +58,7 @@ vkvg_public int vkvg_diff_backward(VkvgDiffScene s, const float *ctrl, const flo
                        const float *grad_image, float *grad_ctrl, float *grad_rgba, float *grad_width);
 
 /* Device time of the last forward / backward call in milliseconds, and frame statistics:
- * out[0] edges, out[1] segments, out[2] commands, out[3] batches. */
+ * out[0] edges, out[1] list entries (edge x tile row), out[2] commands, out[3] batches. */
 vkvg_public float vkvg_diff_last_ms(VkvgDiffScene s, int backward);
 vkvg_public void vkvg_diff_stats(VkvgDiffScene s, uint32_t out[4]);
 vkvg_public const char *vkvg_diff_last_error(VkvgDiffScene s);

@@ -1,0 +1,76 @@
+"""Differentiable renderer at the edges of its row units against the FP64 reference: paths of one tile, of
+exactly eight tiles and more (128 columns are added up at a time), across all borders of the image, edges
+on tile borders, images smaller than a tile and paths off the image.
+
+Tolerances: coordinates below 512 are spaced 3e-5 px and an edge's ends take about four roundings, so an
+edge lies within 1.2e-4 px of the reference's, which moves the coverage of a pixel by at most that per
+edge in it, of which these scenes have up to four: 5e-4. Gradients are the integral of numbers known to
+that over pieces known to that: 2e-3 of their norm."""
+import numpy as np
+import pytest
+
+from oracle import diff_ref as D
+
+pytestmark = pytest.mark.gpu
+
+
+def _polygon(points, bend=0.0):
+    """A closed path of cubics through the points, straight (control points at thirds) or bent by that part
+    of their length."""
+    p = np.asarray(points, np.float64)
+    d = np.roll(p, -1, 0) - p
+    side = bend * d[:, ::-1] * [-1, 1]
+    return np.stack([p, p + d / 3 + side, p + 2 * d / 3 + side], 1).reshape(-1, 2)
+
+
+def _scene(name):
+    r = np.random.Generator(np.random.PCG64(77))
+    if name == "tile":  # within one tile, within two
+        return 64, 48, [_polygon(16 + 14 * r.random((4, 2))), _polygon([20, 10] + 20 * r.random((3, 2)), 0.3)], [0, 1]
+    if name == "aligned":  # borders on pixels, tiles and the 128 columns
+        box = lambda x0, y0, x1, y1: _polygon([(x0, y0), (x1, y0), (x1, y1), (x0, y1)])  # noqa: E731
+        return 288, 32, [box(16, 0, 144, 16), box(128, 5, 256, 32), box(0.5, 8, 128, 9), box(-20, 12, 300, 20)], [0] * 4
+    if name == "wide":  # several times 128 columns, across all borders
+        w = np.array([[-40.3, 7.7], [150.2, -9.1], [430.6, 22.3], [260.4, 61.8], [90.1, 44.4]])
+        return 391, 40, [_polygon(w), _polygon(w[::-1] * [0.6, 0.8] + [30.5, 3.1]), _polygon(w * 0.9, 0.3)], [0, 0, 1]
+    if name == "tall":
+        w = np.array([[3.3, -20.7], [17.2, 80.1], [9.6, 200.3], [-6.4, 141.8]])
+        return 15, 177, [_polygon(w), _polygon(w + [2.2, 9.3], 0.3)], [0, 1]
+    if name == "point":  # one pixel, and a path that misses it on each side
+        return 1, 1, [_polygon([[-0.7, 0.3], [0.6, -0.4], [0.9, 1.6]]), _polygon([[5, 5], [7, 5], [6, 8]]),
+                      _polygon([[-9, 0.2], [-4, 0.4], [-6, 0.9]]), _polygon([[0.1, -8], [0.7, -3], [0.3, -5]])], [0, 0, 1, 0]
+    paths = []
+    for _ in range(12):  # "curved": closed cubics of all sizes
+        c, s = r.uniform(0, (211, 75)), np.exp(r.uniform(0, 4.0))
+        paths.append(c + s * r.standard_normal((3 * int(r.integers(1, 5)), 2)))
+    return 211, 75, paths, list(r.integers(0, 2, 12))
+
+
+@pytest.mark.parametrize("name", ["tile", "aligned", "wide", "tall", "point", "curved"])
+def test_rows_match_fp64_reference(name):
+    import torch
+    from vkvg_amd import diff
+    W, H, paths, stroke = _scene(name)
+    r = np.random.Generator(np.random.PCG64(5))
+    n = len(paths)
+    nc = np.array([len(p) // 3 for p in paths], np.uint32)
+    stroke = np.array(stroke, np.uint32)
+    ctrl = np.concatenate(paths).astype(np.float32)
+    rgba = r.uniform(0.2, 0.9, (n, 4)).astype(np.float32)
+    lw = np.where(stroke, r.uniform(1, 5, n), 0).astype(np.float32)
+    g_img = r.standard_normal((H, W, 4)).astype(np.float32)
+    ref_scene = D.Scene(W, H, nc, stroke)
+    ref = D.forward(ref_scene, ctrl, rgba, lw)
+    R = diff.DiffRenderer(W, H, nc, stroke)
+    c, k, w = (torch.tensor(x, device="cuda") for x in (ctrl, rgba, lw))
+    img = R.forward(c, k, w, keep=True)
+    assert np.abs(img.cpu().numpy() - ref).max() < 5e-4
+    if name != "aligned":  # there |coverage| is exactly 1, where the clamp has no derivative
+        g = torch.tensor(g_img, device="cuda")
+        want = D.backward(ref_scene, ctrl, rgba, lw, g_img.astype(np.float64))
+        for _ in range(2):  # a second backward of the same forward gives the same
+            for what, a, b in zip(("ctrl", "rgba", "width"), R.backward(c, k, w, g), want):
+                e = np.linalg.norm(a.cpu().numpy() - b) / max(np.linalg.norm(b), 1e-30)
+                assert e < 2e-3, (what, e)
+    assert np.abs(R.forward64(c, k, w).cpu().numpy() - ref).max() < 1e-9
+    R.close()

@@ -57,7 +57,7 @@ struct PathTile {
     uint32_t seg_off;  // into the segment index array
     union {
         uint32_t sat;    // rendering: the gradient's colour over the tile is its first (1) or last (2) stop's
-        uint32_t ntouch; // differentiable renderer: of the edges, how many touch the tile (listed first)
+        uint32_t ntouch; // differentiable renderer: the edges of the tile row (in the row's first tile)
     };
 };
 
