@@ -5,10 +5,11 @@
 //   k_dflatten      one thread per polyline point: Bernstein sample of its cubic
 //   k_dnormals      one thread per point: unit left normal of the segment leaving it (strokes)
 //   k_dedges        one thread per point: the fill edge, or the stroke's rectangle + 2 bevel
-//                   triangles (10 edges), each endpoint tagged (point, normal, sign) for backward
-//   k_dbbox         one workgroup per path: bbox of its edges (deterministic reduction)
-//   draw tiles, scan, k_dbin (per path: every tile row's list of the edges in it, and from which
-//   tile on the row has coverage), coarse
+//                   triangles (10 edges)
+//   k_dpaths        one workgroup per path: bbox of its edges in tiles and how many list entries the
+//                   tile rows take; k_dalloc: the paths' positions and the totals, for the host
+//   k_dbin          per path: every tile row's list of the edges in it, and from which tile on the row
+//                   has coverage; then the coarse pass
 //   k_dcmd_of       the command of every path tile
 //   k_dcov          one wavefront per (path, tile row): its edges' area deltas are added up in LDS over
 //                   the path's whole width, eight tiles at a time, and prefix-summed along the pixel rows
@@ -21,16 +22,18 @@
 //   k_dback         per tile, batches in reverse: reads the batch's coverage, replays the
 //                   batch's compositing from its checkpoint and walks it backwards to get dL/dA per
 //                   (command, pixel) and the colour gradients
-//   k_dedge_grad    one thread per edge: the boundary integral of dL/dA over every piece of the
-//                   edge inside a pixel, in all tiles that it touches, is its endpoints' gradient
-//   k_dg_normal_sums, k_dg_points, k_dg_ctrl, k_dg_paths: chain rule to normals, half-widths,
-//                   points, control points, colours and widths, all as gathers
+//   k_dedge_grad    one wavefront per 6 points of a stroke or 60 of a fill: the boundary integral of
+//                   dL/dA over every piece of their edges inside a pixel, in all tiles that they
+//                   cross, added up to the gradients of the points and normals that the edges hang on
+//   k_dg_points, k_dg_ctrl, k_dg_paths: chain rule to points, half-widths, control points, colours and
+//                   widths, all as gathers
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "vkh_internal.h"
@@ -44,10 +47,6 @@
 #define VKD_BIN_MARGIN 0.01f // px added around an edge when binning (rounding safety)
 
 namespace {
-
-struct DSrc { // endpoint tags of an edge: point index, normal index | (sign + 1) << 30
-    uint32_t ia, ka, ib, kb;
-};
 
 __device__ __forceinline__ float2 f2(float x, float y) { return make_float2(x, y); }
 
@@ -102,7 +101,6 @@ __global__ void k_dnormals(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
     nrm[p] = L > (R)0 ? r2<R>(-dy / L, dx / L) : r2<R>((R)0, (R)0);
 }
 
-__device__ __forceinline__ uint32_t tag(uint32_t k, int s) { return k | ((uint32_t)(s + 1) << 30); }
 template <typename R>
 __device__ __forceinline__ RV2<R> vpos(const RV2<R> *pts, const RV2<R> *nrm, R h, uint32_t i, uint32_t k, int s) {
     if (!s)
@@ -115,8 +113,7 @@ template <typename R>
 __global__ void k_dedges(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
                          const uint32_t *__restrict__ path_first_pt, const uint32_t *__restrict__ path_first_edge,
                          const uint32_t *__restrict__ path_stroke, const float *__restrict__ width,
-                         const RV2<R> *__restrict__ pts, const RV2<R> *__restrict__ nrm, RV4<R> *__restrict__ edges,
-                         DSrc *__restrict__ src) {
+                         const RV2<R> *__restrict__ pts, const RV2<R> *__restrict__ nrm, RV4<R> *__restrict__ edges) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n_pts)
         return;
@@ -127,8 +124,6 @@ __global__ void k_dedges(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
     if (!path_stroke[path]) {
         uint32_t e = path_first_edge[path] + j;
         edges[e] = RV4<R>{pts[p].x, pts[p].y, pts[nx].x, pts[nx].y};
-        if (src)
-            src[e] = DSrc{p, tag(0, 0), nx, tag(0, 0)};
         return;
     }
     const R h = (R)0.5 * (R)width[path];
@@ -139,8 +134,6 @@ __global__ void k_dedges(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
         int b = (a + 1) & 3;
         RV2<R> A = vpos(pts, nrm, h, vi[a], vk[a], vs[a]), Bv = vpos(pts, nrm, h, vi[b], vk[b], vs[b]);
         edges[e] = RV4<R>{A.x, A.y, Bv.x, Bv.y};
-        if (src)
-            src[e] = DSrc{vi[a], tag(vk[a], vs[a]), vi[b], tag(vk[b], vs[b])};
         e++;
     }
     uint32_t pp = prev_pt(p, first, end);
@@ -157,58 +150,8 @@ __global__ void k_dedges(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
             int b = a == 2 ? 0 : a + 1;
             RV2<R> A = vpos(pts, nrm, h, ti[a], tk[a], ts[a]), Bv = vpos(pts, nrm, h, ti[b], tk[b], ts[b]);
             edges[e] = RV4<R>{A.x, A.y, Bv.x, Bv.y};
-            if (src)
-                src[e] = DSrc{ti[a], tag(tk[a], ts[a]), ti[b], tag(tk[b], ts[b])};
             e++;
         }
-    }
-}
-
-// bbox of a path's edges in 24.8 fixed point (floor / ceil), one workgroup per path
-template <typename R>
-__global__ __launch_bounds__(256) void k_dbbox(const uint32_t *__restrict__ path_first_edge,
-                                               const RV4<R> *__restrict__ edges, int4 *__restrict__ bbox) {
-    __shared__ int32_t red[4][4];
-    uint32_t d = blockIdx.x, tid = threadIdx.x;
-    float x0 = 3.0e38f, y0 = 3.0e38f, x1 = -3.0e38f, y1 = -3.0e38f;
-    for (uint32_t e = path_first_edge[d] + tid; e < path_first_edge[d + 1]; e += 256) {
-        const RV4<R> v = edges[e];
-        if (v.y == v.w || isnan(v.x) || isnan(v.y) || isnan(v.z) || isnan(v.w))
-            continue; // horizontal edges contribute nothing
-        // widened by the binning margin so that rounding to float never loses a tile
-        x0 = fminf(x0, (float)fmin(v.x, v.z) - VKD_BIN_MARGIN);
-        x1 = fmaxf(x1, (float)fmax(v.x, v.z) + VKD_BIN_MARGIN);
-        y0 = fminf(y0, (float)fmin(v.y, v.w) - VKD_BIN_MARGIN);
-        y1 = fmaxf(y1, (float)fmax(v.y, v.w) + VKD_BIN_MARGIN);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        x0 = fminf(x0, __shfl_xor(x0, o));
-        y0 = fminf(y0, __shfl_xor(y0, o));
-        x1 = fmaxf(x1, __shfl_xor(x1, o));
-        y1 = fmaxf(y1, __shfl_xor(y1, o));
-    }
-    auto fx = [](float v, bool up) -> int32_t {
-        float s = v * 256.0f;
-        s = up ? ceilf(s) : floorf(s);
-        return (int32_t)fminf(fmaxf(s, -8.0e6f), 8.0e6f);
-    };
-    if ((tid & 63) == 0) {
-        int w = tid >> 6;
-        red[w][0] = x0 > x1 ? INT32_MAX : fx(x0, false);
-        red[w][1] = x0 > x1 ? INT32_MAX : fx(y0, false);
-        red[w][2] = x0 > x1 ? INT32_MIN : fx(x1, true);
-        red[w][3] = x0 > x1 ? INT32_MIN : fx(y1, true);
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int4 b = make_int4(INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN);
-        for (int w = 0; w < 4; w++) {
-            b.x = min(b.x, red[w][0]);
-            b.y = min(b.y, red[w][1]);
-            b.z = max(b.z, red[w][2]);
-            b.w = max(b.w, red[w][3]);
-        }
-        bbox[d] = b;
     }
 }
 
@@ -238,6 +181,135 @@ __device__ __forceinline__ void dbin_range(const RV4<R> &v, const DrawTiles &dt,
         return;
     r0 = max(tile_of(ymin), dt.by0);
     r1 = min(tile_of(ymax), dt.by1);
+}
+
+// What a path takes: path tiles, tile rows, list entries; then where its own begin
+struct PathAlloc {
+    uint32_t tiles, rows, segs;
+};
+
+// One workgroup per path: bbox of its edges in 24.8 fixed point (floor / ceil) and from it the tiles
+template <typename R>
+__global__ __launch_bounds__(256) void k_dpaths(const uint32_t *__restrict__ path_first_edge,
+                                                const RV4<R> *__restrict__ edges, int32_t tilesW, int32_t tilesH,
+                                                DrawTiles *__restrict__ dts, PathAlloc *__restrict__ alloc) {
+    __shared__ int32_t red[4][4];
+    __shared__ uint32_t s_sum[4];
+    const uint32_t d = blockIdx.x, tid = threadIdx.x;
+    const uint32_t e0 = path_first_edge[d], e1 = path_first_edge[d + 1];
+    float x0 = 3.0e38f, y0 = 3.0e38f, x1 = -3.0e38f, y1 = -3.0e38f;
+    for (uint32_t e = e0 + tid; e < e1; e += 256) {
+        const RV4<R> v = edges[e];
+        if (v.y == v.w || isnan(v.x) || isnan(v.y) || isnan(v.z) || isnan(v.w))
+            continue; // horizontal edges contribute nothing
+        // widened by the binning margin so that rounding to float never loses a tile
+        x0 = fminf(x0, (float)fmin(v.x, v.z) - VKD_BIN_MARGIN);
+        x1 = fmaxf(x1, (float)fmax(v.x, v.z) + VKD_BIN_MARGIN);
+        y0 = fminf(y0, (float)fmin(v.y, v.w) - VKD_BIN_MARGIN);
+        y1 = fmaxf(y1, (float)fmax(v.y, v.w) + VKD_BIN_MARGIN);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        x0 = fminf(x0, __shfl_xor(x0, o));
+        y0 = fminf(y0, __shfl_xor(y0, o));
+        x1 = fmaxf(x1, __shfl_xor(x1, o));
+        y1 = fmaxf(y1, __shfl_xor(y1, o));
+    }
+    auto fx = [](float v, bool up) -> int32_t {
+        float s = v * 256.0f;
+        s = up ? ceilf(s) : floorf(s);
+        return (int32_t)fminf(fmaxf(s, -8.0e6f), 8.0e6f);
+    };
+    if ((tid & 63) == 0) {
+        int w = tid >> 6;
+        red[w][0] = x0 > x1 ? INT32_MAX : fx(x0, false);
+        red[w][1] = x0 > x1 ? INT32_MAX : fx(y0, false);
+        red[w][2] = x0 > x1 ? INT32_MIN : fx(x1, true);
+        red[w][3] = x0 > x1 ? INT32_MIN : fx(y1, true);
+    }
+    __syncthreads();
+    int4 b = make_int4(INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN);
+    for (int w = 0; w < 4; w++) {
+        b.x = min(b.x, red[w][0]);
+        b.y = min(b.y, red[w][1]);
+        b.z = max(b.z, red[w][2]);
+        b.w = max(b.w, red[w][3]);
+    }
+    constexpr int SSH = 8 + __builtin_ctz(VKD_T);
+    DrawTiles dt;
+    dt.bx0 = dt.by0 = 0;
+    dt.bx1 = dt.by1 = -1;
+    if (b.x <= b.z) {
+        dt.bx0 = max(b.x >> SSH, 0);
+        dt.by0 = max(b.y >> SSH, 0);
+        dt.bx1 = min(b.z >> SSH, tilesW - 1);
+        dt.by1 = min(b.w >> SSH, tilesH - 1);
+    }
+    const bool some = dt.bx0 <= dt.bx1 && dt.by0 <= dt.by1;
+    if (!some) {
+        dt.bx0 = dt.by0 = 0;
+        dt.bx1 = dt.by1 = -1;
+    }
+    dt.pt_base = 0;
+    dt.bw = some ? (uint32_t)(dt.bx1 - dt.bx0 + 1) : 0u;
+    uint32_t n = 0;
+    if (some)
+        for (uint32_t e = e0 + tid; e < e1; e += 256) {
+            int32_t r0, r1, c0;
+            dbin_range(edges[e], dt, r0, r1, c0);
+            n += r0 <= r1 ? (uint32_t)(r1 - r0 + 1) : 0u;
+        }
+    for (int o = 32; o > 0; o >>= 1)
+        n += __shfl_xor(n, o);
+    if ((tid & 63) == 0)
+        s_sum[tid >> 6] = n;
+    __syncthreads();
+    if (tid == 0) {
+        const uint32_t rows = (uint32_t)(dt.by1 - dt.by0 + 1);
+        dts[d] = dt;
+        alloc[d] = PathAlloc{dt.bw * rows, rows, s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]};
+    }
+}
+
+// Positions of every path's tiles, rows and list entries (exclusive sums, in one workgroup), and the totals
+// into the host's memory
+__global__ __launch_bounds__(1024) void k_dalloc(uint32_t n_paths, PathAlloc *__restrict__ alloc,
+                                                 DrawTiles *__restrict__ dts, uint32_t *__restrict__ totals) {
+    __shared__ uint32_t s_w[16][3];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
+    uint32_t run[3] = {0, 0, 0};
+    for (uint32_t base = 0; base < n_paths; base += 1024) {
+        const uint32_t d = base + tid;
+        const PathAlloc a = d < n_paths ? alloc[d] : PathAlloc{0, 0, 0};
+        const uint32_t v[3] = {a.tiles, a.rows, a.segs};
+        uint32_t x[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            x[k] = v[k];
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = __shfl_up(x[k], o);
+                x[k] += (int)lane >= o ? y : 0u;
+            }
+            if (lane == 63)
+                s_w[wv][k] = x[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            x[k] += run[k] - v[k];
+            for (uint32_t w = 0; w < 16; w++) {
+                x[k] += w < wv ? s_w[w][k] : 0u;
+                run[k] += s_w[w][k];
+            }
+        }
+        if (d < n_paths) {
+            alloc[d] = PathAlloc{x[0], x[1], x[2]};
+            dts[d].pt_base = x[0];
+        }
+        __syncthreads();
+    }
+    if (tid == 0)
+        for (int k = 0; k < 3; k++)
+            totals[k] = run[k];
 }
 
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uint32_t *s_wave) {
@@ -275,23 +347,20 @@ struct RowUnit {
     uint32_t draw, row;
 };
 
-// alloc[0]: list entries, alloc[1]: units; both are what the frame needs, also where that is more than
-// seg_cap (then lists are not written, and the host makes room and runs this again)
 template <typename R>
 __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_first_edge,
                                               const RV4<R> *__restrict__ edges, const DrawTiles *__restrict__ dts,
-                                              PathTile *__restrict__ ptl, uint32_t *__restrict__ cmd_of,
-                                              uint32_t *__restrict__ segs, uint32_t seg_cap,
-                                              RowUnit *__restrict__ units, uint32_t *__restrict__ alloc) {
+                                              const PathAlloc *__restrict__ alloc, PathTile *__restrict__ ptl,
+                                              uint32_t *__restrict__ cmd_of, uint32_t *__restrict__ segs,
+                                              RowUnit *__restrict__ units) {
     __shared__ uint32_t s_cnt[VKD_ROWS_MAX]; // edges per row, then offsets, then cursors
     __shared__ int32_t s_col[VKD_ROWS_MAX];  // first tile column reached
     __shared__ uint32_t s_wave[4];
-    __shared__ uint32_t s_base, s_units;
     const uint32_t d = blockIdx.x, tid = threadIdx.x;
     const DrawTiles dt = dts[d];
-    if (dt.bw == 0 || dt.bx0 > dt.bx1 || dt.by0 > dt.by1)
+    if (dt.bw == 0)
         return;
-    const uint32_t e0 = path_first_edge[d], e1 = path_first_edge[d + 1];
+    const uint32_t e0 = path_first_edge[d], e1 = path_first_edge[d + 1], base = alloc[d].segs, unit0 = alloc[d].rows;
     const uint32_t bw = dt.bw, bh = (uint32_t)(dt.by1 - dt.by0 + 1); // at most VKD_ROWS_MAX rows
     for (uint32_t k = tid; k < bh; k += 256) {
         s_cnt[k] = 0;
@@ -308,13 +377,6 @@ __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_
     }
     __syncthreads();
     const uint32_t total = block_excl_scan(s_cnt, bh, s_wave);
-    if (tid == 0) {
-        s_base = atomicAdd(&alloc[0], total);
-        s_units = atomicAdd(&alloc[1], bh);
-    }
-    __syncthreads();
-    const uint32_t base = s_base;
-    const bool fits = (uint64_t)base + total <= (uint64_t)seg_cap;
     for (uint32_t k = tid; k < bh * bw; k += 256) {
         const uint32_t r = k / bw, off = s_cnt[r], next = r + 1 < bh ? s_cnt[r + 1] : total;
         PathTile pt;
@@ -326,10 +388,8 @@ __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_
         cmd_of[dt.pt_base + k] = VKD_NO_CMD;
     }
     for (uint32_t k = tid; k < bh; k += 256)
-        units[s_units + k] = RowUnit{d, k};
+        units[unit0 + k] = RowUnit{d, k};
     __syncthreads();
-    if (!fits)
-        return;
     for (uint32_t e = e0 + tid; e < e1; e += 256) {
         int32_t r0, r1, c0;
         dbin_range(edges[e], dt, r0, r1, c0);
@@ -373,6 +433,36 @@ template <typename R> struct RowPart {
         return x <= xl ? (R)0 : x >= xr ? dy : fabs(param(x) - sL) * dyt;
     }
 };
+
+// Rows shared out over a wavefront: every lane has an edge with cnt (at most 16) pixel rows from row
+// `first` on, and f(lane of the edge, row) is called once for each of all the lanes' rows, 64 at a time. Edges
+// cross few rows, some many: a lane doing its own edge's rows would wait for the longest.
+struct RowShare {
+    uint8_t lane[64 * VKD_T];
+    int32_t row[64]; // of the edge's item 0
+};
+template <class F> __device__ __forceinline__ void share_rows(RowShare &sh, uint32_t lane, int32_t first, uint32_t cnt, F f) {
+    uint32_t x = cnt; // inclusive sum over the lanes
+#define VKD_DPP(ctrl, rows) (uint32_t) __builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xf, false)
+    x += VKD_DPP(0x111, 0xf); // row_shr:1, 2, 4, 8, then row_bcast:15 and 31
+    x += VKD_DPP(0x112, 0xf);
+    x += VKD_DPP(0x114, 0xf);
+    x += VKD_DPP(0x118, 0xf);
+    x += VKD_DPP(0x142, 0xa);
+    x += VKD_DPP(0x143, 0xc);
+#undef VKD_DPP
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)x, 63), at = x - cnt;
+    sh.row[lane] = first - (int32_t)at;
+    for (uint32_t k = 0; k < cnt; k++)
+        sh.lane[at + k] = (uint8_t)lane;
+    // sh is this wavefront's own: its LDS accesses complete in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t it = lane; it < total; it += 64) {
+        const uint32_t j = sh.lane[it];
+        f(j, (int32_t)it + sh.row[j]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
 
 // ---------------------------------------------------------------------------------- forward
 __device__ __forceinline__ float4 premul(float4 c) { return make_float4(c.x * c.w, c.y * c.w, c.z * c.w, c.w); }
@@ -424,97 +514,104 @@ __device__ __forceinline__ float wave_excl_sum(float x, float carry, uint32_t) {
 __device__ __forceinline__ float deposit(float x) { return rintf(x * VKD_GRID) * (1.0f / VKD_GRID); }
 __device__ __forceinline__ double deposit(double x) { return x; }
 
-// Coverage of every command. One wavefront per tile row of a path, VKD_CT tiles at a time: one lane per
-// edge of the row adds the edge's area deltas to the row's cells in LDS, then every pixel row is
-// prefix-summed (two columns per lane, the sum so far carried on) into cov[c * 256 + pixel]. Each edge is
-// so evaluated once per pixel row it crosses (2.7 on edges of 3 px) and not in all 16 rows of every tile up
-// to the right end of the path, which the carry covers. Bound by the lanes' unequal numbers of rows and
-// pieces. 1024x768 with 3000 paths (1.4 M edges): 406 -> 177 us, 512x512 with 1024: 180 -> 103 us.
-template <typename R, int NW>
-__global__ __launch_bounds__(64 * NW) void k_dcov(const uint32_t *__restrict__ alloc, uint32_t max_units,
-                                                  const RowUnit *__restrict__ units,
-                                                  const DrawTiles *__restrict__ dts,
-                                                  const PathTile *__restrict__ ptl,
-                                                  const uint32_t *__restrict__ cmd_of,
-                                                  const uint32_t *__restrict__ segs,
-                                                  const RV4<R> *__restrict__ edges, R *__restrict__ cov) {
+// Coverage of every command. One workgroup per tile row of a path, VKD_CT tiles at a time: its wavefronts
+// share the row's edges, one lane per edge and pixel row adds the area deltas to the row's cells in LDS, then every
+// pixel row is prefix-summed (two columns per lane, the sum so far carried on) into cov[c * 256 + pixel]. Each
+// edge is so evaluated once per pixel row it crosses (2.7 on edges of 3 px) and not in all 16 rows of every
+// tile up to the right end of the path, which the carry covers. Bound by the chains of instructions per row and
+// piece; with one wavefront per tile row, that of the longest list (a path of 1280 edges within a few tile rows)
+// set the time. 1024x768 with 3000 paths (1.4 M edges): 406 us with all rows of all tiles, 175 with a
+// wavefront, now 121; 512x512 with 1024: 180, 93, now 55; 100x72 with 48: 93, 61, now 22 us.
+template <typename R>
+__global__ __launch_bounds__(256) void k_dcov(const RowUnit *__restrict__ units, const DrawTiles *__restrict__ dts,
+                                              const PathTile *__restrict__ ptl, const uint32_t *__restrict__ cmd_of,
+                                              const uint32_t *__restrict__ segs, const RV4<R> *__restrict__ edges,
+                                              R *__restrict__ cov) {
     constexpr int COLS = VKD_CT * VKD_T, LD = COLS + 2; // one more cell takes the last column's overflow
+    constexpr int RW = VKD_T / 4;                       // pixel rows that a wavefront prefix-sums
     static_assert(COLS == 128, "two columns per lane");
-    __shared__ alignas(16) R s_acc[NW][VKD_T][LD];
+    __shared__ alignas(16) R acc[VKD_T * LD];
+    __shared__ RV4<R> s_edge[4][64];
+    __shared__ RowShare s_rows[4];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    R(*acc)[LD] = s_acc[wv];
-    const uint32_t n_units = min(alloc[1], max_units);
-    for (uint32_t i = lane; i < (uint32_t)(VKD_T * LD); i += 64)
-        acc[0][i] = (R)0;
-    for (uint32_t u = blockIdx.x * NW + wv; u < n_units; u += gridDim.x * NW) {
-        const RowUnit ru = units[u];
-        const DrawTiles dt = dts[ru.draw];
-        const uint32_t pt0 = dt.pt_base + ru.row * dt.bw;
-        const uint32_t off = ptl[pt0].seg_off, n = ptl[pt0].ntouch;
-        if (!n)
-            continue;
-        const int32_t Y0 = (dt.by0 + (int32_t)ru.row) * VKD_T;
-        const R X0 = (R)(dt.bx0 * VKD_T); // x is taken from the path's left tile border: less rounding
-        R carry[VKD_T];
+    RV4<R> *const ed = s_edge[wv];
+    const RowUnit ru = units[blockIdx.x];
+    const DrawTiles dt = dts[ru.draw];
+    const uint32_t pt0 = dt.pt_base + ru.row * dt.bw;
+    const uint32_t off = ptl[pt0].seg_off, n = ptl[pt0].ntouch;
+    if (!n)
+        return;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)(VKD_T * LD); i += 256)
+        acc[i] = (R)0;
+    __syncthreads();
+    const int32_t Y0 = (dt.by0 + (int32_t)ru.row) * VKD_T;
+    const R X0 = (R)(dt.bx0 * VKD_T); // x is taken from the path's left tile border: less rounding
+    const uint32_t share = min((n + 3) / 4, 64u); // edges per wavefront and turn
+    R carry[RW];
 #pragma unroll
-        for (int r = 0; r < VKD_T; r++)
-            carry[r] = (R)0;
-        for (uint32_t c0 = 0; c0 < dt.bw; c0 += VKD_CT) {
-            const uint32_t nt = min((uint32_t)VKD_CT, dt.bw - c0);
-            const R XL = (R)(c0 * VKD_T), XR = XL + (R)(nt * VKD_T);
-            // acc is this wavefront's own: its LDS accesses complete in order
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            for (uint32_t i = lane; i < n; i += 64) {
-                RV4<R> v = edges[segs[off + i]];
+    for (int r = 0; r < RW; r++)
+        carry[r] = (R)0;
+    for (uint32_t c0 = 0; c0 < dt.bw; c0 += VKD_CT) {
+        const uint32_t nt = min((uint32_t)VKD_CT, dt.bw - c0);
+        const R XL = (R)(c0 * VKD_T), XR = XL + (R)(nt * VKD_T);
+        for (uint32_t i0 = wv * share; i0 < n; i0 += 4 * share) {
+            int32_t ra = 0, rb = -1;
+            if (lane < share && i0 + lane < n) {
+                RV4<R> v = edges[segs[off + i0 + lane]];
                 v.x -= X0;
                 v.z -= X0;
-                if ((c0 && fmax(v.x, v.z) < XL) || fmin(v.x, v.z) > XR)
-                    continue; // left of these columns: in the carry
-                const int32_t ra = (int32_t)fmax(floor(fmin(v.y, v.w)) - (R)Y0, (R)0);
-                const int32_t rb = (int32_t)fmin(floor(fmax(v.y, v.w)) - (R)Y0, (R)(VKD_T - 1));
-                for (int32_t r = ra; r <= rb; r++) {
-                    RowPart<R> p;
-                    if (!p.clip(v, (R)(Y0 + r)))
-                        continue;
-                    R *a = acc[r];
-                    R done = deposit(p.dy_left(XL));
-                    if (c0 == 0 && done != (R)0)
-                        atomicAdd(&a[0], done);
-                    const R xa0 = fmax(p.xl, XL), xb0 = fmin(p.xr, XR);
-                    if (!(xa0 <= xb0))
-                        continue;
-                    const int32_t cl = (int32_t)(floor(xa0) - XL), cr = min((int32_t)(floor(xb0) - XL), (int32_t)(nt * VKD_T) - 1);
-                    for (int32_t c = cl; c <= cr; c++) {
-                        const R cx = XL + (R)c, cn = cx + (R)1;
-                        const R xa = fmax(p.xl, cx), xb = fmin(p.xr, cn);
-                        const R upto = deposit(p.dy_left(cn)), dy = upto - done;
-                        done = upto;
-                        const R right = deposit(dy * ((R)0.5 * (xa + xb) - cx));
-                        atomicAdd(&a[c], dy - right);
-                        atomicAdd(&a[c + 1], right);
-                    }
+                ed[lane] = v;
+                // left of these columns: in the carry
+                if (!((c0 && fmax(v.x, v.z) < XL) || fmin(v.x, v.z) > XR)) {
+                    ra = (int32_t)fmin(fmax(floor(fmin(v.y, v.w)) - (R)Y0, (R)0), (R)VKD_T);
+                    rb = (int32_t)fmax(fmin(floor(fmax(v.y, v.w)) - (R)Y0, (R)(VKD_T - 1)), (R)-1);
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const uint32_t tl = lane / (64 / VKD_CT); // this lane's tile
-            const uint32_t cmd = tl < nt ? cmd_of[pt0 + c0 + tl] : VKD_NO_CMD;
-            R *out = cov + (size_t)cmd * 256 + 2 * (lane & (64 / VKD_CT - 1));
-#pragma unroll
-            for (int r = 0; r < VKD_T; r++) {
-                RV2<R> *cell = (RV2<R> *)&acc[r][2 * lane];
-                const RV2<R> v = *cell;
-                const R over = acc[r][COLS];
-                *cell = RV2<R>{(R)0, (R)0};
-                RV2<R> o;
-                o.x = wave_excl_sum(v.x + v.y, carry[r], lane) + v.x;
-                o.y = o.x + v.y;
-                if (cmd != VKD_NO_CMD)
-                    *(RV2<R> *)(out + r * VKD_T) = o;
-                carry[r] = __shfl(o.y, 63) + over;
-            }
-            if (lane < VKD_T)
-                acc[lane][COLS] = (R)0;
+            share_rows(s_rows[wv], lane, ra, (uint32_t)max(rb - ra + 1, 0), [&](uint32_t j, int32_t r) {
+                RowPart<R> p;
+                if (!p.clip(ed[j], (R)(Y0 + r)))
+                    return;
+                R *a = acc + r * LD;
+                R done = deposit(p.dy_left(XL));
+                if (c0 == 0 && done != (R)0)
+                    atomicAdd(&a[0], done);
+                const R xa0 = fmax(p.xl, XL), xb0 = fmin(p.xr, XR);
+                if (!(xa0 <= xb0))
+                    return;
+                const int32_t cl = (int32_t)(floor(xa0) - XL);
+                const int32_t cr = min((int32_t)(floor(xb0) - XL), (int32_t)(nt * VKD_T) - 1);
+                for (int32_t c = cl; c <= cr; c++) {
+                    const R cx = XL + (R)c, cn = cx + (R)1;
+                    const R xa = fmax(p.xl, cx), xb = fmin(p.xr, cn);
+                    const R upto = deposit(p.dy_left(cn)), dy = upto - done;
+                    done = upto;
+                    const R right = deposit(dy * ((R)0.5 * (xa + xb) - cx));
+                    atomicAdd(&a[c], dy - right);
+                    atomicAdd(&a[c + 1], right);
+                }
+            });
         }
+        __syncthreads();
+        const uint32_t tl = lane / (64 / VKD_CT); // this lane's tile
+        const uint32_t cmd = tl < nt ? cmd_of[pt0 + c0 + tl] : VKD_NO_CMD;
+        R *out = cov + (size_t)cmd * 256 + 2 * (lane & (64 / VKD_CT - 1));
+#pragma unroll
+        for (int q = 0; q < RW; q++) {
+            const int r = (int)wv * RW + q;
+            RV2<R> *cell = (RV2<R> *)&acc[r * LD + 2 * lane];
+            const RV2<R> v = *cell;
+            const R over = acc[r * LD + COLS];
+            *cell = RV2<R>{(R)0, (R)0};
+            RV2<R> o;
+            o.x = wave_excl_sum(v.x + v.y, carry[q], lane) + v.x;
+            o.y = o.x + v.y;
+            if (cmd != VKD_NO_CMD)
+                *(RV2<R> *)(out + r * VKD_T) = o;
+            carry[q] = __shfl(o.y, 63) + over;
+        }
+        if (lane < RW)
+            acc[(wv * RW + lane) * LD + COLS] = (R)0;
+        __syncthreads();
     }
 }
 
@@ -549,35 +646,44 @@ __global__ __launch_bounds__(256) void k_dcomp(uint32_t W, uint32_t H, uint32_t 
 }
 
 // --------------------------------------------------------------------------------- backward
-// sums each of v[0..15] over the 64 lanes of the wavefront with 15 + 2 shuffles; lane l returns
-// the total of value index l >> 2
-__device__ __forceinline__ float wave_multi_sum16(float (&v)[16], uint32_t lane) {
+// sums each of v[0..15] over the 64 lanes of the wavefront; lane l returns the total of value l >> 2. Two
+// values take part in one exchange of halves (then of rows) and one addition each; within rows both are
+// summed by moves in the adders' operands and a lane keeps the one it is to end up with.
+__device__ __forceinline__ float wave_multi_sum16(const float (&v)[16], uint32_t lane) {
+    auto swapped = [](auto r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+    float a[8], b[4], c[2];
 #pragma unroll
-    for (int step = 0; step < 4; step++) {
-        const int o = 32 >> step;   // 32, 16, 8, 4
-        const int half = 8 >> step; // values kept after this step
-        const bool hi = (lane & (uint32_t)o) != 0;
+    for (int i = 0; i < 8; i++)
+        a[i] = swapped(__builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false));
 #pragma unroll
-        for (int i = 0; i < half; i++) {
-            float send = hi ? v[i] : v[i + half];
-            float keep = hi ? v[i + half] : v[i];
-            v[i] = keep + __shfl_xor(send, o);
-        }
+    for (int i = 0; i < 4; i++)
+        b[i] = swapped(__builtin_amdgcn_permlane16_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 4]), false, false));
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float x = b[i] + lane_move<0x128, 0xf>(0.f, b[i]); // row_ror:8
+        const float y = b[i + 2] + lane_move<0x128, 0xf>(0.f, b[i + 2]);
+        c[i] = (lane & 8u) ? y : x;
     }
-    const float x = v[0] + __shfl_xor(v[0], 2);
-    return x + __shfl_xor(x, 1);
+    const float x = c[0] + lane_move<0x141, 0xf>(0.f, c[0]); // row_half_mirror
+    const float y = c[1] + lane_move<0x141, 0xf>(0.f, c[1]);
+    float d = (lane & 4u) ? y : x;
+    d += lane_move<0x4E, 0xf>(0.f, d); // quad_perm [2, 3, 0, 1]
+    d += lane_move<0xB1, 0xf>(0.f, d); // quad_perm [1, 0, 3, 2]
+    return d;
 }
 
 // Compositing backwards: one workgroup per tile, one thread per pixel. dL/dA of every (command, pixel)
-// goes to g_cov, in the layout of cov, for k_dedge_grad.
-__global__ __launch_bounds__(256, 4) void k_dback(uint32_t W, uint32_t H, uint32_t tilesW, uint32_t nch,
+// goes to g_cov, in the layout of cov, for k_dedge_grad. Moves 270 MB on 1024x768 with 3000 paths (54 us at
+// what a copy reaches) in 64 us; with the sums' values chosen by indexing, which compiled into chains of
+// compares over the whole array, it was bound by 280 instructions per command and pixel: 181 us.
+__global__ __launch_bounds__(256) void k_dback(uint32_t W, uint32_t H, uint32_t tilesW, uint32_t nch,
                                                const uint32_t *__restrict__ tile_off, const Cmd *__restrict__ cmds,
                                                const float4 *__restrict__ rgba,
                                                const float4 *__restrict__ grad_img, const float4 *__restrict__ ckpt,
                                                const uint32_t *__restrict__ batch_off, const float *__restrict__ cov,
                                                float *__restrict__ g_cov, double *__restrict__ g_col,
                                                const uint32_t *__restrict__ tile_order) {
-    __shared__ float s_red[4][32];
+    __shared__ float s_red2[2][4][32]; // by turns: one barrier a batch
     const uint32_t t = tile_order[blockIdx.x], tid = threadIdx.x, lane = tid & 63;
     const uint32_t c0 = tile_off[(size_t)t * nch], c1 = tile_off[(size_t)(t + 1) * nch];
     if (c0 == c1)
@@ -590,6 +696,7 @@ __global__ __launch_bounds__(256, 4) void k_dback(uint32_t W, uint32_t H, uint32
     for (uint32_t bb = nbatch; bb-- > 0;) {
         const uint32_t base = c0 + bb * VKD_B;
         const uint32_t nb = min((uint32_t)VKD_B, c1 - base);
+        float(*s_red)[32] = s_red2[bb & 1];
         uint32_t c_draw[VKD_B];
 #pragma unroll
         for (uint32_t j = 0; j < VKD_B; j++)
@@ -611,95 +718,113 @@ __global__ __launch_bounds__(256, 4) void k_dback(uint32_t W, uint32_t H, uint32
                 st[j + 1] = st[j];
             }
         }
-        float gc[16]; // colour gradients of four commands, summed over the tile
+        auto back4 = [&](auto first) __attribute__((always_inline)) { // four commands, backwards
+            constexpr int J0 = decltype(first)::value;
+            float gc[16]; // their colour gradients
 #pragma unroll
-        for (int jj = VKD_B - 1; jj >= 0; jj--) {
-            const uint32_t j = (uint32_t)jj;
-            if ((j & 3u) == 3u) {
-#pragma unroll
-                for (int q = 0; q < 16; q++)
-                    gc[q] = 0.f;
-            }
-            if (j < nb) {
+            for (int i = 3; i >= 0; i--) {
+                const int j = J0 + i;
                 const float A = Av[j];
                 const float k = fminf(1.0f, fabsf(A));
                 const float fp = fabsf(A) < 1.0f ? (A > 0.f ? 1.f : (A < 0.f ? -1.f : 0.f)) : 0.f;
                 const float4 c = premul(rgba[c_draw[j]]);
                 const float4 s = st[j];
-                float dk = 0.f, gs = 0.f;
-                if (valid) {
-                    dk = g.x * (c.x - c.w * s.x) + g.y * (c.y - c.w * s.y) + g.z * (c.z - c.w * s.z) + g.w * (c.w - c.w * s.w);
-                    gs = g.x * s.x + g.y * s.y + g.z * s.z + g.w * s.w;
-                    gc[4 * (j & 3u) + 0] = g.x * k;
-                    gc[4 * (j & 3u) + 1] = g.y * k;
-                    gc[4 * (j & 3u) + 2] = g.z * k;
-                    gc[4 * (j & 3u) + 3] = g.w * k - gs * k;
+                const float dk =
+                    g.x * (c.x - c.w * s.x) + g.y * (c.y - c.w * s.y) + g.z * (c.z - c.w * s.z) + g.w * (c.w - c.w * s.w);
+                const float gs = g.x * s.x + g.y * s.y + g.z * s.z + g.w * s.w;
+                const bool on = valid && j < (int)nb;
+                gc[4 * i + 0] = on ? g.x * k : 0.f;
+                gc[4 * i + 1] = on ? g.y * k : 0.f;
+                gc[4 * i + 2] = on ? g.z * k : 0.f;
+                gc[4 * i + 3] = on ? g.w * k - gs * k : 0.f;
+                if (j < (int)nb) {
+                    g_cov[(size_t)(base + j) * 256 + tid] = valid ? dk * fp : 0.f;
+                    const float ia = 1.0f - c.w * k;
+                    g = make_float4(g.x * ia, g.y * ia, g.z * ia, g.w * ia);
                 }
-                g_cov[(size_t)(base + j) * 256 + tid] = valid ? dk * fp : 0.f;
-                const float ia = 1.0f - c.w * k;
-                g = make_float4(g.x * ia, g.y * ia, g.z * ia, g.w * ia);
             }
-            if ((j & 3u) == 0u) {
-                const float tot = wave_multi_sum16(gc, lane);
-                if ((lane & 3u) == 0)
-                    s_red[tid >> 6][4 * j + (lane >> 2)] = tot;
-            }
-        }
+            const float tot = wave_multi_sum16(gc, lane); // summed over the tile's pixels
+            if ((lane & 3u) == 0)
+                s_red[tid >> 6][4 * J0 + (lane >> 2)] = tot;
+        };
+        static_assert(VKD_B == 8, "two fours");
+        back4(std::integral_constant<int, 4>());
+        back4(std::integral_constant<int, 0>());
         __syncthreads();
         if (tid < 4 * nb) { // double: a path's tiles add up in any order
             const double v = ((double)s_red[0][tid] + s_red[1][tid]) + ((double)s_red[2][tid] + s_red[3][tid]);
             if (v != 0.0)
                 unsafeAtomicAdd(&g_col[4 * cmds[base + (tid >> 2)].draw + (tid & 3)], v); // device memory
         }
-        __syncthreads(); // s_red is written again
     }
 }
 
-// Edge-endpoint gradients: one thread per edge integrates dL/dA along its pieces, row by row, over all
-// the tiles that it crosses. Its neighbours are the next edges of the outline, so a wavefront reads few
-// cache lines of g_cov, and the sum is written once. With k_dback 1024x768 with 3000 paths takes 125 + 189 us;
-// both in one kernel per tile, the edges of its commands adding to theirs with atomics, took 734 us.
-__global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_edges, uint32_t n_paths,
+// Gradients of the points and normals that the edges hang on. One wavefront takes the edges of 6 points of
+// a stroke (60) or 60 of a fill; one lane per edge and pixel row integrates dL/dA along the edge's pieces in the
+// row, over all tiles that it crosses, and adds to the edge's two sums in LDS. The edge's endpoint gradients are
+// (-dy, dx) times the sums. Edge layout per path: a fill has edge j = p_j -> p_j+1; a stroke has, per point j, 10
+// edges: the rectangle of segment j (p_j + n_j, p_j+1 + n_j, p_j+1 - n_j, p_j - n_j) and two bevel triangles at
+// vertex j (p_j, then p_j + s n_j-1 and p_j + s n_j in the order of k_dedges; s = 1, -1), in units of the
+// half-width. Per point p the sums go to own[p] (on point p, on the next point) and, for strokes, to own_n[p]
+// (on normal p, on the previous normal, without the half-width). Bound by the loads of g_cov that wait for
+// the tile's command. With k_dg_points 83 us on 1024x768 with 3000 paths; one lane per edge for all its rows, the
+// edges' gradients written (23 MB) and gathered by two kernels, took 125 + 110 us.
+struct GradUnit {
+    uint32_t first_pt, path;
+};
+__host__ __device__ constexpr uint32_t grad_unit_points(bool stroke) { return stroke ? 6u : 60u; }
+__global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const GradUnit *__restrict__ units,
+                                                    const uint32_t *__restrict__ path_first_pt,
                                                     const uint32_t *__restrict__ path_first_edge,
+                                                    const uint32_t *__restrict__ path_stroke,
                                                     const DrawTiles *__restrict__ dts,
                                                     const uint32_t *__restrict__ cmd_of,
                                                     const RV4<float> *__restrict__ edges,
-                                                    const float *__restrict__ g_cov, float4 *__restrict__ g_edge) {
-    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-    if (e >= n_edges)
+                                                    const float2 *__restrict__ nrm,
+                                                    const float *__restrict__ g_cov, float4 *__restrict__ own,
+                                                    float4 *__restrict__ own_n) {
+    __shared__ float4 s_edge[4][64];
+    __shared__ float s_sum[4][64][2];
+    __shared__ RowShare s_rows[4];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, u = blockIdx.x * 4u + wv;
+    if (u >= n_units)
         return;
-    // the path of the wavefront's first edge (the same search on all lanes), then on to this edge's
-    const uint32_t ew = (uint32_t)__builtin_amdgcn_readfirstlane((int)e);
-    uint32_t d = 0, hi = n_paths;
-    while (hi - d > 1) { // last d with path_first_edge[d] <= ew
-        const uint32_t mid = (d + hi) >> 1;
-        if (path_first_edge[mid] <= ew)
-            d = mid;
-        else
-            hi = mid;
-    }
-    while (d + 1 < n_paths && path_first_edge[d + 1] <= e)
-        d++;
+    const GradUnit gu = units[u];
+    const uint32_t d = gu.path, first = path_first_pt[d], end = path_first_pt[d + 1];
+    const bool stroke = path_stroke[d] != 0;
+    const uint32_t per = stroke ? 10u : 1u, np = min(grad_unit_points(stroke), end - gu.first_pt);
     const DrawTiles dt = dts[d];
-    const RV4<float> v = edges[e];
-    float ga = 0.f, gb = 0.f; // scalar factors of (-dy, dx)
-    int32_t r0 = 1, r1 = 0, c0;
-    if (dt.bw && dt.bx0 <= dt.bx1 && dt.by0 <= dt.by1)
-        dbin_range(v, dt, r0, r1, c0);
-    if (r0 <= r1) {
-        const float lo = (float)(dt.bx0 * VKD_T), hiX = (float)((dt.bx1 + 1) * VKD_T);
-        r0 = (int32_t)fmaxf(floorf(fminf(v.y, v.w)), (float)(dt.by0 * VKD_T));
-        r1 = (int32_t)fminf(floorf(fmaxf(v.y, v.w)), (float)(dt.by1 * VKD_T + VKD_T - 1));
-        for (int32_t r = r0; r <= r1; r++) {
+    float4 *ed = s_edge[wv];
+    float(*sum)[2] = s_sum[wv];
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    int32_t r0 = 1, r1 = 0;
+    if (lane < np * per) {
+        const RV4<float> e = edges[path_first_edge[d] + (gu.first_pt - first) * per + lane];
+        v = make_float4(e.x, e.y, e.z, e.w);
+        int32_t c0;
+        if (dt.bw)
+            dbin_range(e, dt, r0, r1, c0);
+        if (r0 <= r1) {
+            r0 = (int32_t)fmaxf(floorf(fminf(v.y, v.w)), (float)(dt.by0 * VKD_T));
+            r1 = (int32_t)fminf(floorf(fmaxf(v.y, v.w)), (float)(dt.by1 * VKD_T + VKD_T - 1));
+        }
+    }
+    ed[lane] = v;
+    sum[lane][0] = sum[lane][1] = 0.f;
+    const float lo = (float)(dt.bx0 * VKD_T), hi = (float)((dt.bx1 + 1) * VKD_T);
+    while (__any(r0 <= r1)) { // up to 16 rows of every edge at a time
+        const uint32_t cnt = (uint32_t)min(max(r1 - r0 + 1, 0), VKD_T);
+        share_rows(s_rows[wv], lane, r0, cnt, [&](uint32_t j, int32_t r) {
+            const float4 q = ed[j];
             RowPart<float> p;
-            if (!p.clip(v, (float)r))
-                continue;
-            const float xa = fmaxf(p.xl, lo), xb = fminf(p.xr, hiX);
+            if (!p.clip(RV4<float>{q.x, q.y, q.z, q.w}, (float)r))
+                return;
+            const float xa = fmaxf(p.xl, lo), xb = fminf(p.xr, hi);
             if (!(xa <= xb))
-                continue;
+                return;
             const uint32_t *co = cmd_of + dt.pt_base + (uint32_t)(r / VKD_T - dt.by0) * dt.bw;
             const int32_t cl = (int32_t)floorf(xa), cr = min((int32_t)floorf(xb), (dt.bx1 + 1) * VKD_T - 1);
-            float from = p.param(xa);
+            float from = p.param(xa), ga = 0.f, gb = 0.f;
             for (int32_t c = cl; c <= cr; c++) {
                 const float to = p.param((float)(c + 1));
                 const uint32_t cmd = co[c / VKD_T - dt.bx0];
@@ -713,72 +838,53 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_edges, uint32_t n
                 ga += Gv * I0;
                 gb += Gv * I1;
             }
-        }
+            if (ga != 0.f || gb != 0.f) {
+                atomicAdd(&sum[j][0], ga);
+                atomicAdd(&sum[j][1], gb);
+            }
+        });
+        r0 += (int32_t)cnt;
     }
-    const float dx = v.z - v.x, dy = v.w - v.y;
-    g_edge[e] = ga != 0.f || gb != 0.f ? make_float4(-dy * ga, dx * ga, -dy * gb, dx * gb) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float ga = sum[lane][0], gb = sum[lane][1], dx = v.z - v.x, dy = v.w - v.y;
+    const bool any = ga != 0.f || gb != 0.f;
+    const float4 ge = any ? make_float4(-dy * ga, dx * ga, -dy * gb, dx * gb) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t p = gu.first_pt + lane;
+    if (!stroke) {
+        if (lane < np)
+            own[p] = ge;
+        return;
+    }
+    ed[lane] = ge;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane >= np)
+        return;
+    const float4 *e = ed + 10 * lane;
+    auto vertex = [&](int before, int after) { // where edge `before` ends and edge `after` begins
+        return f2(e[after].x + e[before].z, e[after].y + e[before].w);
+    };
+    const float2 v0 = vertex(3, 0), v1 = vertex(0, 1), v2 = vertex(1, 2), v3 = vertex(2, 3);
+    float2 self = f2(v0.x + v3.x, v0.y + v3.y), n_self = f2(v0.x + v1.x - v2.x - v3.x, v0.y + v1.y - v2.y - v3.y);
+    float2 n_prev = f2(0.f, 0.f);
+    const float2 n0 = nrm[prev_pt(p, first, end)], n1 = nrm[p];
+    const bool swap = n0.x * n1.y - n0.y * n1.x > 0.f; // as in k_dedges
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const int b = 4 + 3 * s;
+        const float sg = s ? -1.f : 1.f;
+        const float2 t0 = vertex(b + 2, b), t1 = vertex(b, b + 1), t2 = vertex(b + 1, b + 2);
+        self = f2(self.x + t0.x + t1.x + t2.x, self.y + t0.y + t1.y + t2.y);
+        const float2 tp = swap ? t2 : t1, ts = swap ? t1 : t2; // on the previous normal, on this one
+        n_prev = f2(n_prev.x + sg * tp.x, n_prev.y + sg * tp.y);
+        n_self = f2(n_self.x + sg * ts.x, n_self.y + sg * ts.y);
+    }
+    own[p] = make_float4(self.x, self.y, v1.x + v2.x, v1.y + v2.y);
+    own_n[p] = make_float4(n_self.x, n_self.y, n_prev.x, n_prev.y);
 }
 
 // --------------------------------------------------------------------------- chain rule
-// Chain rule from edge endpoints to points, normals and half-widths, as gathers (no atomics).
-// Edge layout per path: a fill has edge j = p_j -> p_j+1; a stroke has, per point j, 10 edges
-// [10j, 10j+10): the rectangle of segment j (points j, j+1, normal j), then the two bevel triangles
-// at vertex j (point j, normals j-1 and j). So the endpoints that use point p or normal p lie in the
-// edges of points p-1 and p (point p) or p and p+1 (normal p).
-__device__ __forceinline__ void endpoint(const DSrc &s, int which, uint32_t &i, uint32_t &k, int &sg) {
-    i = which ? s.ib : s.ia;
-    const uint32_t t = which ? s.kb : s.ka;
-    k = t & 0x3FFFFFFFu;
-    sg = (int)(t >> 30) - 1;
-}
-
-// per stroke point p: g_n[p] and the half-width partial sum of the endpoints using normal p
-__global__ void k_dg_normal_sums(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
-                                 const uint32_t *__restrict__ path_first_pt,
-                                 const uint32_t *__restrict__ path_first_edge, const uint32_t *__restrict__ path_stroke,
-                                 const float *__restrict__ width, const DSrc *__restrict__ src,
-                                 const float4 *__restrict__ g_edge, const float2 *__restrict__ nrm,
-                                 float2 *__restrict__ g_n, float *__restrict__ g_hp) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n_pts)
-        return;
-    const uint32_t path = pt_path[p];
-    if (!path_stroke[path]) {
-        g_n[p] = f2(0.f, 0.f);
-        g_hp[p] = 0.f;
-        return;
-    }
-    const uint32_t first = path_first_pt[path], end = path_first_pt[path + 1];
-    const float h = 0.5f * width[path];
-    float gx = 0.f, gy = 0.f, gh = 0.f;
-    const uint32_t owners[2] = {p, next_pt(p, first, end)};
-    for (int o = 0; o < 2; o++) {
-        const uint32_t e0 = path_first_edge[path] + 10 * (owners[o] - first);
-        for (uint32_t e = e0; e < e0 + 10; e++) {
-            const DSrc sr = src[e];
-            const float4 ge = g_edge[e];
-            for (int w = 0; w < 2; w++) {
-                uint32_t i, k;
-                int sg;
-                endpoint(sr, w, i, k, sg);
-                if (sg == 0 || k != p)
-                    continue;
-                const float vx = w ? ge.z : ge.x, vy = w ? ge.w : ge.y;
-                gx += (float)sg * h * vx;
-                gy += (float)sg * h * vy;
-                gh += (float)sg * (nrm[p].x * vx + nrm[p].y * vy);
-            }
-        }
-    }
-    g_n[p] = f2(gx, gy);
-    g_hp[p] = gh;
-}
-
-// per point p: endpoint gradients using point p, plus, for strokes, the normals' dependence on
-// the segments p-1 -> p and p -> p+1: n = (-d.y, d.x)/|d|, g_d = ((g.y, -g.x) - d (n.g)/|d|)/|d|
-__device__ __forceinline__ float2 seg_grad(const float2 *pts, const float2 *nrm, const float2 *g_n, uint32_t a,
-                                           uint32_t b) {
-    const float2 gn = g_n[a];
+// gradient of segment a -> b's direction d through its normal n = (-d.y, d.x)/|d|:
+// g_d = ((g.y, -g.x) - d (n.g)/|d|)/|d|
+__device__ __forceinline__ float2 seg_grad(const float2 *pts, const float2 *nrm, float2 gn, uint32_t a, uint32_t b) {
     const float dx = pts[b].x - pts[a].x, dy = pts[b].y - pts[a].y;
     const float L = sqrtf(dx * dx + dy * dy);
     if (!(L > 0.f) || (gn.x == 0.f && gn.y == 0.f))
@@ -787,42 +893,30 @@ __device__ __forceinline__ float2 seg_grad(const float2 *pts, const float2 *nrm,
     return f2((gn.y - dx * ng / L) / L, (-gn.x - dy * ng / L) / L);
 }
 
+// per point p: what its own edges and the previous point's give it, plus, for strokes, the normals'
+// dependence on the segments p-1 -> p and p -> p+1, and the half-width's part from normal p
 __global__ void k_dg_points(uint32_t n_pts, const uint32_t *__restrict__ pt_path,
-                            const uint32_t *__restrict__ path_first_pt, const uint32_t *__restrict__ path_first_edge,
-                            const uint32_t *__restrict__ path_stroke, const DSrc *__restrict__ src,
-                            const float4 *__restrict__ g_edge, const float2 *__restrict__ pts,
-                            const float2 *__restrict__ nrm, const float2 *__restrict__ g_n,
-                            float2 *__restrict__ g_pt) {
+                            const uint32_t *__restrict__ path_first_pt, const uint32_t *__restrict__ path_stroke,
+                            const float *__restrict__ width, const float4 *__restrict__ own,
+                            const float4 *__restrict__ own_n, const float2 *__restrict__ pts,
+                            const float2 *__restrict__ nrm, float2 *__restrict__ g_pt, float *__restrict__ g_hp) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n_pts)
         return;
     const uint32_t path = pt_path[p];
     const uint32_t first = path_first_pt[path], end = path_first_pt[path + 1];
     const uint32_t pp = prev_pt(p, first, end), nx = next_pt(p, first, end);
-    const bool stroke = path_stroke[path] != 0;
-    const uint32_t per = stroke ? 10u : 1u;
-    float gx = 0.f, gy = 0.f;
-    const uint32_t owners[2] = {pp, p};
-    for (int o = 0; o < 2; o++) {
-        const uint32_t e0 = path_first_edge[path] + per * (owners[o] - first);
-        for (uint32_t e = e0; e < e0 + per; e++) {
-            const DSrc sr = src[e];
-            const float4 ge = g_edge[e];
-            if (sr.ia == p) {
-                gx += ge.x;
-                gy += ge.y;
-            }
-            if (sr.ib == p) {
-                gx += ge.z;
-                gy += ge.w;
-            }
-        }
-    }
-    if (stroke) {
-        const float2 din = seg_grad(pts, nrm, g_n, pp, p); // segment pp -> p: +g_d at its end p
-        const float2 dout = seg_grad(pts, nrm, g_n, p, nx); // segment p -> nx: -g_d at its start p
+    const float4 o = own[p], op = own[pp];
+    float gx = op.z + o.x, gy = op.w + o.y;
+    if (path_stroke[path]) {
+        const float h = 0.5f * width[path];
+        const float4 a = own_n[pp], b = own_n[p], c = own_n[nx];
+        const float2 sp = f2(a.x + b.z, a.y + b.w), sn = f2(b.x + c.z, b.y + c.w); // sums on normals pp and p
+        const float2 din = seg_grad(pts, nrm, f2(h * sp.x, h * sp.y), pp, p);  // segment pp -> p: +g_d at its end p
+        const float2 dout = seg_grad(pts, nrm, f2(h * sn.x, h * sn.y), p, nx); // p -> nx: -g_d at its start p
         gx += din.x - dout.x;
         gy += din.y - dout.y;
+        g_hp[p] = nrm[p].x * sn.x + nrm[p].y * sn.y;
     }
     g_pt[p] = f2(gx, gy);
 }
@@ -856,22 +950,27 @@ __global__ void k_dg_ctrl(uint32_t n_ctrl, const uint32_t *__restrict__ ctrl_pat
     g_ctrl[ci] = f2(gx, gy);
 }
 
-// per path: colour chain c = (r a, g a, b a, a) and width = 2 h
-__global__ void k_dg_paths(uint32_t n_paths, const float4 *__restrict__ rgba, const double *__restrict__ g_col,
-                           const float *__restrict__ g_hp, const uint32_t *__restrict__ path_first_pt,
-                           const uint32_t *__restrict__ path_stroke, float4 *__restrict__ g_rgba,
-                           float *__restrict__ g_width) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+// one wavefront per path: colour chain c = (r a, g a, b a, a) and width = 2 h
+__global__ __launch_bounds__(256) void k_dg_paths(uint32_t n_paths, const float4 *__restrict__ rgba,
+                                                  const double *__restrict__ g_col, const float *__restrict__ g_hp,
+                                                  const uint32_t *__restrict__ path_first_pt,
+                                                  const uint32_t *__restrict__ path_stroke,
+                                                  float4 *__restrict__ g_rgba, float *__restrict__ g_width) {
+    const uint32_t p = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
     if (p >= n_paths)
+        return;
+    float gh = 0.f;
+    if (path_stroke[p])
+        for (uint32_t k = path_first_pt[p] + lane; k < path_first_pt[p + 1]; k += 64)
+            gh += g_hp[k];
+    for (int o = 32; o > 0; o >>= 1)
+        gh += __shfl_xor(gh, o);
+    if (lane)
         return;
     const float4 c = rgba[p];
     const double g0 = g_col[4 * p], g1 = g_col[4 * p + 1], g2 = g_col[4 * p + 2], g3 = g_col[4 * p + 3];
     g_rgba[p] = make_float4((float)(c.w * g0), (float)(c.w * g1), (float)(c.w * g2),
                             (float)(c.x * g0 + c.y * g1 + c.z * g2 + g3));
-    float gh = 0.f;
-    if (path_stroke[p])
-        for (uint32_t k = path_first_pt[p]; k < path_first_pt[p + 1]; k++)
-            gh += g_hp[k];
     g_width[p] = 0.5f * gh;
 }
 
@@ -883,10 +982,9 @@ __global__ void k_dbatches(uint32_t n_tiles, uint32_t nch, const uint32_t *__res
 }
 
 // the counts that the host sizes its buffers by, written to its memory
-__global__ void k_dcounts(const uint32_t *a, const uint32_t *b, const uint32_t *c, uint32_t *__restrict__ out) {
-    out[0] = a ? *a : 0u;
+__global__ void k_dcounts(const uint32_t *a, const uint32_t *b, uint32_t *__restrict__ out) {
+    out[0] = *a;
     out[1] = b ? *b : 0u;
-    out[2] = c ? *c : 0u;
 }
 
 __global__ void k_dzero(uint32_t *p, size_t n) {
@@ -909,14 +1007,14 @@ struct vkvg_diff_scene_t {
     hipEvent_t ev[4] = {};
     std::string err;
     float ms_fwd = 0, ms_bwd = 0;
-    uint32_t n_segs = 0, n_cmds = 0, n_batches = 0;
+    uint32_t n_segs = 0, n_cmds = 0, n_batches = 0, n_grad_units = 0;
     bool have_ckpt = false;
-    // static topology
-    Buf pt_path, ctrl_path, first_pt, first_ctrl, first_edge, ncubic, stroke, draws, tg;
+    Buf topology; // the static topology, whose parts follow
+    Buf pt_path, ctrl_path, first_pt, first_ctrl, first_edge, ncubic, stroke, draws, tg, grad_units;
     // per call
-    Buf pts, nrm, edges, pts64, nrm64, edges64, src, bbox, dtiles, pt_count, pt_off, ptiles, cmd_of, segs, units,
-        seg_alloc, tile_cnt, tile_off, cmds, nbat, batch_off, ckpt, cov, tile_order, scan_tmp;
-    Buf g_cov, g_edge, g_pt, g_n, g_h, g_col;
+    Buf pts, nrm, edges, pts64, nrm64, edges64, dtiles, alloc, ptiles, cmd_of, segs, units, tile_cnt, tile_off, cmds,
+        nbat, batch_off, ckpt, cov, tile_order, scan_tmp;
+    Buf g_cov, own, own_n, g_pt, g_h, g_col;
     uint32_t *counts = nullptr; // pinned: the counts read back
 };
 
@@ -945,9 +1043,8 @@ template <typename T> T *P(Buf &b) { return (T *)b.p; }
 bool upload(vkvg_diff_scene_t *s, Buf &b, const void *h, size_t bytes) {
     return ensure(s, b, bytes) && ck(s, hipMemcpy(b.p, h, bytes, hipMemcpyHostToDevice), "upload");
 }
-bool read_counts(vkvg_diff_scene_t *s, const uint32_t *a, const uint32_t *b = nullptr, const uint32_t *c = nullptr) {
-    hipLaunchKernelGGL(k_dcounts, dim3(1), dim3(1), 0, s->stream, a, b, c, s->counts);
-    return ck(s, hipGetLastError(), "readback") && ck(s, hipStreamSynchronize(s->stream), "sync");
+bool sync_counts(vkvg_diff_scene_t *s) { // after the kernel that writes s->counts
+    return ck(s, hipGetLastError(), "counts") && ck(s, hipStreamSynchronize(s->stream), "sync");
 }
 bool scan(vkvg_diff_scene_t *s, const uint32_t *in, uint32_t n, uint32_t *out) {
     if (!ensure(s, s->scan_tmp, vkh::scan_temp_words(n) * 4))
@@ -1007,6 +1104,11 @@ VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint32_t n_paths
     s->n_pts = (uint32_t)np;
     s->n_ctrl = (uint32_t)nctl;
     s->n_edges = (uint32_t)ne;
+    std::vector<GradUnit> gu;
+    for (uint32_t i = 0; i < n_paths; i++)
+        for (uint32_t p = first_pt[i]; p < first_pt[i + 1]; p += grad_unit_points(stroke[i] != 0))
+            gu.push_back(GradUnit{p, i});
+    s->n_grad_units = (uint32_t)gu.size();
     // draw records for the shared tile / coarse kernels: one target, kind per path
     std::vector<vkh_draw> dr(n_paths);
     memset(dr.data(), 0, sizeof(vkh_draw) * n_paths);
@@ -1035,20 +1137,43 @@ VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint32_t n_paths
               ck(s, hipHostMalloc((void **)&s->counts, 64, hipHostMallocDefault), "hipHostMalloc");
     for (int k = 0; ok && k < 4; k++)
         ok = ck(s, hipEventCreate(&s->ev[k]), "event");
-    ok = ok && upload(s, s->pt_path, pt_path.data(), 4ull * np) && upload(s, s->ctrl_path, ctrl_path.data(), 4ull * nctl) &&
-         upload(s, s->first_pt, first_pt.data(), 4ull * (n_paths + 1)) &&
-         upload(s, s->first_ctrl, first_ctrl.data(), 4ull * (n_paths + 1)) &&
-         upload(s, s->first_edge, first_edge.data(), 4ull * (n_paths + 1)) &&
-         upload(s, s->ncubic, nc.data(), 4ull * n_paths) && upload(s, s->stroke, stroke.data(), 4ull * n_paths) &&
-         upload(s, s->draws, dr.data(), sizeof(vkh_draw) * n_paths) && upload(s, s->tg, &ti, sizeof(ti)) &&
+    // the topology in one allocation and one copy
+    struct {
+        Buf &b;
+        const void *h;
+        size_t bytes;
+    } parts[] = {{s->pt_path, pt_path.data(), 4ull * np},
+                 {s->ctrl_path, ctrl_path.data(), 4ull * nctl},
+                 {s->first_pt, first_pt.data(), 4ull * (n_paths + 1)},
+                 {s->first_ctrl, first_ctrl.data(), 4ull * (n_paths + 1)},
+                 {s->first_edge, first_edge.data(), 4ull * (n_paths + 1)},
+                 {s->ncubic, nc.data(), 4ull * n_paths},
+                 {s->stroke, stroke.data(), 4ull * n_paths},
+                 {s->draws, dr.data(), sizeof(vkh_draw) * n_paths},
+                 {s->tg, &ti, sizeof(ti)},
+                 {s->grad_units, gu.data(), sizeof(GradUnit) * gu.size()}};
+    size_t bytes = 0;
+    for (auto &x : parts)
+        bytes += (x.bytes + 255) & ~(size_t)255;
+    std::vector<char> blob(bytes);
+    bytes = 0;
+    for (auto &x : parts) {
+        memcpy(blob.data() + bytes, x.h, x.bytes);
+        bytes += (x.bytes + 255) & ~(size_t)255;
+    }
+    ok = ok && upload(s, s->topology, blob.data(), bytes);
+    bytes = 0;
+    for (auto &x : parts) {
+        x.b.p = s->topology.p ? (char *)s->topology.p + bytes : nullptr;
+        bytes += (x.bytes + 255) & ~(size_t)255;
+    }
+    ok = ok &&
          ensure(s, s->pts, 8ull * np) && ensure(s, s->nrm, 8ull * np) && ensure(s, s->edges, 16ull * ne) &&
-         ensure(s, s->src, sizeof(DSrc) * ne) && ensure(s, s->bbox, 16ull * n_paths) &&
-         ensure(s, s->dtiles, sizeof(DrawTiles) * n_paths) && ensure(s, s->pt_count, 4ull * (n_paths + 1)) &&
-         ensure(s, s->pt_off, 4ull * (n_paths + 1)) && ensure(s, s->seg_alloc, 256) && ensure(s, s->segs, 4096) &&
-         ensure(s, s->tile_cnt, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
+         ensure(s, s->dtiles, sizeof(DrawTiles) * n_paths) && ensure(s, s->alloc, sizeof(PathAlloc) * n_paths) &&
+         ensure(s, s->segs, 4096) && ensure(s, s->tile_cnt, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->tile_off, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->nbat, 4ull * (s->n_tiles + 1)) && ensure(s, s->batch_off, 4ull * (s->n_tiles + 1)) &&
-         ensure(s, s->g_edge, 16ull * ne) && ensure(s, s->g_pt, 8ull * np) && ensure(s, s->g_n, 8ull * np) &&
+         ensure(s, s->own, 16ull * np) && ensure(s, s->own_n, 16ull * np) && ensure(s, s->g_pt, 8ull * np) &&
          ensure(s, s->g_h, 4ull * np) && ensure(s, s->g_col, 32ull * n_paths);
     if (!ok) {
         fprintf(stderr, "vkvg_diff_create: %s\n", s->err.c_str());
@@ -1063,11 +1188,10 @@ void vkvg_diff_destroy(VkvgDiffScene s) {
         return;
     if (s->stream)
         (void)hipStreamSynchronize(s->stream);
-    Buf *bufs[] = {&s->pt_path, &s->ctrl_path, &s->first_pt, &s->first_ctrl, &s->first_edge, &s->ncubic, &s->stroke,
-                   &s->draws, &s->tg, &s->pts, &s->nrm, &s->edges, &s->pts64, &s->nrm64, &s->edges64, &s->src, &s->bbox,
-                   &s->dtiles, &s->pt_count, &s->pt_off, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->seg_alloc,
-                   &s->tile_cnt, &s->tile_off, &s->cmds, &s->nbat, &s->batch_off, &s->ckpt, &s->cov, &s->tile_order,
-                   &s->scan_tmp, &s->g_cov, &s->g_edge, &s->g_pt, &s->g_n, &s->g_h, &s->g_col};
+    Buf *bufs[] = {&s->topology, &s->pts, &s->nrm, &s->edges, &s->pts64, &s->nrm64, &s->edges64,
+                   &s->dtiles, &s->alloc, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->tile_cnt, &s->tile_off,
+                   &s->cmds, &s->nbat, &s->batch_off, &s->ckpt, &s->cov, &s->tile_order, &s->scan_tmp, &s->g_cov,
+                   &s->own, &s->own_n, &s->g_pt, &s->g_h, &s->g_col};
     for (Buf *b : bufs)
         if (b->p)
             (void)hipFree(b->p);
@@ -1105,32 +1229,23 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
                        P<uint32_t>(s->first_pt), P<RV2<R>>(pts), P<RV2<R>>(nrm));
     hipLaunchKernelGGL(k_dedges<R>, dim3(blocks(np)), dim3(256), 0, st, np, P<uint32_t>(s->pt_path),
                        P<uint32_t>(s->first_pt), P<uint32_t>(s->first_edge), P<uint32_t>(s->stroke), width,
-                       P<RV2<R>>(pts), P<RV2<R>>(nrm), P<RV4<R>>(edges),
-                       sizeof(R) == sizeof(float) ? P<DSrc>(s->src) : (DSrc *)nullptr);
-    hipLaunchKernelGGL(k_dbbox<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
-                       P<int4>(s->bbox));
-    vkh::launch_draw_tiles(st, P<vkh_draw>(s->draws), nd, P<TargetInfo>(s->tg), P<int4>(s->bbox), VKD_T,
-                           P<DrawTiles>(s->dtiles), P<uint32_t>(s->pt_count));
-    if (!scan(s, P<uint32_t>(s->pt_count), nd, P<uint32_t>(s->pt_off)))
+                       P<RV2<R>>(pts), P<RV2<R>>(nrm), P<RV4<R>>(edges));
+    hipLaunchKernelGGL(k_dpaths<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
+                       (int32_t)s->tilesW, (int32_t)s->tilesH, P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc));
+    hipLaunchKernelGGL(k_dalloc, dim3(1), dim3(1024), 0, st, nd, P<PathAlloc>(s->alloc), P<DrawTiles>(s->dtiles),
+                       s->counts);
+    if (!sync_counts(s))
         return -1;
-    if (!read_counts(s, P<uint32_t>(s->pt_off) + nd))
-        return -1;
-    const uint32_t n_ptiles = s->counts[0];
-    vkh::launch_set_pt_base(st, P<DrawTiles>(s->dtiles), P<uint32_t>(s->pt_off), nd);
-    // a unit per tile row of a path's bbox, which has at least one path tile
+    const uint32_t n_ptiles = s->counts[0], n_units = s->counts[1];
+    s->n_segs = s->counts[2];
     if (!ensure(s, s->ptiles, sizeof(PathTile) * ((size_t)n_ptiles + 1)) ||
         !ensure(s, s->cmd_of, 4ull * ((size_t)n_ptiles + 1)) ||
-        !ensure(s, s->units, sizeof(RowUnit) * ((size_t)n_ptiles + 1)))
+        !ensure(s, s->units, sizeof(RowUnit) * ((size_t)n_units + 1)) ||
+        !ensure(s, s->segs, 4ull * ((size_t)s->n_segs + 1)))
         return -1;
-    auto bin = [&] {
-        zero(s, s->seg_alloc, 2);
-        hipLaunchKernelGGL(k_dbin<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
-                           P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles), P<uint32_t>(s->cmd_of),
-                           P<uint32_t>(s->segs), (uint32_t)std::min<size_t>(s->segs.cap / 4, 0xFFFFFFFFull),
-                           P<RowUnit>(s->units), P<uint32_t>(s->seg_alloc));
-    };
-    bin();
-    // commands and checkpoints depend on the path tiles only, which do not need the lists to fit
+    hipLaunchKernelGGL(k_dbin<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
+                       P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc), P<PathTile>(s->ptiles),
+                       P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RowUnit>(s->units));
     const uint32_t n_tc = s->n_tiles * s->nch;
     const bool keep_ckpt = keep && sizeof(R) == sizeof(float);
     zero(s, s->tile_cnt, n_tc + 1);
@@ -1144,22 +1259,17 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
         if (!scan(s, P<uint32_t>(s->nbat), s->n_tiles, P<uint32_t>(s->batch_off)))
             return -1;
     }
-    if (!read_counts(s, P<uint32_t>(s->seg_alloc), P<uint32_t>(s->tile_off) + n_tc,
-                     keep_ckpt ? P<uint32_t>(s->batch_off) + s->n_tiles : nullptr))
+    hipLaunchKernelGGL(k_dcounts, dim3(1), dim3(1), 0, st, P<uint32_t>(s->tile_off) + n_tc,
+                       keep_ckpt ? P<uint32_t>(s->batch_off) + s->n_tiles : nullptr, s->counts);
+    if (!sync_counts(s))
         return -1;
-    s->n_segs = s->counts[0];
-    s->n_cmds = s->counts[1];
+    s->n_cmds = s->counts[0];
     float4 *ck_ptr = nullptr;
     if (keep_ckpt) {
-        s->n_batches = s->counts[2];
+        s->n_batches = s->counts[1];
         if (!ensure(s, s->ckpt, 16ull * 256 * ((size_t)s->n_batches + 1)))
             return -1;
         ck_ptr = P<float4>(s->ckpt);
-    }
-    if (s->n_segs > s->segs.cap / 4) {
-        if (!ensure(s, s->segs, 4ull * s->n_segs + 4))
-            return -1;
-        bin();
     }
     if (!ensure(s, s->cmds, sizeof(Cmd) * ((size_t)s->n_cmds + 1)) ||
         !ensure(s, s->cov, sizeof(R) * 256 * ((size_t)s->n_cmds + 1)))
@@ -1170,11 +1280,9 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
     if (s->n_cmds) {
         hipLaunchKernelGGL(k_dcmd_of, dim3(blocks(s->n_cmds)), dim3(256), 0, st, s->n_cmds, P<Cmd>(s->cmds),
                            P<uint32_t>(s->cmd_of));
-        constexpr int NW = sizeof(R) == sizeof(float) ? 4 : 2; // wavefronts per workgroup: 33 KB of LDS
-        const unsigned grid = (unsigned)std::min<size_t>(((size_t)n_ptiles + NW - 1) / NW, 4096);
-        hipLaunchKernelGGL((k_dcov<R, NW>), dim3(grid), dim3(64 * NW), 0, st, P<uint32_t>(s->seg_alloc), n_ptiles,
-                           P<RowUnit>(s->units), P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles),
-                           P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RV4<R>>(edges), P<R>(s->cov));
+        hipLaunchKernelGGL(k_dcov<R>, dim3(n_units), dim3(256), 0, st, P<RowUnit>(s->units), P<DrawTiles>(s->dtiles),
+                           P<PathTile>(s->ptiles), P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RV4<R>>(edges),
+                           P<R>(s->cov));
     }
     // tiles heaviest first (commands per tile vary several-fold), for compositing and the backward
     if (!ensure(s, s->tile_order, 4ull * vkh::order_words(s->n_tiles)))
@@ -1230,21 +1338,19 @@ int vkvg_diff_backward(VkvgDiffScene s, const float *ctrl, const float *rgba, co
                        P<uint32_t>(s->tile_off), P<Cmd>(s->cmds), (const float4 *)rgba, (const float4 *)grad_image,
                        P<float4>(s->ckpt), P<uint32_t>(s->batch_off), P<float>(s->cov), P<float>(s->g_cov),
                        P<double>(s->g_col), P<uint32_t>(s->tile_order));
-    hipLaunchKernelGGL(k_dedge_grad, dim3(blocks(s->n_edges)), dim3(256), 0, st, s->n_edges, s->n_paths,
-                       P<uint32_t>(s->first_edge), P<DrawTiles>(s->dtiles), P<uint32_t>(s->cmd_of),
-                       P<RV4<float>>(s->edges), P<float>(s->g_cov), P<float4>(s->g_edge));
-    hipLaunchKernelGGL(k_dg_normal_sums, dim3(blocks(s->n_pts)), dim3(256), 0, st, s->n_pts,
-                       P<uint32_t>(s->pt_path), P<uint32_t>(s->first_pt), P<uint32_t>(s->first_edge),
-                       P<uint32_t>(s->stroke), width, P<DSrc>(s->src), P<float4>(s->g_edge), P<float2>(s->nrm),
-                       P<float2>(s->g_n), P<float>(s->g_h));
+    hipLaunchKernelGGL(k_dedge_grad, dim3((s->n_grad_units + 3) / 4), dim3(256), 0, st, s->n_grad_units,
+                       P<GradUnit>(s->grad_units), P<uint32_t>(s->first_pt), P<uint32_t>(s->first_edge),
+                       P<uint32_t>(s->stroke), P<DrawTiles>(s->dtiles), P<uint32_t>(s->cmd_of),
+                       P<RV4<float>>(s->edges), P<float2>(s->nrm), P<float>(s->g_cov), P<float4>(s->own),
+                       P<float4>(s->own_n));
     hipLaunchKernelGGL(k_dg_points, dim3(blocks(s->n_pts)), dim3(256), 0, st, s->n_pts, P<uint32_t>(s->pt_path),
-                       P<uint32_t>(s->first_pt), P<uint32_t>(s->first_edge), P<uint32_t>(s->stroke),
-                       P<DSrc>(s->src), P<float4>(s->g_edge), P<float2>(s->pts), P<float2>(s->nrm),
-                       P<float2>(s->g_n), P<float2>(s->g_pt));
+                       P<uint32_t>(s->first_pt), P<uint32_t>(s->stroke), width, P<float4>(s->own),
+                       P<float4>(s->own_n), P<float2>(s->pts), P<float2>(s->nrm), P<float2>(s->g_pt),
+                       P<float>(s->g_h));
     hipLaunchKernelGGL(k_dg_ctrl, dim3(blocks(s->n_ctrl)), dim3(256), 0, st, s->n_ctrl, P<uint32_t>(s->ctrl_path),
                        P<uint32_t>(s->first_ctrl), P<uint32_t>(s->first_pt), P<uint32_t>(s->ncubic),
                        P<float2>(s->g_pt), (float2 *)grad_ctrl);
-    hipLaunchKernelGGL(k_dg_paths, dim3(blocks(s->n_paths)), dim3(256), 0, st, s->n_paths, (const float4 *)rgba,
+    hipLaunchKernelGGL(k_dg_paths, dim3((s->n_paths + 3) / 4), dim3(256), 0, st, s->n_paths, (const float4 *)rgba,
                        P<double>(s->g_col), P<float>(s->g_h), P<uint32_t>(s->first_pt), P<uint32_t>(s->stroke),
                        (float4 *)grad_rgba, grad_width);
     if (!ck(s, hipGetLastError(), "backward launch") || !ck(s, hipEventRecord(s->ev[3], st), "event") ||
