@@ -21,8 +21,8 @@ static __device__ __align__(256) uint8_t scratch[VKH_NOALLOC_SCRATCH_BYTES];
 // Exclusive prefix sum over n uint32 values into out[0..n] (out[n] = total): block scans of
 // 1024 values (256 threads x 4), then the block totals added back (summed per block when there
 // are at most 1024 of them, scanned recursively otherwise).
-__global__ __launch_bounds__(256) void k_scan_block(const uint32_t *__restrict__ in, uint32_t n,
-                                                    uint32_t *__restrict__ out, uint32_t *__restrict__ sums) {
+__device__ __forceinline__ void scan_block(const uint32_t *__restrict__ in, uint32_t n, uint32_t *__restrict__ out,
+                                           uint32_t *__restrict__ sums) {
     __shared__ uint32_t wsum[4];
     uint32_t base = blockIdx.x * 1024u + threadIdx.x * 4u;
     uint32_t v[4];
@@ -54,9 +54,13 @@ __global__ __launch_bounds__(256) void k_scan_block(const uint32_t *__restrict__
     if (threadIdx.x == 255 && sums)
         sums[blockIdx.x] = woff + incl;
 }
+__global__ __launch_bounds__(256) void k_scan_block(const uint32_t *__restrict__ in, uint32_t n,
+                                                    uint32_t *__restrict__ out, uint32_t *__restrict__ sums) {
+    scan_block(in, n, out, sums);
+}
 // block b adds the total of blocks 0 .. b-1 (at most 1024 block sums, reduced by the workgroup)
-__global__ __launch_bounds__(256) void k_scan_add_sums(uint32_t *__restrict__ out, uint32_t n,
-                                                       const uint32_t *__restrict__ sums) {
+__device__ __forceinline__ void scan_add_sums(uint32_t *__restrict__ out, uint32_t n,
+                                              const uint32_t *__restrict__ sums) {
     __shared__ uint32_t wsum[4];
     const uint32_t b = blockIdx.x, tid = threadIdx.x;
     uint32_t x = 0;
@@ -79,6 +83,36 @@ __global__ __launch_bounds__(256) void k_scan_add_sums(uint32_t *__restrict__ ou
         if (j <= n)
             out[j] += o;
     }
+}
+__global__ __launch_bounds__(256) void k_scan_add_sums(uint32_t *__restrict__ out, uint32_t n,
+                                                       const uint32_t *__restrict__ sums) {
+    scan_add_sums(out, n, sums);
+}
+// the same for two scans of one length, blockIdx.y saying which
+__global__ __launch_bounds__(256) void k_scan_block2(const uint32_t *__restrict__ in0,
+                                                     const uint32_t *__restrict__ in1, uint32_t n,
+                                                     uint32_t *__restrict__ out0, uint32_t *__restrict__ out1,
+                                                     uint32_t *__restrict__ sums0, uint32_t *__restrict__ sums1) {
+    if (blockIdx.y)
+        scan_block(in1, n, out1, sums1);
+    else
+        scan_block(in0, n, out0, sums0);
+}
+__global__ __launch_bounds__(256) void k_scan_add_sums2(uint32_t *__restrict__ out0, uint32_t *__restrict__ out1,
+                                                        uint32_t n, const uint32_t *__restrict__ sums0,
+                                                        const uint32_t *__restrict__ sums1) {
+    if (blockIdx.y)
+        scan_add_sums(out1, n, sums1);
+    else
+        scan_add_sums(out0, n, sums0);
+}
+// up to four counts into the host's memory
+__global__ void k_totals(const uint32_t *a, const uint32_t *b, const uint32_t *c, const uint32_t *d,
+                         uint32_t *__restrict__ out) {
+    out[0] = a ? *a : 0u;
+    out[1] = b ? *b : 0u;
+    out[2] = c ? *c : 0u;
+    out[3] = d ? *d : 0u;
 }
 __global__ void k_scan_add(uint32_t *__restrict__ out, uint32_t n, const uint32_t *__restrict__ offs) {
     uint32_t i = blockIdx.x * 1024u + threadIdx.x;
@@ -120,6 +154,20 @@ void scan_u32(hipStream_t s, const uint32_t *in, uint32_t n, uint32_t *out, uint
     scan_u32(s, sums, nb, sscan, tmp + 2ull * nb + 1);
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(256), 0, s, out, n, sscan);
 }
+// two scans of one length; tmp holds twice scan_temp_words(n) words
+static void scan_u32_pair(hipStream_t s, const uint32_t *in0, const uint32_t *in1, uint32_t n, uint32_t *out0,
+                          uint32_t *out1, uint32_t *tmp) {
+    const uint32_t nb = (n + 1 + 1023) / 1024;
+    if (nb > 1024) {
+        scan_u32(s, in0, n, out0, tmp);
+        scan_u32(s, in1, n, out1, tmp);
+        return;
+    }
+    uint32_t *sums0 = nb > 1 ? tmp : nullptr, *sums1 = nb > 1 ? tmp + nb : nullptr;
+    hipLaunchKernelGGL(k_scan_block2, dim3(nb, 2), dim3(256), 0, s, in0, in1, n, out0, out1, sums0, sums1);
+    if (nb > 1)
+        hipLaunchKernelGGL(k_scan_add_sums2, dim3(nb, 2), dim3(256), 0, s, out0, out1, n, sums0, sums1);
+}
 } // namespace vkh
 
 namespace {
@@ -141,7 +189,6 @@ struct vkh_engine {
     uint8_t *noalloc_scratch = nullptr; // this device's address of `scratch` (allocation-free readback)
     hipStream_t stream = nullptr;
     hipStream_t own = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     uint32_t tile = 16;
     std::string err;
     vkh_stats stats{};
@@ -170,6 +217,7 @@ struct vkh_engine {
     // chunk) how many of them there are: every tile of the target holds their commands
     std::vector<uint2> h_tileless;
     std::vector<uint32_t> h_tl_table;
+    uint32_t *d_tl_table = nullptr; // of an upload in its blob, of a retile in tl_table
 
     // the uploaded (resident) frame
     bool resident = false;
@@ -241,12 +289,22 @@ static int scan_u32(vkh_engine *eng, const uint32_t *in, uint32_t n, uint32_t *o
     return check(eng, hipGetLastError(), "scan") ? 0 : -1;
 }
 
+static int scan_u32_pair(vkh_engine *eng, const uint32_t *in0, const uint32_t *in1, uint32_t n, uint32_t *out0,
+                         uint32_t *out1, bool cap) {
+    if (!need(eng, cap, eng->scan_tmp, 2 * vkh::scan_temp_words(n) * sizeof(uint32_t)))
+        return -1;
+    vkh::scan_u32_pair(eng->stream, in0, in1, n, out0, out1, P<uint32_t>(eng->scan_tmp));
+    return check(eng, hipGetLastError(), "scan") ? 0 : -1;
+}
+
+// at most four counts: one kernel writes them into pinned memory (a copy each took some 5 us of a frame)
 static int read_totals(vkh_engine *eng, const std::vector<const uint32_t *> &srcs, uint32_t *dst) {
     if (!ensure_host(eng, eng->htot, 64 * sizeof(uint32_t)))
         return -1;
     uint32_t *h = (uint32_t *)eng->htot.p;
-    for (size_t i = 0; i < srcs.size(); i++)
-        CK(hipMemcpyAsync(h + i, srcs[i], 4, hipMemcpyDeviceToHost, eng->stream));
+    auto src = [&](size_t i) { return i < srcs.size() ? srcs[i] : nullptr; };
+    hipLaunchKernelGGL(k_totals, dim3(1), dim3(1), 0, eng->stream, src(0), src(1), src(2), src(3), h);
+    CK(hipGetLastError());
     CK(hipStreamSynchronize(eng->stream));
     for (size_t i = 0; i < srcs.size(); i++)
         dst[i] = h[i];
@@ -277,8 +335,6 @@ vkh_engine *vkvg_hip_engine_create(int device_ordinal) {
         (void)hipGetLastError();
         e->noalloc_scratch = nullptr;
     }
-    (void)hipEventCreate(&e->ev0);
-    (void)hipEventCreate(&e->ev1);
     (void)hipEventCreate(&e->ev_begin);
     (void)hipEventCreate(&e->ev_end);
     for (hipEvent_t &ev : e->ev_stage)
@@ -310,10 +366,6 @@ void vkvg_hip_engine_destroy(vkh_engine *e) {
         (void)hipHostFree(e->hblob.p);
     if (e->htot.p)
         (void)hipHostFree(e->htot.p);
-    if (e->ev0)
-        (void)hipEventDestroy(e->ev0);
-    if (e->ev1)
-        (void)hipEventDestroy(e->ev1);
     if (e->ev_begin)
         (void)hipEventDestroy(e->ev_begin);
     if (e->ev_end)
@@ -443,19 +495,15 @@ void vkvg_hip_get_stats(vkh_engine *e, vkh_stats *out) {
 }
 const char *vkvg_hip_last_error(vkh_engine *e) { return e ? e->err.c_str() : "null engine"; }
 
-// coarse work split for the current tiling: draws per chunk and chunks per bin
-static int set_coarse_chunks(vkh_engine *eng) {
+// coarse work split for the current tiling: draws per chunk and chunks per bin, and the table (per target and
+// chunk) of draws without path tiles
+static void set_coarse_chunks(vkh_engine *eng) {
     eng->coarse_chunk = vkh::coarse_chunk(eng->most_draws, eng->bin_total);
     eng->coarse_nch = (eng->most_draws + eng->coarse_chunk - 1) / eng->coarse_chunk;
     const size_t n = (size_t)std::max<uint32_t>(eng->n_targets, 1u) * eng->coarse_nch;
     eng->h_tl_table.assign(n, 0u);
     for (const uint2 &tl : eng->h_tileless)
         eng->h_tl_table[(size_t)tl.x * eng->coarse_nch + tl.y / eng->coarse_chunk]++;
-    if (!ensure(eng, eng->tl_table, 4 * n))
-        return -1;
-    CK(hipMemcpyAsync(eng->tl_table.p, eng->h_tl_table.data(), 4 * n, hipMemcpyHostToDevice, eng->stream));
-    CK(hipStreamSynchronize(eng->stream));
-    return 0;
 }
 
 int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
@@ -588,7 +636,19 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     size_t o_tg = align256(o_grads + sizeof(vkh_gradient) * f->n_grads);
     size_t o_units = align256(o_tg + sizeof(TargetInfo) * f->n_targets);
     size_t o_srcs = align256(o_units + sizeof(Unit) * n_units);
-    size_t total = align256(o_srcs + sizeof(vkh_surface_source) * f->n_sources) + 256;
+    size_t o_tl = align256(o_srcs + sizeof(vkh_surface_source) * f->n_sources);
+    // what the coarse table depends on
+    eng->n_targets = f->n_targets;
+    eng->bin_total = bin_total;
+    eng->most_draws = 1;
+    for (const TargetInfo &ti : tg)
+        eng->most_draws = std::max(eng->most_draws, ti.draw_end - ti.draw_begin);
+    eng->h_tileless.clear();
+    for (uint32_t i = 0; i < n_draws; i++)
+        if (!kind_has_tiles(f->draws[i].kind))
+            eng->h_tileless.push_back(make_uint2(f->draws[i].target, i - tg[f->draws[i].target].draw_begin));
+    set_coarse_chunks(eng);
+    size_t total = align256(o_tl + sizeof(uint32_t) * eng->h_tl_table.size()) + 256;
     if (!ensure_host(eng, eng->hblob, total) || !ensure(eng, eng->blob, total))
         return -1;
     uint8_t *hb = (uint8_t *)eng->hblob.p;
@@ -622,6 +682,7 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
         memcpy(hb + o_units, units.data(), sizeof(Unit) * n_units);
     if (f->n_sources)
         memcpy(hb + o_srcs, f->sources, sizeof(vkh_surface_source) * f->n_sources);
+    memcpy(hb + o_tl, eng->h_tl_table.data(), sizeof(uint32_t) * eng->h_tl_table.size());
     CK(hipMemcpyAsync((uint8_t *)eng->blob.p + sent, hb + sent, total - sent, hipMemcpyHostToDevice, s));
     eng->o_items = o_items;
     eng->o_sp = o_sp;
@@ -632,30 +693,20 @@ int vkvg_hip_upload(vkh_engine *eng, const vkh_frame *f) {
     eng->o_tg = o_tg;
     eng->o_units = o_units;
     eng->o_srcs = o_srcs;
+    eng->d_tl_table = (uint32_t *)((uint8_t *)eng->blob.p + o_tl);
     eng->n_items = n_items;
     eng->n_sp = n_sp;
     eng->n_draws = n_draws;
     eng->n_styles = f->n_styles;
     eng->n_dashes = f->n_dashes;
     eng->n_grads = f->n_grads;
-    eng->n_targets = f->n_targets;
     eng->n_units = n_units;
     eng->tile_total = tile_total;
-    eng->bin_total = bin_total;
     eng->frame_tile = T;
     eng->h_tg = tg;
     eng->n_cubic_items = n_cubics;
-    eng->most_draws = 1;
-    for (const TargetInfo &ti : tg)
-        eng->most_draws = std::max(eng->most_draws, ti.draw_end - ti.draw_begin);
     eng->frame_ext = any_stencil || any_source;
     eng->frame_sig = any_sig;
-    eng->h_tileless.clear();
-    for (uint32_t i = 0; i < n_draws; i++)
-        if (!kind_has_tiles(f->draws[i].kind))
-            eng->h_tileless.push_back(make_uint2(f->draws[i].target, i - tg[f->draws[i].target].draw_begin));
-    if (set_coarse_chunks(eng))
-        return -1;
     eng->frame_gen++;
     eng->gfail_key = 0;
     eng->resident = true;
@@ -718,7 +769,7 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     // [0] segments, [1] flatten slots, [2] overflow cubics, [3] long dashed pieces, [4] a dash walk
     // stopped at its cap bound
     uint32_t *ctr = P<uint32_t>(eng->counters);
-    vkh::launch_zero_u32(s, ctr + 1, 4);
+    vkh::launch_zero_u32(s, ctr, 5);
     if (n_items) {
         uint32_t *whist = P<uint32_t>(eng->flat_wh), *wcur = whist + n_wh + 1;
         vkh::launch_flat_hist(s, d_items, n_items, whist);
@@ -736,13 +787,29 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                                   P<uint32_t>(eng->flat_ovf));
     if (scan_u32(eng, P<uint32_t>(eng->item_cnt), n_items, P<uint32_t>(eng->item_off), cap))
         return -1;
-    uint32_t tot[8];
-    if (totals(eng, cap, {P<uint32_t>(eng->item_off) + n_items, ctr + 2}, tot, 0))
+    // the subpaths' points and with them the fill edges and stroke steps of every unit follow from the
+    // items' counts alone, so one wait for the counts covers them too
+    size_t un4 = 4ull * (n_units + 1);
+    if (!need(eng, cap, eng->sp_first, 4 * (n_sp + 1)) || !need(eng, cap, eng->sp_count, 4 * (n_sp + 1)) ||
+        !need(eng, cap, eng->fe, un4) || !need(eng, cap, eng->nv, un4) || !need(eng, cap, eng->fe_off, un4) ||
+        !need(eng, cap, eng->nv_off, un4) || !need(eng, cap, eng->u_toff, un4) || !need(eng, cap, eng->u_vbeg, un4) ||
+        !need(eng, cap, eng->u_vend, un4))
         return -1;
+    uint32_t *d_steps = P<uint32_t>(eng->nv), *d_step_off = P<uint32_t>(eng->nv_off);
+    vkh::launch_subpath_ranges(s, d_sp, n_sp, P<uint32_t>(eng->item_off), P<uint32_t>(eng->sp_first),
+                               P<uint32_t>(eng->sp_count));
+    vkh::launch_unit_count(s, d_units, n_units, d_draws, d_sp, P<uint32_t>(eng->sp_count), d_styles,
+                           P<uint32_t>(eng->fe), d_steps);
+    if (scan_u32_pair(eng, P<uint32_t>(eng->fe), d_steps, n_units, P<uint32_t>(eng->fe_off), d_step_off, cap))
+        return -1;
+    uint32_t tot[8];
+    if (totals(eng, cap, {P<uint32_t>(eng->item_off) + n_items, ctr + 2, P<uint32_t>(eng->fe_off) + n_units,
+                          d_step_off + n_units}, tot, 0))
+        return -1;
+    const uint32_t n_fill_edges = tot[2], n_steps = tot[3];
     const uint32_t n_pts = tot[0], n_ovf = tot[1];
     st.points = n_pts;
-    if (!need(eng, cap, eng->pts, 8ull * n_pts + 8) || !need(eng, cap, eng->pflags, n_pts + 8) ||
-        !need(eng, cap, eng->sp_first, 4 * (n_sp + 1)) || !need(eng, cap, eng->sp_count, 4 * (n_sp + 1)))
+    if (!need(eng, cap, eng->pts, 8ull * n_pts + 8) || !need(eng, cap, eng->pflags, n_pts + 8))
         return -1;
     if (split)
         vkh::launch_flatten_split_copy(s, d_items, n_cubics, P<uint32_t>(eng->flat_perm), P<uint32_t>(eng->slot_item),
@@ -756,27 +823,11 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                               P<uint8_t>(eng->pflags));
     vkh::launch_flatten_overflow(s, d_items, P<uint32_t>(eng->flat_ovf), n_ovf, P<uint32_t>(eng->item_off),
                                  P<v2>(eng->pts), P<uint8_t>(eng->pflags));
-    vkh::launch_subpath_ranges(s, d_sp, n_sp, P<uint32_t>(eng->item_off), P<uint32_t>(eng->sp_first),
-                               P<uint32_t>(eng->sp_count));
     CK(hipGetLastError());
 
     if (!cap)
         CK(hipEventRecord(eng->ev_stage[0], s)); // flatten done
-    // ---- per-unit geometry: fill edge counts and stroke work steps
-    size_t un4 = 4ull * (n_units + 1);
-    if (!need(eng, cap, eng->fe, un4) || !need(eng, cap, eng->nv, un4) || !need(eng, cap, eng->fe_off, un4) ||
-        !need(eng, cap, eng->nv_off, un4) || !need(eng, cap, eng->u_toff, un4) || !need(eng, cap, eng->u_vbeg, un4) ||
-        !need(eng, cap, eng->u_vend, un4))
-        return -1;
-    uint32_t *d_steps = P<uint32_t>(eng->nv), *d_step_off = P<uint32_t>(eng->nv_off);
-    vkh::launch_unit_count(s, d_units, n_units, d_draws, d_sp, P<uint32_t>(eng->sp_count), d_styles,
-                           P<uint32_t>(eng->fe), d_steps);
-    if (scan_u32(eng, P<uint32_t>(eng->fe), n_units, P<uint32_t>(eng->fe_off), cap) ||
-        scan_u32(eng, d_steps, n_units, d_step_off, cap))
-        return -1;
-    if (totals(eng, cap, {P<uint32_t>(eng->fe_off) + n_units, d_step_off + n_units}, tot, 2))
-        return -1;
-    const uint32_t n_fill_edges = tot[0], n_steps = tot[1];
+    // ---- stroke geometry
     size_t sn4 = 4ull * (n_steps + 1);
     if (!need(eng, cap, eng->step_nv, sn4) || !need(eng, cap, eng->step_nt, sn4) || !need(eng, cap, eng->sv_off, sn4) ||
         !need(eng, cap, eng->st_off, sn4) || !need(eng, cap, eng->dash_st, 2 * sn4) ||
@@ -786,8 +837,8 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                              P<uint32_t>(eng->sp_count), P<v2>(eng->pts), P<uint8_t>(eng->pflags), d_styles, d_dashes,
                              P<uint32_t>(eng->step_nv), P<uint32_t>(eng->step_nt), nullptr, nullptr, nullptr, nullptr,
                              P<uint2>(eng->dash_st), P<uint4>(eng->dash_list), ctr + 3);
-    if (scan_u32(eng, P<uint32_t>(eng->step_nv), n_steps, P<uint32_t>(eng->sv_off), cap) ||
-        scan_u32(eng, P<uint32_t>(eng->step_nt), n_steps, P<uint32_t>(eng->st_off), cap))
+    if (scan_u32_pair(eng, P<uint32_t>(eng->step_nv), P<uint32_t>(eng->step_nt), n_steps, P<uint32_t>(eng->sv_off),
+                      P<uint32_t>(eng->st_off), cap))
         return -1;
     if (totals(eng, cap, {P<uint32_t>(eng->sv_off) + n_steps, P<uint32_t>(eng->st_off) + n_steps, ctr + 4}, tot, 4))
         return -1;
@@ -850,12 +901,16 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                           d_gprep);
     if (scan_u32(eng, P<uint32_t>(eng->pt_count), n_draws, P<uint32_t>(eng->pt_off), cap))
         return -1;
-    if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws}, tot, 7))
-        return -1;
-    const uint32_t n_ptiles = tot[0];
-    st.path_tiles = n_ptiles;
-    vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws);
-    if (!need(eng, cap, eng->ptiles, sizeof(PathTile) * (size_t)n_ptiles + 16) || !need(eng, cap, eng->segs, 4096))
+    // The path tiles, the binned segments and the commands are counted in one go with the buffers as they
+    // are: draws whose path tiles do not fit are left out of the binning and segments that do not fit are
+    // not written, and where that happened the buffers grow and the pass runs again. A wait for each of
+    // the three counts took some 20 us. The first frame of an engine has no buffers to try and waits for its path tiles.
+    if (!eng->ptiles.p) {
+        if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws}, tot, 7) ||
+            !need(eng, cap, eng->ptiles, sizeof(PathTile) * (size_t)tot[0] + 16))
+            return -1;
+    }
+    if (!need(eng, cap, eng->ptiles, sizeof(PathTile) + 16) || !need(eng, cap, eng->segs, 4096))
         return -1;
     if (!cap)
         CK(hipEventRecord(eng->ev_stage[2], s)); // tile setup done
@@ -876,37 +931,44 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     const uint32_t n_tc = (uint32_t)n_tc64;
     if (!need(eng, cap, eng->tile_cnt, 4ull * (n_tc + 1)) || !need(eng, cap, eng->tile_off, 4ull * (n_tc + 1)))
         return -1;
-    for (int pass = 0; pass < 2; pass++) {
+    uint32_t n_ptiles = 0;
+    for (int pass = 0;; pass++) {
         const uint32_t seg_cap = (uint32_t)std::min<size_t>(eng->segs.cap / sizeof(Edge), 0xFFFFFFFFull);
-        vkh::launch_zero_u32(s, P<uint32_t>(eng->counters), 1);
-        vkh::launch_tile_cnt_init(s, d_tg, n_targets, nch, P<uint32_t>(eng->tl_table), P<uint32_t>(eng->tile_cnt), n_tc);
+        const uint32_t pt_cap = (uint32_t)std::min<size_t>(eng->ptiles.cap / sizeof(PathTile), 0xFFFFFFFFull);
+        if (pass) {
+            vkh::launch_zero_u32(s, ctr, 1);
+            vkh::launch_draw_tiles(s, d_draws, n_draws, d_tg, P<int4>(eng->bbox), T, P<DrawTiles>(eng->dtiles),
+                                   P<uint32_t>(eng->pt_count)); // those left out are back
+        }
+        vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws, pt_cap);
+        vkh::launch_tile_cnt_init(s, d_tg, n_targets, nch, eng->d_tl_table, P<uint32_t>(eng->tile_cnt), n_tc);
         vkh::launch_bin_draws(s, P<Edge>(eng->edges), P<uint2>(eng->erange),
                               P<DrawTiles>(eng->dtiles), n_draws, T, P<PathTile>(eng->ptiles), P<Edge>(eng->segs),
-                              seg_cap, P<uint32_t>(eng->counters), P<uint32_t>(eng->draw_order), d_draws, d_tg, nch,
+                              seg_cap, ctr, P<uint32_t>(eng->draw_order), d_draws, d_tg, nch,
                               eng->coarse_chunk, P<uint32_t>(eng->tile_cnt), P<DrawPrep>(eng->dprep));
         CK(hipGetLastError());
-        if (totals(eng, cap, {P<uint32_t>(eng->counters)}, tot, 8))
+        if (!cap)
+            CK(hipEventRecord(eng->ev_stage[3], s)); // binning done
+        // ---- coarse: ordered command list per tile (the counts came from binning)
+        if (scan_u32(eng, P<uint32_t>(eng->tile_cnt), n_tc, P<uint32_t>(eng->tile_off), cap))
             return -1;
-        n_segs = tot[0];
-        if (n_segs <= seg_cap)
+        if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws, ctr, P<uint32_t>(eng->tile_off) + n_tc}, tot, 7))
+            return -1;
+        n_ptiles = tot[0];
+        n_segs = tot[1]; // of the draws that were not left out
+        if (n_ptiles <= pt_cap && n_segs <= seg_cap)
             break;
-        if (pass == 1) {
+        if (pass == 2) { // one pass for the path tiles, one for the segments
             eng->err = "segment buffer overflow after resize";
             return -1;
         }
-        if (!need(eng, cap, eng->segs, sizeof(Edge) * (size_t)n_segs + sizeof(Edge)))
+        if (!need(eng, cap, eng->ptiles, sizeof(PathTile) * (size_t)n_ptiles + 16) ||
+            !need(eng, cap, eng->segs, sizeof(Edge) * (size_t)n_segs + sizeof(Edge)))
             return -1;
     }
+    st.path_tiles = n_ptiles;
     st.segments = n_segs;
-
-    if (!cap)
-        CK(hipEventRecord(eng->ev_stage[3], s)); // binning done
-    // ---- coarse: ordered command list per tile (the counts came from binning)
-    if (scan_u32(eng, P<uint32_t>(eng->tile_cnt), n_tc, P<uint32_t>(eng->tile_off), cap))
-        return -1;
-    if (totals(eng, cap, {P<uint32_t>(eng->tile_off) + n_tc}, tot, 9))
-        return -1;
-    const uint32_t n_cmds = tot[0];
+    const uint32_t n_cmds = tot[2];
     st.commands = n_cmds;
     st.tiles = tile_total;
     if (!need(eng, cap, eng->cmds, sizeof(Cmd) * (size_t)n_cmds + 16))
@@ -921,8 +983,6 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     // ---- fine: coverage + compositing
     if (!cap)
         CK(hipEventRecord(eng->ev_stage[4], s)); // coarse done
-    if (!cap)
-        CK(hipEventRecord(eng->ev0, s));
     vkh::launch_fine(s, eng->frame_ext, eng->frame_sig, T, eng->fine_words, tile_total, d_tg, n_targets, P<DrawPrep>(eng->dprep), d_grec, d_grads, d_gprep,
                      P<PathTile>(eng->ptiles),
                      P<Edge>(eng->segs), nch, P<uint32_t>(eng->tile_off),
@@ -930,13 +990,9 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     CK(hipGetLastError());
     if (cap)
         return 0;
-    CK(hipEventRecord(eng->ev1, s));
     CK(hipEventRecord(eng->ev_end, s));
     CK(hipStreamSynchronize(s));
     float ms = 0;
-    (void)hipEventElapsedTime(&ms, eng->ev0, eng->ev1);
-    st.ms_fine = ms;
-    ms = 0;
     (void)hipEventElapsedTime(&ms, eng->ev_begin, eng->ev_end);
     st.ms_device = ms;
     hipEvent_t marks[7] = {eng->ev_begin, eng->ev_stage[0], eng->ev_stage[1], eng->ev_stage[2],
@@ -946,6 +1002,7 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
         (void)hipEventElapsedTime(&ms, marks[k], marks[k + 1]);
         st.ms_stage[k] = ms;
     }
+    st.ms_fine = st.ms_stage[5];
     st.ms_total = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
     eng->stats = st;
     return 0;
@@ -1059,8 +1116,13 @@ int vkvg_hip_retile(vkh_engine *eng, uint32_t T) {
     eng->tile_total = tile_total;
     eng->bin_total = bin_total;
     eng->frame_tile = T;
-    if (set_coarse_chunks(eng))
+    set_coarse_chunks(eng);
+    const size_t tl_bytes = sizeof(uint32_t) * eng->h_tl_table.size();
+    if (!ensure(eng, eng->tl_table, tl_bytes))
         return -1;
+    CK(hipMemcpyAsync(eng->tl_table.p, eng->h_tl_table.data(), tl_bytes, hipMemcpyHostToDevice, s));
+    CK(hipStreamSynchronize(s));
+    eng->d_tl_table = P<uint32_t>(eng->tl_table);
     eng->frame_gen++;
     eng->gfail_key = 0;
     return 0;

@@ -79,10 +79,18 @@ __global__ void k_draw_tiles(const vkh_draw *__restrict__ draws, uint32_t n, con
     dt[i] = o;
 }
 
-__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
+// first path tile of every draw; one whose path tiles are not all below pt_cap loses its tiles
+__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t pt_cap) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        dt[i].pt_base = pt_off[i];
+    if (i >= n)
+        return;
+    const uint32_t a = pt_off[i], b = pt_off[i + 1];
+    dt[i].pt_base = a;
+    if (a != b && b > pt_cap) {
+        dt[i].bx0 = dt[i].by0 = 0;
+        dt[i].bx1 = dt[i].by1 = -1;
+        dt[i].bw = 0;
+    }
 }
 
 // ----------------------------------------------------------------------------------- edge binning
@@ -515,6 +523,54 @@ __global__ __launch_bounds__(256) void k_work_order(uint32_t n, W weight, uint32
     __syncthreads();
     if (i < n)
         order[h[b] + rank] = i;
+}
+
+// up to VKH_ORDER_ONE items by one workgroup: one launch of 5 us where the three passes and the clearing of
+// the buckets take four of 4 to 5 each; beyond, that workgroup takes as long as they do
+#define VKH_ORDER_ONE 8192u
+template <class W>
+__global__ __launch_bounds__(1024) void k_work_order_one(uint32_t n, W weight, uint32_t *__restrict__ order) {
+    __shared__ uint32_t h[VKH_ORDER_BUCKETS];
+    __shared__ uint32_t s_wave[4];
+    constexpr uint32_t K = VKH_ORDER_ONE / 1024u;
+    const uint32_t tid = threadIdx.x;
+    if (tid < VKH_ORDER_BUCKETS)
+        h[tid] = 0u;
+    __syncthreads();
+    uint32_t b[K], rank[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+        const uint32_t i = k * 1024u + tid;
+        b[k] = i < n ? order_bucket(weight(i)) : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++)
+        rank[k] = k * 1024u + tid < n ? atomicAdd(&h[b[k]], 1u) : 0u;
+    __syncthreads();
+    uint32_t v = 0, x = 0;
+    if (tid < VKH_ORDER_BUCKETS) { // exclusive scan of the bucket sizes
+        v = x = h[tid];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if ((int)(tid & 63u) >= o)
+                x += y;
+        }
+        if ((tid & 63u) == 63u)
+            s_wave[tid >> 6] = x;
+    }
+    __syncthreads();
+    if (tid < VKH_ORDER_BUCKETS) {
+        uint32_t before = 0;
+        for (uint32_t k = 0; k < tid >> 6; k++)
+            before += s_wave[k];
+        h[tid] = before + x - v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++)
+        if (k * 1024u + tid < n)
+            order[h[b[k]] + rank[k]] = k * 1024u + tid;
 }
 
 // exclusive scan of the bucket sizes into bucket starts (one workgroup)
@@ -1263,9 +1319,9 @@ void launch_draw_tiles(hipStream_t s, const vkh_draw *draws, uint32_t n, const T
         hipLaunchKernelGGL(k_draw_tiles, dim3((n + 255) / 256), dim3(256), 0, s, draws, n, tg, bbox, tile, dt,
                            pt_count);
 }
-void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
+void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t pt_cap) {
     if (n)
-        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n);
+        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n, pt_cap);
 }
 void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n) {
     if (n)
@@ -1355,6 +1411,10 @@ static void launch_order(hipStream_t s, uint32_t n, W weight, uint32_t *work) {
     if (!n)
         return;
     uint32_t *bucket = work + n, *order = work;
+    if (n <= VKH_ORDER_ONE) {
+        hipLaunchKernelGGL((k_work_order_one<W>), dim3(1), dim3(1024), 0, s, n, weight, order);
+        return;
+    }
     const unsigned g = (n + 255u) / 256u;
     launch_zero_u32(s, bucket, VKH_ORDER_BUCKETS);
     hipLaunchKernelGGL((k_work_order<false, W>), dim3(g), dim3(256), 0, s, n, weight, bucket, order);
