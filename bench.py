@@ -388,7 +388,7 @@ def main() -> int:
         "tuned": tune["best"] if tune else {"tile": st["tile_size"], "fine_words": st["fine_words"]},
         "stages_ms": stage,
         "counts": {k: st[k] for k in ("points", "stroke_triangles", "edges", "path_tiles", "segments", "commands")},
-        "roofline": {"kernel": f"k_fine<{st['tile_size']},{st['fine_words']},false>", "bound": "hbm",
+        "roofline": {"kernel": f"k_fine (tile {st['tile_size']}, {st['fine_words']} words)", "bound": "hbm",
                      "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "algorithmic_bytes_per_launch": fine_bytes, "avg_launch_ms": fine_ms,

@@ -912,13 +912,14 @@ template <int T> __device__ __forceinline__ int32_t tile_row_prefix(int32_t x, c
 // of the tile's sample rows into per-command LDS row deltas, walking only the rows the edge spans;
 // then every pixel applies the commands in order: its winding is the prefix of its row's deltas,
 // taken across the lanes that hold the row, and the command's record is read as wave-uniform values.
-// Bound by vector issue (93 % of it on the 1920x1080 stroke scene, 9.8 M commands: 1.25 G wave VALU
-// instructions). Two pixels per thread share what a command costs once per wave (its record's LDS
+// Bound by vector issue (85 % of it on the 1920x1080 stroke scene, 9.8 M commands: 1.21 G wave VALU
+// instructions in 2.33 ms). Two pixels per thread share what a command costs once per wave (its record's LDS
 // reads, decode, branches); pixels stay unpacked in 16-bit lanes between blends; the row prefix is four
 // DPP additions instead of a pass of 16-way conflicting LDS reads and writes per row; signatures are
 // compiled out where no target keeps them. One pixel per thread with the row pass: 3.11 ms there and
-// 1.82 ms on the 4096x4096 dense scene (4.0 M commands); this form 2.29 and 1.55 ms (four pixels per
-// thread: 3.01 and 1.89 ms, at 10 KB of LDS per wavefront too few wavefronts are resident).
+// 1.82 ms on the 4096x4096 dense scene (4.0 M commands); this form 2.29 and 1.55 ms (1.40 since gradients
+// are solid over tiles where they have one colour; four pixels per thread: 3.01 and 1.89 ms, at 10 KB of LDS
+// per wavefront too few wavefronts are resident).
 // EXT: the frame has surface sources or targets with a stencil plane (the plain variant compiles
 // neither). With a stencil plane each pixel also carries its stencil word
 // (loaded from the plane or zero, stored back at the end): draws blend only where CLIP is 0, clear
