@@ -813,15 +813,13 @@ __device__ __forceinline__ uint32_t dash_arc_count(float a, float a1, bool start
 #define VKH_DASH_WAVE_BIT 0x80000000u
 // Caps from which a piece is given a wavefront: a wavefront's set-up costs about as much as a thread's
 // work on some 16 caps when the pieces fill the chip; with few pieces only the longest chain counts.
-#ifndef VKH_DASH_WAVE_MIN
 #define VKH_DASH_WAVE_MIN 16
-#endif
 #define VKH_DASH_WAVE_MIN_FEW 4
 #define VKH_DASH_FEW 16384 // stroke steps up to which a frame counts as having few pieces
 static_assert(VKH_DASH_WAVE_MIN_FEW <= VKH_DASH_WAVE_MIN, "the caps of a thread's piece fit its row of offsets");
 
-// A piece of fewer than VKH_DASH_WAVE_MIN caps emitted by one thread: the dash offsets of its caps go to the thread's row offs (stride lanes apart), then every arc angle is
-// evaluated once and written for all caps.
+// A piece of fewer than VKH_DASH_WAVE_MIN caps emitted by one thread: the dash offsets of its caps go to the
+// thread's row offs (stride lanes apart), then every arc angle is evaluated once and written for all caps.
 __device__ void dash_piece_emit(const StrokeCtx &c, bool closed, uint32_t k, DashState dc, EmitSink s, float *offs,
                                 uint32_t stride) {
     uint32_t iL, cp, iR;
@@ -1062,11 +1060,14 @@ __global__ void k_dash_walk(const Unit *__restrict__ units, uint32_t n_units, co
 // sines and cosines are evaluated once per piece (one lane per vertex, the angle by the same additions
 // as the loop) and kept in LDS; then the lanes write the caps' vertices and triangles in order, each its
 // own, so that the stores are contiguous (a start cap refers to the next cap's first two vertices, which
-// lie where the sequential emission puts them). The piece's totals come from dash_piece_count; what its
-// caps leave of them is the join's.
-// 1920x1080 strokes, a quarter of them dashed: a lane per cap that evaluated its own arc, and threads
-// doing so for pieces below 64 caps, took 830 us (threads) + 457 us (wavefronts); now 55 + 235 us.
-#define VKH_DASH_ARC 128 // arc vertices kept per cap kind; finer arcs are evaluated per vertex
+// lie where the sequential emission puts them). Arcs of more vertices than are kept (a half-width above
+// 320 device pixels) go through LDS in turns, once per 64 caps, the angle carried on from turn to turn.
+// The piece's totals come from dash_piece_count; what its caps leave of them is the join's.
+// Bound by the stores and the chain of additions. 1920x1080 strokes, a quarter of them dashed: 235 us, and 55 us
+// for the shorter pieces in k_stroke_steps (457 and 830 us with an arc evaluated per cap). A line of 66 caps of
+// half-width 1000, 4000 and 16000 px, geometry stage: 0.54, 2.0 and 7.7 ms (3.1, 37.5 and 546 ms where a
+// vertex that is not kept repeats the additions from the arc's first on).
+#define VKH_DASH_ARC 128 // arc vertices kept per cap kind
 __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ units,
                                                      const uint32_t *__restrict__ step_off,
                                                      const vkh_draw *__restrict__ draws,
@@ -1127,33 +1128,57 @@ __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ un
             dash_arc_angle(C.n, false, a1e);
             C.ks = dash_arc_count(a0, a1s, true, C.step);
             C.ke = dash_arc_count(a0, a1e, false, C.step);
+        }
+        // n <= VKH_DASH_ARC vertices of the start (w = 0) or end caps' arc into arc[w], from the vertex after
+        // the one of angle a on; the last one's angle
+        auto fill_arc = [&](int w, uint32_t n, float a) {
+            uint32_t at = 0;
+            for (uint32_t i = lane; i < n; i += 64) {
+                for (; at <= i; at++)
+                    a = w ? a - C.step : a + C.step;
+                float sy, cx;
+                d_sincosf(a, &sy, &cx);
+                arc[w][i] = make_float2(cx * C.hw, sy * C.hw);
+            }
+            for (; at < n; at++)
+                a = w ? a - C.step : a + C.step;
+            return a;
+        };
+        const bool turns = max(C.ks, C.ke) > VKH_DASH_ARC; // as many vertices as one turn keeps at a time
+        if (!turns) {
+            fill_arc(0, C.ks, a0);
+            fill_arc(1, C.ke, a0);
+        }
+        // The vertices of m caps of which D.on0 is the first's kind, from vertex v on, cap j at at(j): the
+        // pairs, then the arcs by turns, whose angle goes on from the turn before
+        auto turn_vertices = [&](const DashCaps &D, uint32_t v, uint32_t m, auto at) {
+            for (uint32_t i = lane; i < 2 * m; i += 64) {
+                const bool st = D.start(i >> 1);
+                verts[v + D.nv_before(i >> 1) + (st ? D.ks : 0u) + (i & 1)] = D.side(st, at(i >> 1), (i & 1) != 0);
+            }
             for (int w = 0; w < 2; w++) {
-                const uint32_t n = min(w ? C.ke : C.ks, (uint32_t)VKH_DASH_ARC);
-                float a = a0; // advanced to vertex i's angle
-                uint32_t at = 0;
-                for (uint32_t i = lane; i < n; i += 64) {
-                    for (; at <= i; at++)
-                        a = w ? a - C.step : a + C.step;
-                    float sy, cx;
-                    d_sincosf(a, &sy, &cx);
-                    arc[w][i] = make_float2(cx * C.hw, sy * C.hw);
+                const bool st = w == 0;
+                const uint32_t n = st ? D.ks : D.ke, j0 = st == D.on0 ? 0u : 1u;
+                const uint32_t n_caps = m > j0 ? (m - j0 + 1) / 2 : 0u;
+                float a = a0;
+                for (uint32_t i0 = 0; n_caps && i0 < n; i0 += VKH_DASH_ARC) {
+                    const uint32_t k = min(n - i0, (uint32_t)VKH_DASH_ARC);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    a = fill_arc(w, k, a);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    for (uint32_t i = lane; i < n_caps * k; i += 64) {
+                        const uint32_t q = i / k, r = i - q * k, j = j0 + 2 * q;
+                        const float2 e = arc[w][r];
+                        verts[v + D.nv_before(j) + (st ? 0u : 2u) + i0 + r] = D.arc(at(j), e.x, e.y);
+                    }
                 }
             }
-        }
-        auto arc_at = [&](bool start, uint32_t i) {
-            if (i < VKH_DASH_ARC)
-                return arc[start ? 0 : 1][i];
-            float a = a0, sy, cx;
-            for (uint32_t t = 0; t <= i; t++)
-                a = start ? a + C.step : a - C.step;
-            d_sincosf(a, &sy, &cx);
-            return make_float2(cx * C.hw, sy * C.hw);
         };
         auto vertex = [&](bool start, v2 p0, uint32_t q) { // vertex q of a cap at p0
             const uint32_t pair = start ? C.ks : 0u;
             if (q == pair || q == pair + 1)
                 return C.side(start, p0, q != pair);
-            const float2 e = arc_at(start, start ? q : q - 2);
+            const float2 e = arc[start ? 0 : 1][start ? q : q - 2];
             return C.arc(p0, e.x, e.y);
         };
         const bool end_on = C.on0 == ((caps & 1) == 0); // dashOn after the last cap
@@ -1180,7 +1205,9 @@ __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ un
             offs[lane] = off;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             const uint32_t n_v = C.nv_before(m), n_t = C.nt_before(m);
-            for (uint32_t i = lane; i < n_v; i += 64) {
+            if (turns)
+                turn_vertices(C, nv, m, [&](uint32_t j) { return C.at(offs[j]); });
+            for (uint32_t i = lane; !turns && i < n_v; i += 64) {
                 const uint32_t pair = i / per, r = i - pair * per;
                 const bool second = r >= first, start = second ? !C.on0 : C.on0;
                 verts[nv + i] = vertex(start, C.at(offs[2 * pair + (second ? 1u : 0u)]), second ? r - first : r);
@@ -1203,7 +1230,12 @@ __global__ __launch_bounds__(256) void k_dash_pieces(const Unit *__restrict__ un
             const uint32_t prev = cur ? cur - 1 : c.dashCount - 1, now = cur ? cur : c.dashCount - 1;
             const float back = fminf(dash(prev) - end, dash(now));
             const v2 p0 = vsub(c.P[iR], vmul(C.n, back));
-            for (uint32_t i = lane; i < C.nv(false); i += 64)
+            if (turns) {
+                DashCaps E = C;
+                E.on0 = false;
+                turn_vertices(E, nv, 1, [&](uint32_t) { return p0; });
+            }
+            for (uint32_t i = lane; !turns && i < C.nv(false); i += 64)
                 verts[nv + i] = vertex(false, p0, i);
             for (uint32_t i = lane; i < C.nt(false); i += 64)
                 C.tri(false, nv, i, tris + 3 * ((size_t)nt + i));
