@@ -1,6 +1,8 @@
 """Frames that outgrow the buffers of the frames before them on the same engine, in path tiles, segments,
 commands or all of them, and frames after them that do not: the pass that counts them runs with the buffers as
-they are, leaves out what does not fit and runs again."""
+they are, counts what does not fit without writing it, and is followed by one more that writes everything."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -54,3 +56,31 @@ def test_work_order_of_one_workgroup_and_of_many(size, n):
         g_rgba, g_sig, _ = render_gpu(dev, sc)
     r = compare(g_rgba, g_sig, rgba, sig)
     assert r["mask_mismatch_px"] == 0 and r["rgba_max_err"] == 0, r
+
+
+def test_outgrown_buffers_cost_one_more_binning_and_no_wait():
+    """Three waits for counts in every frame; the draws of a frame that outgrows path tiles, segments or both are
+    binned twice, those of one that outgrows nothing once."""
+    import vkvg_amd
+    L = vkvg_amd.lib()
+    passes = L.vkh_last_frame_passes
+    passes.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint32)]
+    passes.restype = None
+    out = (ctypes.c_uint32 * 2)()
+    most = np.array([24, 400])  # path tiles and segments that a new engine's buffers hold, rounded up
+    outgrown = set()
+    with vkvg_amd.Device() as dev:
+        for n, size, extent in [(60, 80, 20), (4000, 200, 9), (40, 2000, 1700), (40000, 200, 6), (30000, 1000, 60)]:
+            s = vkvg_amd.Surface(dev, size, size)
+            s.upload(_scene(n, size, extent).words())
+            for times in (2, 1):  # it outgrows the buffers, and then no more
+                vkvg_amd.execute(dev)
+                passes(dev._engine(), out)
+                assert list(out) == [3, times], (n, size, extent, list(out))
+            s.close()
+            st = dev.stats()
+            counts = np.array([st["path_tiles"], st["segments"]])
+            print(n, size, extent, counts, most)
+            outgrown.add(tuple(counts > 1.6 * most))  # a buffer grows to half as much again as needed
+            most = np.maximum(most, counts)
+    assert outgrown >= {(True, False), (False, True), (True, True)}, outgrown

@@ -212,6 +212,7 @@ struct vkh_engine {
     uint32_t sz[10] = {}; // points, overflow cubics, fill edges, stroke steps, stroke vertices, triangles, dash
                           // walk stopped, path tiles, segments, commands
     uint32_t fine_words = 4096;
+    uint32_t waits = 0, bin_passes = 0; // of the last eager frame: waits for counts, times its draws were binned
     std::vector<TargetInfo> h_tg;
     // draws without path tiles (target, index within the target's draws), and per (target, coarse
     // chunk) how many of them there are: every tile of the target holds their commands
@@ -722,6 +723,7 @@ static int totals(vkh_engine *eng, bool cap, const std::vector<const uint32_t *>
             dst[i] = eng->sz[slot + i];
         return 0;
     }
+    eng->waits++;
     if (read_totals(eng, srcs, dst))
         return -1;
     for (size_t i = 0; i < srcs.size(); i++)
@@ -740,8 +742,10 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     const uint32_t n_items = eng->n_items, n_sp = eng->n_sp, n_draws = eng->n_draws, n_units = eng->n_units;
     const uint32_t tile_total = eng->tile_total, bin_total = eng->bin_total;
     const uint32_t n_targets = eng->n_targets;
-    if (!cap)
+    if (!cap) {
+        eng->waits = 0;
         CK(hipEventRecord(eng->ev_begin, s));
+    }
     uint8_t *db = (uint8_t *)eng->blob.p;
     const vkh_item *d_items = (const vkh_item *)(db + eng->o_items);
     const vkh_subpath *d_sp = (const vkh_subpath *)(db + eng->o_sp);
@@ -901,22 +905,12 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                           d_gprep);
     if (scan_u32(eng, P<uint32_t>(eng->pt_count), n_draws, P<uint32_t>(eng->pt_off), cap))
         return -1;
-    // The path tiles, the binned segments and the commands are counted in one go with the buffers as they
-    // are: draws whose path tiles do not fit are left out of the binning and segments that do not fit are
-    // not written, and where that happened the buffers grow and the pass runs again. A wait for each of
-    // the three counts took some 20 us. The first frame of an engine has no buffers to try and waits for its path tiles.
-    if (!eng->ptiles.p) {
-        if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws}, tot, 7) ||
-            !need(eng, cap, eng->ptiles, sizeof(PathTile) * (size_t)tot[0] + 16))
-            return -1;
-    }
+    vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws);
     if (!need(eng, cap, eng->ptiles, sizeof(PathTile) + 16) || !need(eng, cap, eng->segs, 4096))
         return -1;
     if (!cap)
         CK(hipEventRecord(eng->ev_stage[2], s)); // tile setup done
-    // ---- binning: per-draw segment lists and backdrops; bins again once if the segment buffer
-    // was too small (the allocator then holds the exact total)
-    uint32_t n_segs = 0;
+    // ---- binning: per-draw segment lists and backdrops
     if (!need(eng, cap, eng->draw_order, 4ull * vkh::order_words(n_draws)))
         return -1;
     vkh::launch_draw_order(s, n_draws, P<uint2>(eng->erange), P<uint32_t>(eng->draw_order));
@@ -931,41 +925,43 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     const uint32_t n_tc = (uint32_t)n_tc64;
     if (!need(eng, cap, eng->tile_cnt, 4ull * (n_tc + 1)) || !need(eng, cap, eng->tile_off, 4ull * (n_tc + 1)))
         return -1;
-    uint32_t n_ptiles = 0;
-    for (int pass = 0;; pass++) {
-        const uint32_t seg_cap = (uint32_t)std::min<size_t>(eng->segs.cap / sizeof(Edge), 0xFFFFFFFFull);
-        const uint32_t pt_cap = (uint32_t)std::min<size_t>(eng->ptiles.cap / sizeof(PathTile), 0xFFFFFFFFull);
-        if (pass) {
-            vkh::launch_zero_u32(s, ctr, 1);
-            vkh::launch_draw_tiles(s, d_draws, n_draws, d_tg, P<int4>(eng->bbox), T, P<DrawTiles>(eng->dtiles),
-                                   P<uint32_t>(eng->pt_count)); // those left out are back
-        }
-        vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws, pt_cap);
-        vkh::launch_tile_cnt_init(s, d_tg, n_targets, nch, eng->d_tl_table, P<uint32_t>(eng->tile_cnt), n_tc);
-        vkh::launch_bin_draws(s, P<Edge>(eng->edges), P<uint2>(eng->erange),
-                              P<DrawTiles>(eng->dtiles), n_draws, T, P<PathTile>(eng->ptiles), P<Edge>(eng->segs),
-                              seg_cap, ctr, P<uint32_t>(eng->draw_order), d_draws, d_tg, nch,
-                              eng->coarse_chunk, P<uint32_t>(eng->tile_cnt), P<DrawPrep>(eng->dprep));
+    vkh::launch_tile_cnt_init(s, d_tg, n_targets, nch, eng->d_tl_table, P<uint32_t>(eng->tile_cnt), n_tc);
+    // The path tiles, the segments and the commands are counted in one go with the buffers as they are (a
+    // wait for each of the three took some 20 us). What does not fit is counted and not written, so where
+    // that happened the buffers grow and the draws are binned once more: the counts stand.
+    uint32_t passes = 0;
+    auto bin = [&]() {
+        vkh::launch_bin_draws(s, P<Edge>(eng->edges), P<uint2>(eng->erange), P<DrawTiles>(eng->dtiles), n_draws, T,
+                              P<PathTile>(eng->ptiles),
+                              (uint32_t)std::min<size_t>(eng->ptiles.cap / sizeof(PathTile), 0xFFFFFFFFull),
+                              P<Edge>(eng->segs),
+                              (uint32_t)std::min<size_t>(eng->segs.cap / sizeof(Edge), 0xFFFFFFFFull), ctr,
+                              P<uint32_t>(eng->draw_order), d_draws, d_tg, nch, eng->coarse_chunk,
+                              P<uint32_t>(eng->tile_cnt), P<DrawPrep>(eng->dprep));
+        passes++;
+    };
+    bin();
+    CK(hipGetLastError());
+    if (!cap)
+        CK(hipEventRecord(eng->ev_stage[3], s)); // binning done
+    // ---- coarse: ordered command list per tile (the counts came from binning)
+    if (scan_u32(eng, P<uint32_t>(eng->tile_cnt), n_tc, P<uint32_t>(eng->tile_off), cap))
+        return -1;
+    if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws, ctr, P<uint32_t>(eng->tile_off) + n_tc}, tot, 7))
+        return -1;
+    const uint32_t n_ptiles = tot[0], n_segs = tot[1];
+    const size_t pt_bytes = sizeof(PathTile) * (size_t)n_ptiles, seg_bytes = sizeof(Edge) * (size_t)n_segs;
+    if (pt_bytes > eng->ptiles.cap || seg_bytes > eng->segs.cap) {
+        if (!need(eng, cap, eng->ptiles, pt_bytes) || !need(eng, cap, eng->segs, seg_bytes))
+            return -1;
+        vkh::launch_zero_u32(s, ctr, 1);
+        bin();
         CK(hipGetLastError());
         if (!cap)
-            CK(hipEventRecord(eng->ev_stage[3], s)); // binning done
-        // ---- coarse: ordered command list per tile (the counts came from binning)
-        if (scan_u32(eng, P<uint32_t>(eng->tile_cnt), n_tc, P<uint32_t>(eng->tile_off), cap))
-            return -1;
-        if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws, ctr, P<uint32_t>(eng->tile_off) + n_tc}, tot, 7))
-            return -1;
-        n_ptiles = tot[0];
-        n_segs = tot[1]; // of the draws that were not left out
-        if (n_ptiles <= pt_cap && n_segs <= seg_cap)
-            break;
-        if (pass == 2) { // one pass for the path tiles, one for the segments
-            eng->err = "segment buffer overflow after resize";
-            return -1;
-        }
-        if (!need(eng, cap, eng->ptiles, sizeof(PathTile) * (size_t)n_ptiles + 16) ||
-            !need(eng, cap, eng->segs, sizeof(Edge) * (size_t)n_segs + sizeof(Edge)))
-            return -1;
+            CK(hipEventRecord(eng->ev_stage[3], s));
     }
+    if (!cap)
+        eng->bin_passes = passes;
     st.path_tiles = n_ptiles;
     st.segments = n_segs;
     const uint32_t n_cmds = tot[2];
@@ -1178,6 +1174,13 @@ int vkvg_hip_render(vkh_engine *eng, const vkh_frame *f) {
     if (r)
         return r;
     return vkvg_hip_execute(eng);
+}
+
+// Diagnostic, not part of the public headers: of the last frame that ran eagerly, how often the host waited
+// for counts and how often its draws were binned
+__attribute__((visibility("default"))) void vkh_last_frame_passes(vkh_engine *eng, uint32_t out[2]) {
+    out[0] = eng->waits;
+    out[1] = eng->bin_passes;
 }
 
 // Diagnostics, not part of the public headers (0 expected, -1 on error): mismatches of the hardware

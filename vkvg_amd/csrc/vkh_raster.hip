@@ -79,18 +79,10 @@ __global__ void k_draw_tiles(const vkh_draw *__restrict__ draws, uint32_t n, con
     dt[i] = o;
 }
 
-// first path tile of every draw; one whose path tiles are not all below pt_cap loses its tiles
-__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t pt_cap) {
+__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    const uint32_t a = pt_off[i], b = pt_off[i + 1];
-    dt[i].pt_base = a;
-    if (a != b && b > pt_cap) {
-        dt[i].bx0 = dt[i].by0 = 0;
-        dt[i].bx1 = dt[i].by1 = -1;
-        dt[i].bw = 0;
-    }
+    if (i < n)
+        dt[i].pt_base = pt_off[i];
 }
 
 // ----------------------------------------------------------------------------------- edge binning
@@ -212,11 +204,13 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t *a, uint32_t n
 // Besides the path tiles and segments, every path tile that will hold a command (segments, a
 // non-zero blend count from its backdrop, or a clip) adds one to its tile's command count in the
 // draw's chunk (tile_cnt[tile * nch + chunk], the coarse pass's layout), so the coarse pass needs
-// no counting pass of its own.
+// no counting pass of its own. Path tiles beyond pt_cap and a band's segments beyond seg_cap are counted
+// like the others and not written.
 __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges, const uint2 *__restrict__ erange,
                                                   const DrawTiles *__restrict__ dts, uint32_t T,
-                                                  PathTile *__restrict__ pts, Edge *__restrict__ segs,
-                                                  uint32_t seg_cap, uint32_t *__restrict__ seg_alloc,
+                                                  PathTile *__restrict__ pts, uint32_t pt_cap,
+                                                  Edge *__restrict__ segs, uint32_t seg_cap,
+                                                  uint32_t *__restrict__ seg_alloc,
                                                   const uint32_t *__restrict__ draw_order,
                                                   const vkh_draw *__restrict__ draws, const TargetInfo *__restrict__ tg,
                                                   uint32_t nch, uint32_t chunk_draws, uint32_t *__restrict__ tile_cnt,
@@ -299,6 +293,7 @@ __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges
         __syncthreads();
         const uint32_t base = s_base;
         const bool fits = (uint64_t)base + total <= (uint64_t)seg_cap;
+        const bool room = (uint64_t)dt.pt_base + r0 * bw + nt <= (uint64_t)pt_cap;
         PathTile *out = pts + dt.pt_base + r0 * bw;
         for (uint32_t k = tid; k < nt; k += 256) {
             const uint32_t off = s_cnt[k];
@@ -316,7 +311,8 @@ __global__ __launch_bounds__(256) void k_bin_draw(const Edge *__restrict__ edges
                     (float)min(x + (1 << lt), (int32_t)TI.width) - 0.5f,
                     (float)min(y + (1 << lt), (int32_t)TI.height) - 0.5f, (float)TI.width, (float)TI.height);
             }
-            out[k] = p;
+            if (room)
+                out[k] = p;
             if (p.nseg || clip || coverage_count(kind, p.backdrop) != 0) {
                 const uint32_t gtile = TI.tile_base + (uint32_t)(ty_lo + (int32_t)r) * TI.tilesW + (uint32_t)dt.bx0 + c;
                 atomicAdd(&tile_cnt[(size_t)gtile * nch + chunk], 1u);
@@ -1320,21 +1316,21 @@ void launch_draw_tiles(hipStream_t s, const vkh_draw *draws, uint32_t n, const T
         hipLaunchKernelGGL(k_draw_tiles, dim3((n + 255) / 256), dim3(256), 0, s, draws, n, tg, bbox, tile, dt,
                            pt_count);
 }
-void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t pt_cap) {
+void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
     if (n)
-        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n, pt_cap);
+        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n);
 }
 void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n) {
     if (n)
         hipLaunchKernelGGL(k_zero_u32, dim3((n + 255) / 256), dim3(256), 0, s, p, n);
 }
 void launch_bin_draws(hipStream_t s, const Edge *edges, const uint2 *erange,
-                      const DrawTiles *dt, uint32_t n_draws, uint32_t tile, PathTile *pts, Edge *segs,
+                      const DrawTiles *dt, uint32_t n_draws, uint32_t tile, PathTile *pts, uint32_t pt_cap, Edge *segs,
                       uint32_t seg_cap, uint32_t *seg_alloc, const uint32_t *order, const vkh_draw *draws,
                       const TargetInfo *tg, uint32_t nch, uint32_t chunk_draws, uint32_t *tile_cnt,
                       const DrawPrep *dprep) {
     if (n_draws)
-        hipLaunchKernelGGL(k_bin_draw, dim3(n_draws), dim3(256), 0, s, edges, erange, dt, tile, pts, segs,
+        hipLaunchKernelGGL(k_bin_draw, dim3(n_draws), dim3(256), 0, s, edges, erange, dt, tile, pts, pt_cap, segs,
                            seg_cap, seg_alloc, order, draws, tg, nch, chunk_draws, tile_cnt, dprep);
 }
 void launch_tile_cnt_init(hipStream_t s, const TargetInfo *tg, uint32_t n_targets, uint32_t nch,
