@@ -84,3 +84,34 @@ def test_outgrown_buffers_cost_one_more_binning_and_no_wait():
             outgrown.add(tuple(counts > 1.6 * most))  # a buffer grows to half as much again as needed
             most = np.maximum(most, counts)
     assert outgrown >= {(True, False), (False, True), (True, True)}, outgrown
+
+
+def test_more_path_tiles_than_32_bits_are_refused():
+    """1025 slivers across a 32768x32768 surface: 2048x2048 tiles of 16 pixels each, 2^32 + 2^22 path tiles, whose
+    32-bit sum would be 2^22. The frame is refused and the next one renders."""
+    import vkvg_amd
+    s = Stream()
+    s.set_source_rgba(0, 0, 0, 1)
+    for _ in range(1025):
+        s.move_to(0.5, 0.5)
+        s.line_to(32767.5, 32767.5)
+        s.line_to(32767.5, 32766.5)
+        s.fill()
+    t = Stream()
+    t.set_source_rgba(0, 0, 1, 1)
+    t.rectangle(100, 100, 8, 8)
+    t.fill()
+    with vkvg_amd.Device() as dev:
+        surf = vkvg_amd.Surface(dev, 32768, 32768)
+        surf.upload(s.words())
+        with pytest.raises(vkvg_amd.VkvgError):
+            vkvg_amd.execute(dev)
+        L = vkvg_amd.lib()
+        L.vkvg_hip_last_error.restype = ctypes.c_char_p
+        L.vkvg_hip_last_error.argtypes = [ctypes.c_void_p]
+        assert b"path tiles" in L.vkvg_hip_last_error(dev._engine())
+        small = vkvg_amd.Surface(dev, 128, 128)
+        small.replay(t.words())
+        assert small.premultiplied()[104, 104].tolist() == [0, 0, 255, 255]
+        small.close()
+        surf.close()

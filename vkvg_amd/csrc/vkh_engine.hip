@@ -209,8 +209,8 @@ struct vkh_engine {
     hipGraphExec_t gexec = nullptr;
     uint64_t gkey = 0, gfail_key = 0;
     uint64_t frame_gen = 0, alloc_gen = 0;
-    uint32_t sz[10] = {}; // points, overflow cubics, fill edges, stroke steps, stroke vertices, triangles, dash
-                          // walk stopped, path tiles, segments, commands
+    uint32_t sz[11] = {}; // points, overflow cubics, fill edges, stroke steps, stroke vertices, triangles, dash
+                          // walk stopped, path tiles, segments, commands, path tiles overflowed
     uint32_t fine_words = 4096;
     uint32_t waits = 0, bin_passes = 0; // of the last eager frame: waits for counts, times its draws were binned
     std::vector<TargetInfo> h_tg;
@@ -771,9 +771,9 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     if (!need(eng, cap, eng->flat_wh, 4ull * (2ull * n_wh + 2)))
         return -1;
     // [0] segments, [1] flatten slots, [2] overflow cubics, [3] long dashed pieces, [4] a dash walk
-    // stopped at its cap bound
+    // stopped at its cap bound, [5] more path tiles than 32 bits count
     uint32_t *ctr = P<uint32_t>(eng->counters);
-    vkh::launch_zero_u32(s, ctr, 5);
+    vkh::launch_zero_u32(s, ctr, 6);
     if (n_items) {
         uint32_t *whist = P<uint32_t>(eng->flat_wh), *wcur = whist + n_wh + 1;
         vkh::launch_flat_hist(s, d_items, n_items, whist);
@@ -905,7 +905,7 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
                           d_gprep);
     if (scan_u32(eng, P<uint32_t>(eng->pt_count), n_draws, P<uint32_t>(eng->pt_off), cap))
         return -1;
-    vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws);
+    vkh::launch_set_pt_base(s, P<DrawTiles>(eng->dtiles), P<uint32_t>(eng->pt_off), n_draws, ctr + 5);
     if (!need(eng, cap, eng->ptiles, sizeof(PathTile) + 16) || !need(eng, cap, eng->segs, 4096))
         return -1;
     if (!cap)
@@ -947,8 +947,13 @@ static int run_pipeline(vkh_engine *eng, bool cap) {
     // ---- coarse: ordered command list per tile (the counts came from binning)
     if (scan_u32(eng, P<uint32_t>(eng->tile_cnt), n_tc, P<uint32_t>(eng->tile_off), cap))
         return -1;
-    if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws, ctr, P<uint32_t>(eng->tile_off) + n_tc}, tot, 7))
+    if (totals(eng, cap, {P<uint32_t>(eng->pt_off) + n_draws, ctr, P<uint32_t>(eng->tile_off) + n_tc, ctr + 5}, tot,
+               7))
         return -1;
+    if (tot[3]) {
+        eng->err = "frame too large (path tiles)";
+        return -3;
+    }
     const uint32_t n_ptiles = tot[0], n_segs = tot[1];
     const size_t pt_bytes = sizeof(PathTile) * (size_t)n_ptiles, seg_bytes = sizeof(Edge) * (size_t)n_segs;
     if (pt_bytes > eng->ptiles.cap || seg_bytes > eng->segs.cap) {

@@ -179,7 +179,7 @@ void launch_tri_edges(hipStream_t s, const Unit *units, uint32_t n_units, const 
 void launch_draw_bbox_init(hipStream_t s, int4 *bbox, uint2 *erange, uint32_t n_draws);
 void launch_draw_tiles(hipStream_t s, const vkh_draw *draws, uint32_t n_draws, const TargetInfo *tg,
                        const int4 *bbox, uint32_t tile, DrawTiles *dt, uint32_t *pt_count);
-void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n_draws);
+void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n_draws, uint32_t *over);
 void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n);
 void launch_bin_draws(hipStream_t s, const Edge *edges, const uint2 *erange,
                       const DrawTiles *dt, uint32_t n_draws, uint32_t tile, PathTile *pts, uint32_t pt_cap, Edge *segs,

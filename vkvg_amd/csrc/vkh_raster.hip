@@ -79,10 +79,16 @@ __global__ void k_draw_tiles(const vkh_draw *__restrict__ draws, uint32_t n, con
     dt[i] = o;
 }
 
-__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
+// a draw holds fewer than 2^32 path tiles, so where the frame's sum passes 2^32 a draw's end lies below its
+// begin: *over is set
+__global__ void k_set_pt_base(DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t *over) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        dt[i].pt_base = pt_off[i];
+    if (i >= n)
+        return;
+    const uint32_t a = pt_off[i];
+    dt[i].pt_base = a;
+    if (pt_off[i + 1] < a)
+        *over = 1u;
 }
 
 // ----------------------------------------------------------------------------------- edge binning
@@ -1316,9 +1322,9 @@ void launch_draw_tiles(hipStream_t s, const vkh_draw *draws, uint32_t n, const T
         hipLaunchKernelGGL(k_draw_tiles, dim3((n + 255) / 256), dim3(256), 0, s, draws, n, tg, bbox, tile, dt,
                            pt_count);
 }
-void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n) {
+void launch_set_pt_base(hipStream_t s, DrawTiles *dt, const uint32_t *pt_off, uint32_t n, uint32_t *over) {
     if (n)
-        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n);
+        hipLaunchKernelGGL(k_set_pt_base, dim3((n + 255) / 256), dim3(256), 0, s, dt, pt_off, n, over);
 }
 void launch_zero_u32(hipStream_t s, uint32_t *p, uint32_t n) {
     if (n)
