@@ -48,6 +48,10 @@ def _scene(name):
         a = np.arange(6) * (2 * np.pi / 6)
         w = np.stack([90.3 + 6 * np.cos(a), 40.7 + 5 * np.sin(a)], 1)
         return 160, 80, [_polygon(w, 0.13), _polygon([[20, 20], [60, 12], [40, 66]], 0.2)], [46.0, 0]
+    if name == "long":  # rows of 1300 edges and three times 128 columns, shared out over workgroups
+        a = np.sort(r.uniform(0, 2 * np.pi, 170))
+        w = np.stack([150 + 170 * np.cos(a), 18 + 13 * np.sin(a)], 1) + r.normal(0, 1, (170, 2))
+        return 291, 37, [_polygon(w), _polygon([[20, 5], [60, 30], [99, 7]]), _polygon(w[::12] * [0.9, 1.1], 0.1)], [0, 0, 1]
     if name == "point":  # one pixel, and a path that misses it on each side
         return 1, 1, [_polygon([[-0.7, 0.3], [0.6, -0.4], [0.9, 1.6]]), _polygon([[5, 5], [7, 5], [6, 8]]),
                       _polygon([[-9, 0.2], [-4, 0.4], [-6, 0.9]]), _polygon([[0.1, -8], [0.7, -3], [0.3, -5]])], [0, 0, 1, 0]
@@ -58,7 +62,7 @@ def _scene(name):
     return 211, 75, paths, list(r.integers(0, 2, 12))
 
 
-@pytest.mark.parametrize("name", ["tile", "aligned", "wide", "tall", "tight", "point", "curved"])
+@pytest.mark.parametrize("name", ["tile", "aligned", "wide", "tall", "tight", "long", "point", "curved"])
 def test_rows_match_fp64_reference(name):
     import torch
     from vkvg_amd import diff
@@ -126,3 +130,43 @@ def test_coverage_beside_an_outline_is_exact(kind):
         inside, outside = ~near & (ref < 0.5), ~near & (ref > 0.5)
         assert inside.sum() > 1000 and outside.sum() > 1000
         assert (img[outside] == 1).all() and (img[inside] == 0).all()
+
+
+def test_a_path_in_few_rows_is_shared_out():
+    """One path of 200 cubics over a strip of 8192x64 px: four tile rows of 64 times 128 columns and up to 3200 edges.
+    With one workgroup per tile row its forward took 8.9 ms."""
+    import torch
+    from vkvg_amd import diff
+    r = np.random.Generator(np.random.PCG64(1))
+    ctrl = (np.array([4096, 32]) + [2500, 20] * r.standard_normal((600, 2))).astype(np.float32)
+    R = diff.DiffRenderer(8192, 64, np.array([200], np.uint32), np.zeros(1, np.uint32))
+    args = [torch.tensor(x, device="cuda") for x in (ctrl, np.full((1, 4), 0.5, np.float32), np.zeros(1, np.float32))]
+    ms = []
+    for _ in range(5):
+        img = R.forward(*args)
+        ms.append(R.last_ms())
+    print(ms, flush=True)
+    assert float((img.double() - R.forward64(*args)).abs().max()) < 2e-2  # coordinates of 8192 are spaced 1e-3
+    R.close()
+    assert min(ms) < 1.7, ms
+
+
+def test_more_row_units_than_a_launch_takes():
+    """8200 paths over 1024 tile rows are 2^23 + 8192 workgroups: the last paths' rows are in a second launch."""
+    import torch
+    from vkvg_amd import diff
+    n = 8200
+    r = np.random.Generator(np.random.PCG64(2))
+    one = np.array([[2, 4], [2, 16300], [14, 16380]], np.float32)  # a closed cubic from top to bottom
+    ctrl = np.tile(one, (n, 1))
+    rgba = np.concatenate([r.uniform(0, 1, (n, 3)), np.full((n, 1), 0.001)], 1).astype(np.float32)
+    rgba[-1] = 0.25, 0.5, 0.75, 1
+    nc, stroke = np.ones(n, np.uint32), np.zeros(n, np.uint32)
+    img = []
+    for k in (n, 1):  # all of them, and the last one alone
+        R = diff.DiffRenderer(16, 16384, nc[-k:], stroke[-k:])
+        args = [torch.tensor(x, device="cuda") for x in (ctrl[-3 * k:], rgba[-k:], np.zeros(k, np.float32))]
+        img.append(R.forward(*args))
+        R.close()
+    inside = (img[1] - torch.tensor([0.25, 0.5, 0.75, 1.0], device="cuda")).abs().amax(-1) == 0
+    assert int(inside.sum()) > 10000 and bool((img[0][inside] == img[1][inside]).all())

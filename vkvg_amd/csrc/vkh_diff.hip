@@ -14,6 +14,7 @@
 //   k_dcov          one wavefront per (path, tile row): its edges' area deltas are added up in LDS over
 //                   the path's whole width, eight tiles at a time, and prefix-summed along the pixel rows
 //                   into the coverage buffer (A per command and pixel)
+//   k_dcov_split, k_dcov_sum   the same for the rows whose lists are too long or too wide for one workgroup
 //   k_work_order    the tiles heaviest first (commands per tile), for k_dcomp and k_dback
 //   k_dcomp         one workgroup per 16x16 tile, one thread per pixel: composites the tile's
 //                   commands in draw order from the coverage buffer. With checkpoints on, the pixel
@@ -271,9 +272,10 @@ __global__ __launch_bounds__(256) void k_dpaths(const uint32_t *__restrict__ pat
 }
 
 // Positions of every path's tiles, rows and list entries (exclusive sums, in one workgroup), and the totals
-// into the host's memory
+// into the host's memory; clears k_dbin's counters of split rows
 __global__ __launch_bounds__(1024) void k_dalloc(uint32_t n_paths, PathAlloc *__restrict__ alloc,
-                                                 DrawTiles *__restrict__ dts, uint32_t *__restrict__ totals) {
+                                                 DrawTiles *__restrict__ dts, uint32_t *__restrict__ split,
+                                                 uint32_t *__restrict__ totals) {
     __shared__ uint32_t s_w[16][3];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
     uint32_t run[3] = {0, 0, 0};
@@ -308,8 +310,10 @@ __global__ __launch_bounds__(1024) void k_dalloc(uint32_t n_paths, PathAlloc *__
         __syncthreads();
     }
     if (tid == 0)
-        for (int k = 0; k < 3; k++)
+        for (int k = 0; k < 3; k++) {
             totals[k] = run[k];
+            split[k] = 0;
+        }
 }
 
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uint32_t *s_wave) {
@@ -342,17 +346,36 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t *a, uint32_t n, uin
 }
 
 // A tile row with coverage: path and row within its bbox. Its list is in the row's first path tile
-// (seg_off, ntouch); nseg of every path tile says whether it gets a command.
+// (seg_off, ntouch); nseg of every path tile says whether it gets a command. acc: VKD_WHOLE, or where the sums
+// of a row begin that is split over workgroups (SplitRow).
+#define VKD_WHOLE 0xFFFFFFFFu
 struct RowUnit {
-    uint32_t draw, row;
+    uint32_t draw, row, acc;
 };
+// A row that k_dcov_split shares out: one workgroup per VKD_CT tiles and VKD_SLICE entries of the list,
+// from workgroup `first` on
+#define VKD_SLICE 1024u
+struct SplitRow {
+    uint32_t unit, first;
+};
+// What a tile row costs its workgroup, in steps of some 2 us: one per 256 list entries and eight tiles, mostly entries
+// passed over, and four per 256 entries for what they add. A row is split beyond 96 steps (splitting takes 20
+// to 50 us itself: 10 strokes of 30 cubics on 1024x1024, 60 steps, 210 us whole and 266 split; 6 paths of 50 cubics on
+// 300x40, 112 steps, 332 and 234), and beyond four times what the frame's rows take together on some 2048 workgroups at a
+// time: up to there a whole row ends with the others.
+__device__ __forceinline__ uint32_t row_steps(uint32_t eights, uint32_t n) { return (eights + 4u) * ((n + 255u) / 256u); }
+inline uint32_t split_steps(uint32_t n_ptiles, uint32_t n_rows, uint32_t n_segs) {
+    return std::max<uint32_t>(96u, (uint32_t)((n_ptiles / VKD_CT + 4ull * n_rows + n_segs / 64u) / 512u));
+}
 
 template <typename R>
 __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_first_edge,
                                               const RV4<R> *__restrict__ edges, const DrawTiles *__restrict__ dts,
                                               const PathAlloc *__restrict__ alloc, PathTile *__restrict__ ptl,
                                               uint32_t *__restrict__ cmd_of, uint32_t *__restrict__ segs,
-                                              RowUnit *__restrict__ units) {
+                                              RowUnit *__restrict__ units, SplitRow *__restrict__ splits,
+                                              unsigned long long *__restrict__ n_split, uint32_t *__restrict__ n_acc,
+                                              uint32_t max_steps) {
     __shared__ uint32_t s_cnt[VKD_ROWS_MAX]; // edges per row, then offsets, then cursors
     __shared__ int32_t s_col[VKD_ROWS_MAX];  // first tile column reached
     __shared__ uint32_t s_wave[4];
@@ -387,8 +410,17 @@ __global__ __launch_bounds__(256) void k_dbin(const uint32_t *__restrict__ path_
         ptl[dt.pt_base + k] = pt;
         cmd_of[dt.pt_base + k] = VKD_NO_CMD;
     }
-    for (uint32_t k = tid; k < bh; k += 256)
-        units[unit0 + k] = RowUnit{d, k};
+    for (uint32_t k = tid; k < bh; k += 256) {
+        const uint32_t n = (k + 1 < bh ? s_cnt[k + 1] : total) - s_cnt[k], eights = (bw + VKD_CT - 1) / VKD_CT;
+        uint32_t acc = VKD_WHOLE;
+        if (row_steps(eights, n) > max_steps) { // rows in the upper half, workgroups in the lower: in one order
+            const unsigned long long at =
+                atomicAdd(n_split, (1ull << 32) + (unsigned long long)eights * ((n + VKD_SLICE - 1) / VKD_SLICE));
+            splits[at >> 32] = SplitRow{unit0 + k, (uint32_t)at};
+            acc = atomicAdd(n_acc, eights);
+        }
+        units[unit0 + k] = RowUnit{d, k, acc};
+    }
     __syncthreads();
     for (uint32_t e = e0 + tid; e < e1; e += 256) {
         int32_t r0, r1, c0;
@@ -519,100 +551,171 @@ __device__ __forceinline__ double deposit(double x) { return x; }
 // pixel row is prefix-summed (two columns per lane, the sum so far carried on) into cov[c * 256 + pixel]. Each
 // edge is so evaluated once per pixel row it crosses (2.7 on edges of 3 px) and not in all 16 rows of every
 // tile up to the right end of the path, which the carry covers. Bound by the chains of instructions per row and
-// piece; with one wavefront per tile row, that of the longest list (a path of 1280 edges within a few tile rows)
-// set the time. 1024x768 with 3000 paths (1.4 M edges): 406 us with all rows of all tiles, 175 with a
-// wavefront, now 121; 512x512 with 1024: 180, 93, now 55; 100x72 with 48: 93, 61, now 22 us.
+// piece. 1024x768 with 3000 paths (1.4 M edges): 121 us (406 with all rows of all tiles); 512x512 with 1024: 55 (180);
+// 100x72 with 48: 22 (93).
+constexpr int VKD_COLS = VKD_CT * VKD_T, VKD_LD = VKD_COLS + 2; // one more cell takes the last column's overflow
+constexpr int VKD_RW = VKD_T / 4;                               // pixel rows that a wavefront prefix-sums
+static_assert(VKD_COLS == 128, "two columns per lane");
+
+// adds what the entries [i0, end) of a list, `share` at a time for this wavefront and every fourth such
+// share from i0 on, cover of the nt tiles from tile c0 of the row on to acc; ed and rows are the wavefront's own
+template <typename R>
+__device__ __forceinline__ void dcov_add(R *acc, RV4<R> *ed, RowShare &rows, uint32_t lane, const DrawTiles &dt, int32_t Y0,
+                                         uint32_t c0, uint32_t nt, uint32_t i0, uint32_t end, uint32_t share,
+                                         const uint32_t *__restrict__ list, const RV4<R> *__restrict__ edges) {
+    const R X0 = (R)(dt.bx0 * VKD_T); // x is taken from the path's left tile border: less rounding
+    const R XL = (R)(c0 * VKD_T), XR = XL + (R)(nt * VKD_T);
+    for (; i0 < end; i0 += 4 * share) {
+        int32_t ra = 0, rb = -1;
+        if (lane < share && i0 + lane < end) {
+            RV4<R> v = edges[list[i0 + lane]];
+            v.x -= X0;
+            v.z -= X0;
+            ed[lane] = v;
+            // left of these columns: in the carry
+            if (!((c0 && fmax(v.x, v.z) < XL) || fmin(v.x, v.z) > XR)) {
+                ra = (int32_t)fmin(fmax(floor(fmin(v.y, v.w)) - (R)Y0, (R)0), (R)VKD_T);
+                rb = (int32_t)fmax(fmin(floor(fmax(v.y, v.w)) - (R)Y0, (R)(VKD_T - 1)), (R)-1);
+            }
+        }
+        share_rows(rows, lane, ra, (uint32_t)max(rb - ra + 1, 0), [&](uint32_t j, int32_t r) {
+            RowPart<R> p;
+            if (!p.clip(ed[j], (R)(Y0 + r)))
+                return;
+            R *a = acc + r * VKD_LD;
+            R done = deposit(p.dy_left(XL));
+            if (c0 == 0 && done != (R)0)
+                atomicAdd(&a[0], done);
+            const R xa0 = fmax(p.xl, XL), xb0 = fmin(p.xr, XR);
+            if (!(xa0 <= xb0))
+                return;
+            const int32_t cl = (int32_t)(floor(xa0) - XL);
+            const int32_t cr = min((int32_t)(floor(xb0) - XL), (int32_t)(nt * VKD_T) - 1);
+            for (int32_t c = cl; c <= cr; c++) {
+                const R cx = XL + (R)c, cn = cx + (R)1;
+                const R xa = fmax(p.xl, cx), xb = fmin(p.xr, cn);
+                const R upto = deposit(p.dy_left(cn)), dy = upto - done;
+                done = upto;
+                const R right = deposit(dy * ((R)0.5 * (xa + xb) - cx));
+                atomicAdd(&a[c], dy - right);
+                atomicAdd(&a[c + 1], right);
+            }
+        });
+    }
+}
+
+// prefix sums of this wavefront's pixel rows of acc, onto carry and on, to the commands of the nt tiles from path tile pt
+// on; leaves the cells at zero
+template <typename R>
+__device__ __forceinline__ void dcov_sum(R *acc, R (&carry)[VKD_RW], uint32_t lane, uint32_t wv, uint32_t pt, uint32_t nt,
+                                         const uint32_t *__restrict__ cmd_of, R *__restrict__ cov) {
+    const uint32_t tl = lane / (64 / VKD_CT); // this lane's tile
+    const uint32_t cmd = tl < nt ? cmd_of[pt + tl] : VKD_NO_CMD;
+    R *out = cov + (size_t)cmd * 256 + 2 * (lane & (64 / VKD_CT - 1));
+#pragma unroll
+    for (int q = 0; q < VKD_RW; q++) {
+        const int r = (int)wv * VKD_RW + q;
+        RV2<R> *cell = (RV2<R> *)&acc[r * VKD_LD + 2 * lane];
+        const RV2<R> v = *cell;
+        const R over = acc[r * VKD_LD + VKD_COLS];
+        *cell = RV2<R>{(R)0, (R)0};
+        RV2<R> o;
+        o.x = wave_excl_sum(v.x + v.y, carry[q], lane) + v.x;
+        o.y = o.x + v.y;
+        if (cmd != VKD_NO_CMD)
+            *(RV2<R> *)(out + r * VKD_T) = o;
+        carry[q] = __shfl(o.y, 63) + over;
+    }
+    if (lane < VKD_RW)
+        acc[(wv * VKD_RW + lane) * VKD_LD + VKD_COLS] = (R)0;
+}
+
 template <typename R>
 __global__ __launch_bounds__(256) void k_dcov(const RowUnit *__restrict__ units, const DrawTiles *__restrict__ dts,
                                               const PathTile *__restrict__ ptl, const uint32_t *__restrict__ cmd_of,
                                               const uint32_t *__restrict__ segs, const RV4<R> *__restrict__ edges,
                                               R *__restrict__ cov) {
-    constexpr int COLS = VKD_CT * VKD_T, LD = COLS + 2; // one more cell takes the last column's overflow
-    constexpr int RW = VKD_T / 4;                       // pixel rows that a wavefront prefix-sums
-    static_assert(COLS == 128, "two columns per lane");
-    __shared__ alignas(16) R acc[VKD_T * LD];
+    __shared__ alignas(16) R acc[VKD_T * VKD_LD];
     __shared__ RV4<R> s_edge[4][64];
     __shared__ RowShare s_rows[4];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    RV4<R> *const ed = s_edge[wv];
     const RowUnit ru = units[blockIdx.x];
     const DrawTiles dt = dts[ru.draw];
     const uint32_t pt0 = dt.pt_base + ru.row * dt.bw;
     const uint32_t off = ptl[pt0].seg_off, n = ptl[pt0].ntouch;
-    if (!n)
+    if (!n || ru.acc != VKD_WHOLE)
         return;
-    for (uint32_t i = threadIdx.x; i < (uint32_t)(VKD_T * LD); i += 256)
+    for (uint32_t i = threadIdx.x; i < (uint32_t)(VKD_T * VKD_LD); i += 256)
         acc[i] = (R)0;
     __syncthreads();
     const int32_t Y0 = (dt.by0 + (int32_t)ru.row) * VKD_T;
-    const R X0 = (R)(dt.bx0 * VKD_T); // x is taken from the path's left tile border: less rounding
     const uint32_t share = min((n + 3) / 4, 64u); // edges per wavefront and turn
-    R carry[RW];
+    R carry[VKD_RW];
 #pragma unroll
-    for (int r = 0; r < RW; r++)
+    for (int r = 0; r < VKD_RW; r++)
         carry[r] = (R)0;
     for (uint32_t c0 = 0; c0 < dt.bw; c0 += VKD_CT) {
         const uint32_t nt = min((uint32_t)VKD_CT, dt.bw - c0);
-        const R XL = (R)(c0 * VKD_T), XR = XL + (R)(nt * VKD_T);
-        for (uint32_t i0 = wv * share; i0 < n; i0 += 4 * share) {
-            int32_t ra = 0, rb = -1;
-            if (lane < share && i0 + lane < n) {
-                RV4<R> v = edges[segs[off + i0 + lane]];
-                v.x -= X0;
-                v.z -= X0;
-                ed[lane] = v;
-                // left of these columns: in the carry
-                if (!((c0 && fmax(v.x, v.z) < XL) || fmin(v.x, v.z) > XR)) {
-                    ra = (int32_t)fmin(fmax(floor(fmin(v.y, v.w)) - (R)Y0, (R)0), (R)VKD_T);
-                    rb = (int32_t)fmax(fmin(floor(fmax(v.y, v.w)) - (R)Y0, (R)(VKD_T - 1)), (R)-1);
-                }
-            }
-            share_rows(s_rows[wv], lane, ra, (uint32_t)max(rb - ra + 1, 0), [&](uint32_t j, int32_t r) {
-                RowPart<R> p;
-                if (!p.clip(ed[j], (R)(Y0 + r)))
-                    return;
-                R *a = acc + r * LD;
-                R done = deposit(p.dy_left(XL));
-                if (c0 == 0 && done != (R)0)
-                    atomicAdd(&a[0], done);
-                const R xa0 = fmax(p.xl, XL), xb0 = fmin(p.xr, XR);
-                if (!(xa0 <= xb0))
-                    return;
-                const int32_t cl = (int32_t)(floor(xa0) - XL);
-                const int32_t cr = min((int32_t)(floor(xb0) - XL), (int32_t)(nt * VKD_T) - 1);
-                for (int32_t c = cl; c <= cr; c++) {
-                    const R cx = XL + (R)c, cn = cx + (R)1;
-                    const R xa = fmax(p.xl, cx), xb = fmin(p.xr, cn);
-                    const R upto = deposit(p.dy_left(cn)), dy = upto - done;
-                    done = upto;
-                    const R right = deposit(dy * ((R)0.5 * (xa + xb) - cx));
-                    atomicAdd(&a[c], dy - right);
-                    atomicAdd(&a[c + 1], right);
-                }
-            });
-        }
+        dcov_add(acc, s_edge[wv], s_rows[wv], lane, dt, Y0, c0, nt, wv * share, n, share, segs + off, edges);
         __syncthreads();
-        const uint32_t tl = lane / (64 / VKD_CT); // this lane's tile
-        const uint32_t cmd = tl < nt ? cmd_of[pt0 + c0 + tl] : VKD_NO_CMD;
-        R *out = cov + (size_t)cmd * 256 + 2 * (lane & (64 / VKD_CT - 1));
-#pragma unroll
-        for (int q = 0; q < RW; q++) {
-            const int r = (int)wv * RW + q;
-            RV2<R> *cell = (RV2<R> *)&acc[r * LD + 2 * lane];
-            const RV2<R> v = *cell;
-            const R over = acc[r * LD + COLS];
-            *cell = RV2<R>{(R)0, (R)0};
-            RV2<R> o;
-            o.x = wave_excl_sum(v.x + v.y, carry[q], lane) + v.x;
-            o.y = o.x + v.y;
-            if (cmd != VKD_NO_CMD)
-                *(RV2<R> *)(out + r * VKD_T) = o;
-            carry[q] = __shfl(o.y, 63) + over;
-        }
-        if (lane < RW)
-            acc[(wv * RW + lane) * LD + COLS] = (R)0;
+        dcov_sum(acc, carry, lane, wv, pt0 + c0, nt, cmd_of, cov);
         __syncthreads();
     }
+}
+
+// Rows too long for one workgroup (row_steps): one workgroup per eight tiles and VKD_SLICE entries adds its cells up in
+// LDS and then into the row's in memory, which k_dcov_sum carries on from eight to eight. 8192x64 with one path of
+// 200 cubics, forward: 348 us (8878 us with a workgroup per row, 1757 with a list of edges per tile, 64
+// entries at a time); four curled strokes of 300 cubics on 256x256: 517 us (970 and 846).
+template <typename R>
+__global__ __launch_bounds__(256) void k_dcov_split(const SplitRow *__restrict__ splits, uint32_t n_split, uint32_t g0,
+                                                    const RowUnit *__restrict__ units, const DrawTiles *__restrict__ dts,
+                                                    const PathTile *__restrict__ ptl, const uint32_t *__restrict__ segs,
+                                                    const RV4<R> *__restrict__ edges, R *__restrict__ sums) {
+    __shared__ alignas(16) R acc[VKD_T * VKD_LD];
+    __shared__ RV4<R> s_edge[4][64];
+    __shared__ RowShare s_rows[4];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t g = g0 + blockIdx.x;
+    uint32_t lo = 0, hi = n_split; // the last row that begins at or before this workgroup
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (splits[mid].first <= g)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const RowUnit ru = units[splits[lo].unit];
+    const DrawTiles dt = dts[ru.draw];
+    const PathTile &pt = ptl[dt.pt_base + ru.row * dt.bw];
+    const uint32_t eights = (dt.bw + VKD_CT - 1) / VKD_CT, i = g - splits[lo].first;
+    const uint32_t e = i % eights, c0 = e * VKD_CT, first = i / eights * VKD_SLICE, end = min(first + VKD_SLICE, pt.ntouch);
+    for (uint32_t k = threadIdx.x; k < (uint32_t)(VKD_T * VKD_LD); k += 256)
+        acc[k] = (R)0;
+    __syncthreads();
+    dcov_add(acc, s_edge[wv], s_rows[wv], lane, dt, (dt.by0 + (int32_t)ru.row) * VKD_T, c0,
+             min((uint32_t)VKD_CT, dt.bw - c0), first + wv * 64u, end, 64u, segs + pt.seg_off, edges);
+    __syncthreads();
+    R *out = sums + (size_t)(ru.acc + e) * (VKD_T * VKD_LD);
+    for (uint32_t k = threadIdx.x; k < (uint32_t)(VKD_T * VKD_LD); k += 256)
+        if (acc[k] != (R)0)
+            unsafeAtomicAdd(&out[k], acc[k]); // device memory
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_dcov_sum(const SplitRow *__restrict__ splits, const RowUnit *__restrict__ units,
+                                                  const DrawTiles *__restrict__ dts, const uint32_t *__restrict__ cmd_of,
+                                                  R *__restrict__ sums, R *__restrict__ cov) {
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const RowUnit ru = units[splits[blockIdx.x].unit];
+    const DrawTiles dt = dts[ru.draw];
+    const uint32_t pt0 = dt.pt_base + ru.row * dt.bw;
+    R carry[VKD_RW];
+#pragma unroll
+    for (int r = 0; r < VKD_RW; r++)
+        carry[r] = (R)0;
+    R *acc = sums + (size_t)ru.acc * (VKD_T * VKD_LD);
+    for (uint32_t c0 = 0; c0 < dt.bw; c0 += VKD_CT, acc += VKD_T * VKD_LD)
+        dcov_sum(acc, carry, lane, wv, pt0 + c0, min((uint32_t)VKD_CT, dt.bw - c0), cmd_of, cov);
 }
 
 // Compositing in draw order: one workgroup per 16x16 tile, one thread per pixel; coverage comes
@@ -982,9 +1085,11 @@ __global__ void k_dbatches(uint32_t n_tiles, uint32_t nch, const uint32_t *__res
 }
 
 // the counts that the host sizes its buffers by, written to its memory
-__global__ void k_dcounts(const uint32_t *a, const uint32_t *b, uint32_t *__restrict__ out) {
+__global__ void k_dcounts(const uint32_t *a, const uint32_t *b, const uint32_t *split, uint32_t *__restrict__ out) {
     out[0] = *a;
     out[1] = b ? *b : 0u;
+    for (int k = 0; k < 3; k++)
+        out[2 + k] = split[k]; // workgroups, rows, eights of tiles
 }
 
 __global__ void k_dzero(uint32_t *p, size_t n) {
@@ -992,6 +1097,8 @@ __global__ void k_dzero(uint32_t *p, size_t n) {
     if (i < n)
         p[i] = 0;
 }
+
+constexpr uint32_t VKD_LAUNCH = 1u << 23; // workgroups of 256 per launch: a grid holds fewer than 2^32 threads
 
 struct Buf {
     void *p = nullptr;
@@ -1012,7 +1119,7 @@ struct vkvg_diff_scene_t {
     Buf topology; // the static topology, whose parts follow
     Buf pt_path, ctrl_path, first_pt, first_ctrl, first_edge, ncubic, stroke, draws, tg, grad_units;
     // per call
-    Buf pts, nrm, edges, pts64, nrm64, edges64, dtiles, alloc, ptiles, cmd_of, segs, units, tile_cnt, tile_off, cmds,
+    Buf pts, nrm, edges, pts64, nrm64, edges64, dtiles, alloc, ptiles, cmd_of, segs, units, splits, n_split, sums, tile_cnt, tile_off, cmds,
         nbat, batch_off, ckpt, cov, tile_order, scan_tmp;
     Buf g_cov, own, own_n, g_pt, g_h, g_col;
     uint32_t *counts = nullptr; // pinned: the counts read back
@@ -1170,6 +1277,7 @@ VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint32_t n_paths
     ok = ok &&
          ensure(s, s->pts, 8ull * np) && ensure(s, s->nrm, 8ull * np) && ensure(s, s->edges, 16ull * ne) &&
          ensure(s, s->dtiles, sizeof(DrawTiles) * n_paths) && ensure(s, s->alloc, sizeof(PathAlloc) * n_paths) &&
+         ensure(s, s->n_split, 16) &&
          ensure(s, s->segs, 4096) && ensure(s, s->tile_cnt, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->tile_off, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->nbat, 4ull * (s->n_tiles + 1)) && ensure(s, s->batch_off, 4ull * (s->n_tiles + 1)) &&
@@ -1189,7 +1297,7 @@ void vkvg_diff_destroy(VkvgDiffScene s) {
     if (s->stream)
         (void)hipStreamSynchronize(s->stream);
     Buf *bufs[] = {&s->topology, &s->pts, &s->nrm, &s->edges, &s->pts64, &s->nrm64, &s->edges64,
-                   &s->dtiles, &s->alloc, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->tile_cnt, &s->tile_off,
+                   &s->dtiles, &s->alloc, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->splits, &s->n_split, &s->sums, &s->tile_cnt, &s->tile_off,
                    &s->cmds, &s->nbat, &s->batch_off, &s->ckpt, &s->cov, &s->tile_order, &s->scan_tmp, &s->g_cov,
                    &s->own, &s->own_n, &s->g_pt, &s->g_h, &s->g_col};
     for (Buf *b : bufs)
@@ -1233,7 +1341,7 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
     hipLaunchKernelGGL(k_dpaths<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
                        (int32_t)s->tilesW, (int32_t)s->tilesH, P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc));
     hipLaunchKernelGGL(k_dalloc, dim3(1), dim3(1024), 0, st, nd, P<PathAlloc>(s->alloc), P<DrawTiles>(s->dtiles),
-                       s->counts);
+                       P<uint32_t>(s->n_split), s->counts);
     if (!sync_counts(s))
         return -1;
     const uint32_t n_ptiles = s->counts[0], n_units = s->counts[1];
@@ -1241,11 +1349,15 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
     if (!ensure(s, s->ptiles, sizeof(PathTile) * ((size_t)n_ptiles + 1)) ||
         !ensure(s, s->cmd_of, 4ull * ((size_t)n_ptiles + 1)) ||
         !ensure(s, s->units, sizeof(RowUnit) * ((size_t)n_units + 1)) ||
+        !ensure(s, s->splits, sizeof(SplitRow) * ((size_t)n_units + 1)) ||
         !ensure(s, s->segs, 4ull * ((size_t)s->n_segs + 1)))
         return -1;
+    uint32_t *n_split = P<uint32_t>(s->n_split);
+    SplitRow *splits = P<SplitRow>(s->splits);
     hipLaunchKernelGGL(k_dbin<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
                        P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc), P<PathTile>(s->ptiles),
-                       P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RowUnit>(s->units));
+                       P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RowUnit>(s->units), splits,
+                       (unsigned long long *)n_split, n_split + 2, split_steps(n_ptiles, n_units, s->n_segs));
     const uint32_t n_tc = s->n_tiles * s->nch;
     const bool keep_ckpt = keep && sizeof(R) == sizeof(float);
     zero(s, s->tile_cnt, n_tc + 1);
@@ -1260,10 +1372,12 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
             return -1;
     }
     hipLaunchKernelGGL(k_dcounts, dim3(1), dim3(1), 0, st, P<uint32_t>(s->tile_off) + n_tc,
-                       keep_ckpt ? P<uint32_t>(s->batch_off) + s->n_tiles : nullptr, s->counts);
+                       keep_ckpt ? P<uint32_t>(s->batch_off) + s->n_tiles : nullptr, n_split, s->counts);
     if (!sync_counts(s))
         return -1;
     s->n_cmds = s->counts[0];
+    const uint32_t split_groups = s->counts[2], split_rows = s->counts[3];
+    const size_t sum_words = (size_t)s->counts[4] * (VKD_T * VKD_LD) * (sizeof(R) / 4);
     float4 *ck_ptr = nullptr;
     if (keep_ckpt) {
         s->n_batches = s->counts[1];
@@ -1272,7 +1386,7 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
         ck_ptr = P<float4>(s->ckpt);
     }
     if (!ensure(s, s->cmds, sizeof(Cmd) * ((size_t)s->n_cmds + 1)) ||
-        !ensure(s, s->cov, sizeof(R) * 256 * ((size_t)s->n_cmds + 1)))
+        !ensure(s, s->cov, sizeof(R) * 256 * ((size_t)s->n_cmds + 1)) || !ensure(s, s->sums, 4 * sum_words))
         return -1;
     vkh::launch_coarse(st, true, s->bin_total, s->nch, s->chunk, P<TargetInfo>(s->tg), 1, P<vkh_draw>(s->draws),
                        P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles), nullptr, P<uint32_t>(s->tile_off),
@@ -1280,9 +1394,19 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
     if (s->n_cmds) {
         hipLaunchKernelGGL(k_dcmd_of, dim3(blocks(s->n_cmds)), dim3(256), 0, st, s->n_cmds, P<Cmd>(s->cmds),
                            P<uint32_t>(s->cmd_of));
-        hipLaunchKernelGGL(k_dcov<R>, dim3(n_units), dim3(256), 0, st, P<RowUnit>(s->units), P<DrawTiles>(s->dtiles),
-                           P<PathTile>(s->ptiles), P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RV4<R>>(edges),
-                           P<R>(s->cov));
+        for (uint32_t u0 = 0; u0 < n_units; u0 += VKD_LAUNCH)
+            hipLaunchKernelGGL(k_dcov<R>, dim3(std::min(n_units - u0, VKD_LAUNCH)), dim3(256), 0, st,
+                               P<RowUnit>(s->units) + u0, P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles),
+                               P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RV4<R>>(edges), P<R>(s->cov));
+    }
+    if (s->n_cmds && split_rows) {
+        zero(s, s->sums, sum_words);
+        for (uint32_t g0 = 0; g0 < split_groups; g0 += VKD_LAUNCH)
+            hipLaunchKernelGGL(k_dcov_split<R>, dim3(std::min(split_groups - g0, VKD_LAUNCH)), dim3(256), 0, st, splits,
+                               split_rows, g0, P<RowUnit>(s->units), P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles),
+                               P<uint32_t>(s->segs), P<RV4<R>>(edges), P<R>(s->sums));
+        hipLaunchKernelGGL(k_dcov_sum<R>, dim3(split_rows), dim3(256), 0, st, splits, P<RowUnit>(s->units),
+                           P<DrawTiles>(s->dtiles), P<uint32_t>(s->cmd_of), P<R>(s->sums), P<R>(s->cov));
     }
     // tiles heaviest first (commands per tile vary several-fold), for compositing and the backward
     if (!ensure(s, s->tile_order, 4ull * vkh::order_words(s->n_tiles)))
