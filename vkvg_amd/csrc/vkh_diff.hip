@@ -23,7 +23,7 @@
 //   k_dback         per tile, batches in reverse: reads the batch's coverage, replays the
 //                   batch's compositing from its checkpoint and walks it backwards to get dL/dA per
 //                   (command, pixel) and the colour gradients
-//   k_dedge_grad    one wavefront per 6 points of a stroke or 60 of a fill: the boundary integral of
+//   k_dedge_grad    one wavefront per 6 points of a stroke or 8 to 60 of a fill: the boundary integral of
 //                   dL/dA over every piece of their edges inside a pixel, in all tiles that they
 //                   cross, added up to the gradients of the points and normals that the edges hang on
 //   k_dg_points, k_dg_ctrl, k_dg_paths: chain rule to points, half-widths, control points, colours and
@@ -466,7 +466,7 @@ template <typename R> struct RowPart {
     }
 };
 
-// Rows shared out over a wavefront: every lane has an edge with cnt (at most 16) pixel rows from row
+// Rows shared out over a wavefront: every lane has an edge with cnt (at most 16) pixel rows (or other items) from
 // `first` on, and f(lane of the edge, row) is called once for each of all the lanes' rows, 64 at a time. Edges
 // cross few rows, some many: a lane doing its own edge's rows would wait for the longest.
 struct RowShare {
@@ -863,7 +863,7 @@ __global__ __launch_bounds__(256) void k_dback(uint32_t W, uint32_t H, uint32_t 
 }
 
 // Gradients of the points and normals that the edges hang on. One wavefront takes the edges of 6 points of
-// a stroke (60) or 60 of a fill; one lane per edge and pixel row integrates dL/dA along the edge's pieces in the
+// a stroke (60) or 8 to 60 of a fill; one lane per edge and pixel row integrates dL/dA along the edge's pieces in the
 // row, over all tiles that it crosses, and adds to the edge's two sums in LDS. The edge's endpoint gradients are
 // (-dy, dx) times the sums. Edge layout per path: a fill has edge j = p_j -> p_j+1; a stroke has, per point j, 10
 // edges: the rectangle of segment j (p_j + n_j, p_j+1 + n_j, p_j+1 - n_j, p_j - n_j) and two bevel triangles at
@@ -871,11 +871,19 @@ __global__ __launch_bounds__(256) void k_dback(uint32_t W, uint32_t H, uint32_t 
 // half-width. Per point p the sums go to own[p] (on point p, on the next point) and, for strokes, to own_n[p]
 // (on normal p, on the previous normal, without the half-width). Bound by the loads of g_cov that wait for
 // the tile's command. With k_dg_points 83 us on 1024x768 with 3000 paths; one lane per edge for all its rows, the
-// edges' gradients written (23 MB) and gathered by two kernels, took 125 + 110 us.
+// edges' gradients written (23 MB) and gathered by two kernels, took 125 + 110 us. A lane takes at most VKD_EB columns of
+// a row, so that flat edges are shared out too: 8192x64 with one path of 200 cubics, whole backward, 117 us (738 with
+// whole rows, 190 with a thread per edge and tile).
+#define VKD_EB 32
 struct GradUnit {
-    uint32_t first_pt, path;
+    uint32_t first_pt, path, n; // n points
 };
-__host__ __device__ constexpr uint32_t grad_unit_points(bool stroke) { return stroke ? 6u : 60u; }
+// Points of a fill per wavefront: 60, fewer where that leaves the scene fewer than some 4096 wavefronts. 64x8192 with 20
+// paths of 60 cubics, backward: 280 us with 60 points, 203 with 1024 wavefronts, 148 with 4096; 1024x768 with 3000
+// paths: 160, 160 and 153.
+inline uint32_t fill_unit_points(uint64_t fill_points) {
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(fill_points / 4096u, 8u), 60u);
+}
 __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const GradUnit *__restrict__ units,
                                                     const uint32_t *__restrict__ path_first_pt,
                                                     const uint32_t *__restrict__ path_first_edge,
@@ -888,6 +896,7 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const Grad
                                                     float4 *__restrict__ own_n) {
     __shared__ float4 s_edge[4][64];
     __shared__ float s_sum[4][64][2];
+    __shared__ uint32_t s_blocks[4][64];
     __shared__ RowShare s_rows[4];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, u = blockIdx.x * 4u + wv;
     if (u >= n_units)
@@ -895,7 +904,7 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const Grad
     const GradUnit gu = units[u];
     const uint32_t d = gu.path, first = path_first_pt[d], end = path_first_pt[d + 1];
     const bool stroke = path_stroke[d] != 0;
-    const uint32_t per = stroke ? 10u : 1u, np = min(grad_unit_points(stroke), end - gu.first_pt);
+    const uint32_t per = stroke ? 10u : 1u, np = gu.n;
     const DrawTiles dt = dts[d];
     float4 *ed = s_edge[wv];
     float(*sum)[2] = s_sum[wv];
@@ -915,10 +924,28 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const Grad
     ed[lane] = v;
     sum[lane][0] = sum[lane][1] = 0.f;
     const float lo = (float)(dt.bx0 * VKD_T), hi = (float)((dt.bx1 + 1) * VKD_T);
-    while (__any(r0 <= r1)) { // up to 16 rows of every edge at a time
-        const uint32_t cnt = (uint32_t)min(max(r1 - r0 + 1, 0), VKD_T);
-        share_rows(s_rows[wv], lane, r0, cnt, [&](uint32_t j, int32_t r) {
+    // blocks of VKD_EB columns that the edge's part in a row spans at most (a column more at each end, and one for
+    // rounding); the last block takes what is left
+    uint32_t blocks = 1, items = 0;
+    if (r0 <= r1) {
+        const float dx = fabsf(v.z - v.x), w = fminf(fminf(dx, dx / fabsf(v.w - v.y)), hi - lo);
+        blocks = 1u + (uint32_t)((w + 3.f) * (1.f / VKD_EB));
+        items = (uint32_t)(r1 - r0 + 1) * blocks;
+    }
+    const bool wide = __any(blocks > 1u) != 0;
+    s_blocks[wv][lane] = blocks;
+    uint32_t done = 0;
+    while (__any(done < items)) { // up to 16 items of every edge at a time
+        const uint32_t cnt = min(items - done, (uint32_t)VKD_T);
+        share_rows(s_rows[wv], lane, (int32_t)done + (wide ? 0 : r0), cnt, [&](uint32_t j, int32_t r) {
             const float4 q = ed[j];
+            uint32_t b = 0, nb = 1;
+            if (wide) { // item r of the edge: row r / nb, block r % nb
+                nb = s_blocks[wv][j];
+                const uint32_t k = (uint32_t)r / nb;
+                b = (uint32_t)r - k * nb;
+                r = (int32_t)fmaxf(floorf(fminf(q.y, q.w)), (float)(dt.by0 * VKD_T)) + (int32_t)k;
+            }
             RowPart<float> p;
             if (!p.clip(RV4<float>{q.x, q.y, q.z, q.w}, (float)r))
                 return;
@@ -926,8 +953,13 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const Grad
             if (!(xa <= xb))
                 return;
             const uint32_t *co = cmd_of + dt.pt_base + (uint32_t)(r / VKD_T - dt.by0) * dt.bw;
-            const int32_t cl = (int32_t)floorf(xa), cr = min((int32_t)floorf(xb), (dt.bx1 + 1) * VKD_T - 1);
+            int32_t cl = (int32_t)floorf(xa), cr = min((int32_t)floorf(xb), (dt.bx1 + 1) * VKD_T - 1);
             float from = p.param(xa), ga = 0.f, gb = 0.f;
+            if (wide) {
+                cr = b + 1 < nb ? min(cr, cl + (int32_t)(b + 1) * VKD_EB - 1) : cr;
+                cl += (int32_t)b * VKD_EB;
+                from = b ? p.param((float)cl) : from;
+            }
             for (int32_t c = cl; c <= cr; c++) {
                 const float to = p.param((float)(c + 1));
                 const uint32_t cmd = co[c / VKD_T - dt.bx0];
@@ -946,7 +978,7 @@ __global__ __launch_bounds__(256) void k_dedge_grad(uint32_t n_units, const Grad
                 atomicAdd(&sum[j][1], gb);
             }
         });
-        r0 += (int32_t)cnt;
+        done += cnt;
     }
     const float ga = sum[lane][0], gb = sum[lane][1], dx = v.z - v.x, dy = v.w - v.y;
     const bool any = ga != 0.f || gb != 0.f;
@@ -1212,9 +1244,15 @@ VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint32_t n_paths
     s->n_ctrl = (uint32_t)nctl;
     s->n_edges = (uint32_t)ne;
     std::vector<GradUnit> gu;
+    uint64_t fill_points = 0;
     for (uint32_t i = 0; i < n_paths; i++)
-        for (uint32_t p = first_pt[i]; p < first_pt[i + 1]; p += grad_unit_points(stroke[i] != 0))
-            gu.push_back(GradUnit{p, i});
+        fill_points += stroke[i] ? 0u : first_pt[i + 1] - first_pt[i];
+    const uint32_t per_fill = fill_unit_points(fill_points);
+    for (uint32_t i = 0; i < n_paths; i++) {
+        const uint32_t per = stroke[i] ? 6u : per_fill;
+        for (uint32_t p = first_pt[i]; p < first_pt[i + 1]; p += per)
+            gu.push_back(GradUnit{p, i, std::min(per, first_pt[i + 1] - p)});
+    }
     s->n_grad_units = (uint32_t)gu.size();
     // draw records for the shared tile / coarse kernels: one target, kind per path
     std::vector<vkh_draw> dr(n_paths);
