@@ -336,18 +336,22 @@ def main() -> int:
     fine_bytes = 4 * sc.width * sc.height + 32 * sc.n_paths + 24 * sc.gradients + 20 * sc.gradient_stops
     achieved = fine_bytes / (fine_ms / 1e3) / 1e9
     traffic = _read_traffic("fine_c3_pmc.json")
-    # The fine kernel is limited by vector instruction issue, not by HBM: a wave64 VALU instruction
-    # occupies a 16-lane SIMD for 4 cycles, so the chip issues at most 1024 SIMDs x 2.4 GHz / 4 wave
-    # instructions per second. Its VALU instructions per launch come from the same counter summary.
+    # The fine kernel is limited by vector instruction issue, not by HBM. One kind of wave64 instruction
+    # at a time, a SIMD issues one of one or two 32-bit operands (add, subtract, shift, logic, move, float
+    # multiply and add) every 2.08 cycles, other ones (three operands, packed 16-bit, DPP, compares, double)
+    # every 4.06 and reciprocals every 8.1 (profiles/vector_issue_rates.md). The compiled kernel holds 492,
+    # 789 and 34 of these: 3.44 cycles on average, on 1024 SIMDs at 2.4 GHz. Its VALU instructions per
+    # launch come from the same counter summary.
     valu = _read_pmc("fine_c3_pmc.json", "valu_insts_per_launch")
-    issue_peak = 1024 * 2.4e9 / 4
+    issue_cycles = (492 * 2.08 + 789 * 4.06 + 34 * 8.1) / (492 + 789 + 34)
+    issue_peak = 1024 * 2.4e9 / issue_cycles
     issue = None if valu is None else {"achieved": valu / (fine_ms / 1e3), "peak": issue_peak,
                                        "unit": "wave64 VALU instructions/s",
                                        "frac": valu / (fine_ms / 1e3) / issue_peak,
                                        "valu_per_launch": valu,
-                                       "model": "4 cycles per counted wave64 VALU instruction on a 16-lane "
-                                                "SIMD; packed 16-bit instructions issue faster, so frac "
-                                                "near or above 1 means the kernel is at the issue limit"}
+                                       "model": f"{issue_cycles:.2f} cycles per wave64 VALU instruction and SIMD: "
+                                                "the measured issue rates of its kinds (2.08, 4.06 and 8.1 "
+                                                "cycles), weighted by how often the compiled kernel holds them"}
     # LDS from the same counter summary: SQ_LDS_IDX_ACTIVE over (GRBM_GUI_ACTIVE per XCD x 256 CUs)
     # is the fraction of CU-cycles the LDS served indexed accesses (peak 1); LDS atomics per second
     # against one wave64 LDS instruction per CU per cycle

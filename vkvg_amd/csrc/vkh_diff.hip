@@ -536,12 +536,13 @@ __device__ __forceinline__ float wave_excl_sum(float x, float carry, uint32_t) {
     return x;
 }
 
-// Deposits are rounded to 2^-23 and an edge's parts are differences of such numbers, so float sums of
-// them are exact up to 2 and right of a closed outline's edges its coverage is exactly 0 or 1 again, as
-// the sum of the edges' whole heights is. Against float64 over 160 scenes of 100x72 to 282x291 the image's
-// relative error is 0.4 to 1.7e-6 (0.5 to 1.8e-6 with a list of edges per tile, whose sums were not on a
-// grid), the colour gradients' 0.30 to 0.57e-6 (0.34 to 0.61e-6); without the grid the latter were 1.6 times
-// as large, with 2^-24, exact up to 1 only, 1.1 times.
+// Deposits are rounded to 2^-23 and an edge's parts are differences of such numbers, as coordinates from 1 on are.
+// While no partial sum exceeds 2 in magnitude float sums of them are therefore exact: they do not depend on
+// the order of the atomics, and beside a closed outline that winds once the coverage is exactly 0 or 1. Where a path
+// lies over itself more often (a tight bend of a wide stroke) sums are rounded, to 2^-22 from 2 to 4, and their
+// last bits depend on the order. Against float64 over 160 scenes of 100x72 to 282x291 the image's relative error is
+// 0.4 to 1.7e-6 (0.5 to 1.8e-6 with a list of edges per tile, whose sums were not on a grid), the colour
+// gradients' 0.30 to 0.57e-6 (0.34 to 0.61e-6; 1.6 times that without the grid, 1.1 times with 2^-24, exact up to 1 only).
 #define VKD_GRID 8388608.0f
 __device__ __forceinline__ float deposit(float x) { return rintf(x * VKD_GRID) * (1.0f / VKD_GRID); }
 __device__ __forceinline__ double deposit(double x) { return x; }
@@ -870,7 +871,7 @@ __global__ __launch_bounds__(256) void k_dback(uint32_t W, uint32_t H, uint32_t 
 // vertex j (p_j, then p_j + s n_j-1 and p_j + s n_j in the order of k_dedges; s = 1, -1), in units of the
 // half-width. Per point p the sums go to own[p] (on point p, on the next point) and, for strokes, to own_n[p]
 // (on normal p, on the previous normal, without the half-width). Bound by the loads of g_cov that wait for
-// the tile's command. With k_dg_points 83 us on 1024x768 with 3000 paths; one lane per edge for all its rows, the
+// the tile's command. With k_dg_points 76 us on 1024x768 with 3000 paths; one lane per edge for all its rows, the
 // edges' gradients written (23 MB) and gathered by two kernels, took 125 + 110 us. A lane takes at most VKD_EB columns of
 // a row, so that flat edges are shared out too: 8192x64 with one path of 200 cubics, whole backward, 117 us (738 with
 // whole rows, 190 with a thread per edge and tile).

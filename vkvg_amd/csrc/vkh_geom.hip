@@ -168,7 +168,7 @@ __global__ void k_flatten_copy(const vkh_item *__restrict__ items, uint32_t n_sl
 // Lines, one per thread, and arcs: a wavefront's arcs are shared out over its lanes, 64 lanes to a lone
 // one down to eight each, since a point's sine and cosine are a chain of hundreds of instructions and one
 // thread per arc runs them in series for the longest arc of the frame, while the angle's additions, which
-// every lane repeats, are one instruction a point. 777x777 with 150 shapes: 87 -> 23 us; a wavefront
+// every lane repeats, are one instruction a point. 777x777 with 500 shapes: 87 -> 23 us; a wavefront
 // full of arcs does an eighth of the points per lane for each eighth of its arcs, as much as before.
 #define VKH_ARC_LANES 8u
 __global__ __launch_bounds__(256) void k_flatten_lines(const vkh_item *__restrict__ items, uint32_t n,

@@ -914,14 +914,13 @@ template <int T> __device__ __forceinline__ int32_t tile_row_prefix(int32_t x, c
 // of the tile's sample rows into per-command LDS row deltas, walking only the rows the edge spans;
 // then every pixel applies the commands in order: its winding is the prefix of its row's deltas,
 // taken across the lanes that hold the row, and the command's record is read as wave-uniform values.
-// Bound by vector issue (85 % of it on the 1920x1080 stroke scene, 9.8 M commands: 1.21 G wave VALU
-// instructions in 2.33 ms). Two pixels per thread share what a command costs once per wave (its record's LDS
-// reads, decode, branches); pixels stay unpacked in 16-bit lanes between blends; the row prefix is four
-// DPP additions instead of a pass of 16-way conflicting LDS reads and writes per row; signatures are
-// compiled out where no target keeps them. One pixel per thread with the row pass: 3.11 ms there and
-// 1.82 ms on the 4096x4096 dense scene (4.0 M commands); this form 2.29 and 1.55 ms (1.40 since gradients
-// are solid over tiles where they have one colour; four pixels per thread: 3.01 and 1.89 ms, at 10 KB of LDS
-// per wavefront too few wavefronts are resident).
+// Bound by vector issue on the 4096x4096 dense scene (4.0 M commands): 0.97 G wave VALU instructions in 1.40 ms are
+// one per 3.5 cycles and SIMD, and the mix of them takes 3.4 (one or two 32-bit operands 2 cycles; three, packed
+// 16-bit, DPP, compares 4). On the 1920x1080 stroke scene (9.8 M commands) 1.21 G in 2.33 ms are one per 4.6: a
+// command's scalar instructions and LDS round trips take their share. Two pixels per thread share what a command
+// costs once per wave (its record's LDS reads, decode, branches); pixels stay unpacked in 16-bit lanes between
+// blends; the row prefix is four DPP additions; signatures are compiled out where no target keeps them. One pixel
+// per thread with a pass over the rows in LDS: 1.82 and 3.11 ms.
 // EXT: the frame has surface sources or targets with a stencil plane (the plain variant compiles
 // neither). With a stencil plane each pixel also carries its stencil word
 // (loaded from the plane or zero, stored back at the end): draws blend only where CLIP is 0, clear
@@ -1376,13 +1375,16 @@ static void fine_launch(hipStream_t s, bool ext, bool sig, uint32_t n_tiles, A..
     else
         launch(sig ? k_fine<T, NT, B, false, true> : k_fine<T, NT, B, false, false>);
 }
-// Threads and commands rasterized at a time, from the row-delta words W of the capacity setting. Tiles
-// of 16: two wavefronts with half of W, so that 16 workgroups fit a CU's LDS; but a frame of at most
-// VKH_FINE_WIDE tiles (all resident at once: 256 CUs x 16) leaves the chip partly idle and each tile's
-// chain of commands sets its time, so it takes four wavefronts and all of W per tile (512x512 with 200
-// paths: 114 us with two wavefronts, 78 us with four; 8160 heavy tiles of the stroke scene: 2.3 against
-// 3.1 ms). Tiles of 8 (one wavefront) and 32 (four) take half of W: more workgroups per CU (1500x1500
-// dense scene, tile 8: 0.24 -> 0.13 ms).
+// Threads and commands rasterized at a time, from the row-delta words W of the capacity setting. Tiles of 16: two
+// wavefronts with half of W, of which 16 workgroups fit a CU. A frame of few tiles leaves the chip partly idle and each
+// tile's chain of commands sets its time, so up to VKH_FINE_WIDE tiles it takes four wavefronts and all of W per tile.
+// Of these 8 fit a CU (4 at W = 8192, by their LDS), 2048 (1024) tiles at once; above, both forms run in several rounds.
+// Fine stage in us, two / four wavefronts, at 4096 and 5625 tiles with W = 4096, the default: curved fills 114 / 77 and
+// 113 / 91, dense scene 46 / 36 and 53 / 45, shapes 27 / 28 and 31 / 36, strokes 968 / 932 and 1368 / 1468; with
+// W = 2048 at 4096 tiles 142 / 94, 49 / 36, 32 / 30 and 1336 / 1217. With W = 8192 they cross between 2116 tiles (97 / 66,
+// 39 / 28, 27 / 30, 503 / 444) and 4096 (94 / 100, 47 / 48, 32 / 43, 1051 / 1200), by scene: the line of the others
+// serves. Tiles of 8 (one wavefront) and 32 (four) take half of W: more workgroups per CU (1500x1500 dense scene,
+// tile 8: 0.24 -> 0.13 ms).
 #define VKH_FINE_WIDE 4096
 template <int W, class... A>
 static void fine_words(hipStream_t s, bool ext, bool sig, uint32_t tile, uint32_t n_tiles, A... args) {
