@@ -1152,7 +1152,7 @@ struct vkvg_diff_scene_t {
     Buf topology; // the static topology, whose parts follow
     Buf pt_path, ctrl_path, first_pt, first_ctrl, first_edge, ncubic, stroke, draws, tg, grad_units;
     // per call
-    Buf pts, nrm, edges, pts64, nrm64, edges64, dtiles, alloc, ptiles, cmd_of, segs, units, splits, n_split, sums, tile_cnt, tile_off, cmds,
+    Buf pts, nrm, edges, pts64, nrm64, edges64, dtiles, alloc, ptiles, cmd_of, segs, units, sums, tile_cnt, tile_off, cmds,
         nbat, batch_off, ckpt, cov, tile_order, scan_tmp;
     Buf g_cov, own, own_n, g_pt, g_h, g_col;
     uint32_t *counts = nullptr; // pinned: the counts read back
@@ -1315,8 +1315,7 @@ VkvgDiffScene vkvg_diff_create(uint32_t width, uint32_t height, uint32_t n_paths
     }
     ok = ok &&
          ensure(s, s->pts, 8ull * np) && ensure(s, s->nrm, 8ull * np) && ensure(s, s->edges, 16ull * ne) &&
-         ensure(s, s->dtiles, sizeof(DrawTiles) * n_paths) && ensure(s, s->alloc, sizeof(PathAlloc) * n_paths) &&
-         ensure(s, s->n_split, 16) &&
+         ensure(s, s->dtiles, sizeof(DrawTiles) * n_paths) && ensure(s, s->alloc, 16 + sizeof(PathAlloc) * n_paths) &&
          ensure(s, s->segs, 4096) && ensure(s, s->tile_cnt, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->tile_off, 4ull * ((size_t)s->n_tiles * s->nch + 1)) &&
          ensure(s, s->nbat, 4ull * (s->n_tiles + 1)) && ensure(s, s->batch_off, 4ull * (s->n_tiles + 1)) &&
@@ -1336,7 +1335,7 @@ void vkvg_diff_destroy(VkvgDiffScene s) {
     if (s->stream)
         (void)hipStreamSynchronize(s->stream);
     Buf *bufs[] = {&s->topology, &s->pts, &s->nrm, &s->edges, &s->pts64, &s->nrm64, &s->edges64,
-                   &s->dtiles, &s->alloc, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->splits, &s->n_split, &s->sums, &s->tile_cnt, &s->tile_off,
+                   &s->dtiles, &s->alloc, &s->ptiles, &s->cmd_of, &s->segs, &s->units, &s->sums, &s->tile_cnt, &s->tile_off,
                    &s->cmds, &s->nbat, &s->batch_off, &s->ckpt, &s->cov, &s->tile_order, &s->scan_tmp, &s->g_cov,
                    &s->own, &s->own_n, &s->g_pt, &s->g_h, &s->g_col};
     for (Buf *b : bufs)
@@ -1369,6 +1368,8 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
     if (!ck(s, hipEventRecord(s->ev[0], st), "event"))
         return -1;
     const uint32_t np = s->n_pts, nd = s->n_paths;
+    uint32_t *n_split = P<uint32_t>(s->alloc); // counters of split rows, then the paths' records
+    PathAlloc *alloc = (PathAlloc *)(n_split + 4);
     hipLaunchKernelGGL(k_dflatten<R>, dim3(blocks(np)), dim3(256), 0, st, np, P<uint32_t>(s->pt_path),
                        P<uint32_t>(s->first_pt), P<uint32_t>(s->first_ctrl), P<uint32_t>(s->ncubic),
                        (const float2 *)ctrl, P<RV2<R>>(pts));
@@ -1378,23 +1379,20 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
                        P<uint32_t>(s->first_pt), P<uint32_t>(s->first_edge), P<uint32_t>(s->stroke), width,
                        P<RV2<R>>(pts), P<RV2<R>>(nrm), P<RV4<R>>(edges));
     hipLaunchKernelGGL(k_dpaths<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
-                       (int32_t)s->tilesW, (int32_t)s->tilesH, P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc));
-    hipLaunchKernelGGL(k_dalloc, dim3(1), dim3(1024), 0, st, nd, P<PathAlloc>(s->alloc), P<DrawTiles>(s->dtiles),
-                       P<uint32_t>(s->n_split), s->counts);
+                       (int32_t)s->tilesW, (int32_t)s->tilesH, P<DrawTiles>(s->dtiles), alloc);
+    hipLaunchKernelGGL(k_dalloc, dim3(1), dim3(1024), 0, st, nd, alloc, P<DrawTiles>(s->dtiles), n_split, s->counts);
     if (!sync_counts(s))
         return -1;
     const uint32_t n_ptiles = s->counts[0], n_units = s->counts[1];
     s->n_segs = s->counts[2];
     if (!ensure(s, s->ptiles, sizeof(PathTile) * ((size_t)n_ptiles + 1)) ||
         !ensure(s, s->cmd_of, 4ull * ((size_t)n_ptiles + 1)) ||
-        !ensure(s, s->units, sizeof(RowUnit) * ((size_t)n_units + 1)) ||
-        !ensure(s, s->splits, sizeof(SplitRow) * ((size_t)n_units + 1)) ||
+        !ensure(s, s->units, (sizeof(RowUnit) + sizeof(SplitRow)) * ((size_t)n_units + 1)) ||
         !ensure(s, s->segs, 4ull * ((size_t)s->n_segs + 1)))
         return -1;
-    uint32_t *n_split = P<uint32_t>(s->n_split);
-    SplitRow *splits = P<SplitRow>(s->splits);
+    SplitRow *splits = (SplitRow *)(P<RowUnit>(s->units) + n_units + 1);
     hipLaunchKernelGGL(k_dbin<R>, dim3(nd), dim3(256), 0, st, P<uint32_t>(s->first_edge), P<RV4<R>>(edges),
-                       P<DrawTiles>(s->dtiles), P<PathAlloc>(s->alloc), P<PathTile>(s->ptiles),
+                       P<DrawTiles>(s->dtiles), alloc, P<PathTile>(s->ptiles),
                        P<uint32_t>(s->cmd_of), P<uint32_t>(s->segs), P<RowUnit>(s->units), splits,
                        (unsigned long long *)n_split, n_split + 2, split_steps(n_ptiles, n_units, s->n_segs));
     const uint32_t n_tc = s->n_tiles * s->nch;
@@ -1425,7 +1423,8 @@ static int forward_impl(VkvgDiffScene s, const float *ctrl, const float *rgba, c
         ck_ptr = P<float4>(s->ckpt);
     }
     if (!ensure(s, s->cmds, sizeof(Cmd) * ((size_t)s->n_cmds + 1)) ||
-        !ensure(s, s->cov, sizeof(R) * 256 * ((size_t)s->n_cmds + 1)) || !ensure(s, s->sums, 4 * sum_words))
+        !ensure(s, s->cov, sizeof(R) * 256 * ((size_t)s->n_cmds + 1)) ||
+        (sum_words && !ensure(s, s->sums, 4 * sum_words)))
         return -1;
     vkh::launch_coarse(st, true, s->bin_total, s->nch, s->chunk, P<TargetInfo>(s->tg), 1, P<vkh_draw>(s->draws),
                        P<DrawTiles>(s->dtiles), P<PathTile>(s->ptiles), nullptr, P<uint32_t>(s->tile_off),
