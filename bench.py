@@ -340,7 +340,7 @@ def main() -> int:
     # at a time, a SIMD issues one of one or two 32-bit operands (add, subtract, shift, logic, move, float
     # multiply and add) every 2.08 cycles, other ones (three operands, packed 16-bit, DPP, compares, double)
     # every 4.06 and reciprocals every 8.1 (profiles/vector_issue_rates.md). The compiled kernel holds 492,
-    # 789 and 34 of these: 3.44 cycles on average, on 1024 SIMDs at 2.4 GHz. Its VALU instructions per
+    # 789 and 34 of these: 3.42 cycles on average, on 1024 SIMDs at 2.4 GHz. Its VALU instructions per
     # launch come from the same counter summary.
     valu = _read_pmc("fine_c3_pmc.json", "valu_insts_per_launch")
     issue_cycles = (492 * 2.08 + 789 * 4.06 + 34 * 8.1) / (492 + 789 + 34)
